@@ -571,7 +571,7 @@ def bench_pair(args) -> int:
     own = agg_b / agg_s if agg_s > 0 else 0.0
     roofline = {"bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK, "traffic": measured_traffic(args.config),
-                "kernel": "k_path (8 SGM path scans per level and chunk)",
+                "kernel": "k_full, k_sweep, k_path (8 SGM paths per level and chunk)",
                 "algorithmic_bytes": "30 C + 176 P per pair (C cells, P tile pixels, all levels and both directions)",
                 "algorithmic_bytes_per_launch": per_launch,
                 # The scans of a level overlap on two or more streams, so a
@@ -582,8 +582,8 @@ def bench_pair(args) -> int:
                                  "(which waits for the side streams); wall time / launches",
                 "own_model": {"bytes_per_launch": agg_b / max(launches, 1), "achieved": own / 1e9,
                               "frac": own / HBM_PEAK,
-                              "formula": "(40 - 2 w) C + 80 P: C read by 8 scans, S written by 8 and read by "
-                                         "8 - w (w streams), record and intensity per pixel and scan"}}
+                              "formula": "costs, map and records read, S slices or byte planes written and read "
+                                         "back, by each kernel's own dataflow (info.aggregate_bytes)"}}
 
     cpu = None
     if args.cpu_runs > 0:

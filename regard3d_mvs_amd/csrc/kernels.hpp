@@ -110,26 +110,26 @@ void launch_ranges_from_coarse(const float* coarse, int wc, int hc, int width, i
                                std::uint16_t* lo, std::uint16_t* num, std::int64_t rs, hipStream_t s);
 
 // ---- aggregation (kernels_sgm.hip)
-// Cells of every tile row (row_cells[row_base + y]) and the pixel records
-// (cell offset inside the row, lo, num); one block per tile row.
-// row_max = largest label count of the row; bstart[band_base + b * h + y] =
-// row offset of band b's first pixel.
+// Cells of every tile row (row_cells[row_base + y]), its largest label count
+// (row_max) and the pixel records.
 void launch_tile_row_scan(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
                           std::uint64_t total_rows, std::uint64_t* pix, std::uint64_t* row_cells,
-                          std::uint32_t* row_max, std::uint64_t* bstart, hipStream_t s);
-// Band corrections of every tile (see TileDesc): bcorr[band_base + b * h + y];
-// tile_cells[t] = cells of the tile, tile_max[t] = its largest label count.
+                          std::uint32_t* row_max, hipStream_t s);
+// First cell of every tile row in its tile's volume (rowbase[row_base + y]);
+// per tile its cells, its largest label count and the most chunks in a row.
 void launch_tile_cells(const TileDesc* tiles, int ntiles, const std::uint64_t* row_cells, const std::uint32_t* row_max,
-                       const std::uint64_t* bstart, std::uint64_t* bcorr, std::uint64_t* tile_cells,
-                       std::uint32_t* tile_max, hipStream_t s);
+                       std::uint32_t* rowbase, std::uint64_t* tile_cells, std::uint32_t* tile_max,
+                       std::uint32_t* tile_row, hipStream_t s);
 // Path kernel geometry: a wave64 scans kScanPerWave scanlines with
 // kLanesPerScan lanes each (group prefixes count waves).
 constexpr int kLanesPerScan = 8;
 constexpr int kScanPerWave = 64 / kLanesPerScan;
-// Matching costs (u8) of every tile cell into C (same cell indexing as S).
+// Matching costs (u8) of every tile cell into C (same cell indexing as S);
+// cmap (may be null) receives per chunk of 16 cells its column (bits 0-15) and
+// its place in the pixel (bits 16-31).
 void launch_cost(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
-                 std::uint64_t total_rows, const std::uint64_t* bcorr, const std::uint64_t* pix, std::uint8_t* C,
-                 hipStream_t s);
+                 std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix, std::uint8_t* C,
+                 std::uint32_t* cmap, hipStream_t s);
 // One SGM path over every tile (path index 0..7, see kernels_sgm.hip): a
 // persistent launch of at most `slots` waves (path_slots(): the waves that fit
 // on the device) taking scanline groups from `queue` (a zeroed counter).
@@ -139,19 +139,76 @@ std::uint64_t path_slots();
 std::size_t path_scratch_elems(std::uint64_t slots, int max_num);
 int path_scratch_row(int max_num);
 void launch_sgm_path(int path, const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* group_prefix, int ntiles,
-                     std::uint64_t groups, const std::uint64_t* bcorr, const std::uint64_t* pix,
+                     std::uint64_t groups, const std::uint32_t* rowbase, const std::uint64_t* pix,
                      const std::uint8_t* C, std::uint16_t* S, std::uint16_t* scratch, std::uint64_t slots, int max_num,
                      std::uint32_t* queue, bool accumulate, hipStream_t s);
-// Extra elements S and C hold past their last cell.
+// The eight paths of tiles whose pixels all have their job's D labels, each
+// into its own plane of bytes M = L - C (at most P2, which must be at most
+// 255).  A wave takes 64 / lps scanlines (rows for paths 0 and 1, columns for
+// the others); gprefix[t] counts the groups of all paths before tile t.
+// full_lanes: lanes per scanline for D labels, 0 if there is no such kernel.
+struct FullArgs {
+  const JobDesc* jobs;
+  const TileDesc* tiles;
+  const std::uint64_t* gprefix;  // [ntiles + 1]
+  int ntiles;
+  std::uint64_t groups;
+  const std::uint8_t* C;
+  std::uint8_t* M;               // path p's plane at M + p * mstride
+  std::uint64_t mstride;
+};
+int full_lanes(int D);
+void launch_full(const FullArgs& a, int lps, hipStream_t s);
+// The vertical and diagonal paths (2 .. 7) of tiles of at most 1024 columns,
+// row by row: np = 3 takes the three paths downwards (upwards) of a tile at
+// once and stores their sum in slice 0 (1) of S, np = 1 stores path 2 + u in
+// slice u.  Units (2 or 6 per tile) are taken from `queue`, a zeroed counter,
+// in the order of `order`.
+struct SweepArgs {
+  const JobDesc* jobs;
+  const TileDesc* tiles;
+  const std::int32_t* order;
+  std::uint32_t units;
+  const std::uint32_t* rowbase;
+  const std::uint64_t* pix;
+  const std::uint32_t* cmap;
+  const std::uint8_t* C;
+  std::uint16_t* S[6];           // the slice of each unit of a tile
+  std::uint32_t* scratch;        // per block 2 np swords
+  std::uint32_t* queue;
+  int wpad, cap, swords;         // SweepPlan
+};
+// Launch shape for tiles of at most max_w columns and max_chunks chunks a row:
+// words of an LDS row, words of a scratch row (0: none needed), the blocks
+// that run at once.  ok is false where the kernel does not apply.
+struct SweepPlan {
+  bool ok;
+  int wpad, cap, swords, lds_bytes, blocks;
+};
+constexpr int kSweepRowPad = 8;  // words after an LDS row that a window may read
+SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks);
+void launch_sweep(const SweepArgs& a, int np, const SweepPlan& p, std::uint64_t blocks, hipStream_t s);
+// Extra elements S, C and a plane hold past their last cell.
 constexpr std::size_t kSPad = 64;
-// dst[i] = (src[0][i] + ... + src[nsrc - 1][i]) mod 2^16 for i < n rounded up
-// to a multiple of 8 (buffers padded by kSPad); dst may be src[0].
-void launch_sum_u16(std::uint16_t* dst, const std::uint16_t* const* src, int nsrc, std::uint64_t n, hipStream_t s);
+// Aggregated costs: the paths' planes and the costs (m, c), or else n slices
+// of scans that ran side by side (S is their sum mod 2^16), all of p for the
+// tiles whose cells lie below xcells.
+struct SumSrc {
+  const std::uint16_t* p[kPaths];
+  int n;
+  std::uint64_t xcells;
+  const std::uint8_t* m;
+  std::uint64_t mstride;
+  const std::uint8_t* c;
+};
+// dst[i] = (p[0][i] + ... + p[n - 1][i]) mod 2^16 for i < cells rounded up to a
+// multiple of 8 (buffers padded by kSPad); dst may be p[0].
+void launch_sum_u16(std::uint16_t* dst, const SumSrc& src, std::uint64_t cells, hipStream_t s);
 // WTA + sub-pixel + checks of every tile row into per-tile-pixel results.
 void launch_select(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
-                   std::uint64_t total_rows, const std::uint64_t* row_start, const std::uint64_t* pix,
-                   const std::uint16_t* const* S, int nslices, SelectParams p, int max_w, int max_D, float* tdisp,
-                   float* tconf, std::int16_t* tlab, hipStream_t s);
+                   std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix, const SumSrc& src,
+                   SelectParams p, int max_w, int max_D, float* tdisp, float* tconf, std::int16_t* tlab,
+                   hipStream_t s);
 // Packs two valid-interval arrays ([h][2] each) into rows4 ([h][4]).
 void launch_pack_rows(const std::int32_t* base, const std::int32_t* partner, int h, std::int32_t* rows4,
                       hipStream_t s);

@@ -1,19 +1,19 @@
 // gfx950 kernels of the SGM core: tile label layout, matching costs, the 8
 // path scans, winner-takes-all selection and tile blending.
 //
-// Aggregation dataflow (HBM-bound, no MFMA: nothing here is a contraction).
-// k_cost writes the matching cost of every tile cell once per level as one
-// byte (popcount of the Census XOR, or invalid_cost).  Each path direction is
-// one persistent launch over every tile of a chunk: waves take groups of 8
-// adjacent scanlines from a work queue; a scanline is 8 lanes, each holding 4
-// or 8 consecutive labels of the current pixel as packed uint16 pairs, and a
-// pixel's labels are processed in segments (32 labels, then 64 at a time).
-// The predecessor's path costs sit in an LDS row with 0xFFFF sentinels around
-// its labels (a global scratch row for pixels of more than kNarrow labels),
-// the min over a pixel's labels is an 8-lane DPP reduction, and costs, S and
-// the pixel records are prefetched a few steps ahead.  The first path of a
-// stream writes its slice of S, the others add to it (uint16 wrap-around, so
-// the order of the paths does not matter); the selection sums the slices.
+// Aggregation dataflow (no MFMA: nothing here is a contraction).  k_cost
+// writes the matching cost of every tile cell once per level as one byte
+// (popcount of the Census XOR, or invalid_cost).  Three kernels aggregate it:
+//   k_full   tiles without label ranges: all eight paths in one launch, path
+//            costs in registers, a byte plane M = L - C per path;
+//   k_sweep  tiles with label ranges: the vertical and diagonal paths, a block
+//            per tile and direction sweeping row by row, lanes packed with
+//            16-label chunks, up to three paths at once;
+//   k_path   one path direction over every tile by waves of 8 scanlines: the
+//            horizontal paths beside the sweeps, and all eight where the
+//            memory left or the tiles' width rule the others out.
+// Each writes uint16 slices of S (uint16 wrap-around, so the order of the
+// paths does not matter) or byte planes; the selection sums them.
 //
 // Recurrence (sgm_kernels.cpp:176-228, 387-403; stereo_matcher.cpp:1280-1362):
 //   L(p,d) = C(p,d) + min(L(q,d), sat16(min(L(q,d-1), L(q,d+1)) + P1),
@@ -75,6 +75,13 @@ __device__ __forceinline__ __attribute__((address_space(1))) T* gptr_mut(T* p) {
   return (__attribute__((address_space(1))) T*)(p);
 }
 
+// Descriptors that no kernel writes, read through the scalar cache where the
+// address is the same in every lane.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(4))) T* cptr(const T* p) {
+  return (const __attribute__((address_space(4))) T*)(p);
+}
+
 __device__ __forceinline__ void label_range(const JobDesc& J, int X, int Y, int& lo, int& num) {
   if (J.lo != nullptr) {
     lo = J.lo[Y * J.r_stride + X];
@@ -122,17 +129,17 @@ __device__ __forceinline__ std::uint32_t wave_scan_incl(std::uint32_t v) {
 }
 
 // Exclusive scan of the label counts of one tile row into the pixel records:
-// cell offset inside the row, lo, num.  One wave per row (4 rows per block),
-// 64 x kItems pixels per pass, the pass's label ranges loaded before its
-// scans; no block barriers, so a row waits only on its own loads.
+// chunk offset inside the row, chunks, lo, intensity.  One wave per row (4
+// rows per block), 64 x kItems pixels per pass, the pass's label ranges and
+// intensities loaded before its scans; no block barriers, so a row waits only
+// on its own loads.
 __global__ __launch_bounds__(256) void k_tile_row_scan(const JobDesc* __restrict__ jobs,
                                                        const TileDesc* __restrict__ tiles,
                                                        const std::uint64_t* __restrict__ row_prefix, int ntiles,
                                                        std::uint64_t total_rows,
                                                        std::uint64_t* __restrict__ pix,
                                                        std::uint64_t* __restrict__ row_cells,
-                                                       std::uint32_t* __restrict__ row_max,
-                                                       std::uint64_t* __restrict__ bstart) {
+                                                       std::uint32_t* __restrict__ row_max) {
   constexpr int kItems = 8;
   const int lane = static_cast<int>(threadIdx.x & 63);
   const std::uint64_t r = std::uint64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
@@ -144,17 +151,22 @@ __global__ __launch_bounds__(256) void k_tile_row_scan(const JobDesc* __restrict
   const int Y = T.y0 + y;
   const auto jlo = gptr(J.lo), jnum = gptr(J.num);
   const std::int64_t rbase = std::int64_t(Y) * J.r_stride + T.x0;
-  const int bmask = (1 << min(T.band_shift, 30)) - 1;
+  const auto img = gptr(J.img) + std::int64_t(Y) * J.img_stride;
+  // Base columns of a mirrored job read the unmirrored image backwards.
+  const int img_x0 = J.mirrored != 0 ? J.width - 1 - T.x0 : T.x0, img_dx = J.mirrored != 0 ? -1 : 1;
   std::uint64_t* prow = pix + T.px_base + std::uint64_t(y) * T.w;
-  std::uint32_t carry = 0, vmax = 0;
+  std::uint64_t carry = 0;
+  std::uint32_t vmax = 0;
   for (int base = 0; base < T.w; base += 64 * kItems) {
-    int lo[kItems], num[kItems];
+    int lo[kItems], num[kItems], val[kItems];
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
       const int x = base + 64 * k + lane;
       lo[k] = 0;
       num[k] = 0;
+      val[k] = 0;
       if (x < T.w) {
+        val[k] = img[img_x0 + img_dx * x];
         if (jlo != nullptr) {
           lo[k] = jlo[rbase + x];
           num[k] = jnum[rbase + x];
@@ -168,13 +180,7 @@ __global__ __launch_bounds__(256) void k_tile_row_scan(const JobDesc* __restrict
       const int x = base + 64 * k + lane;
       const std::uint32_t v = static_cast<std::uint32_t>(num[k]);
       const std::uint32_t incl = wave_scan_incl(v);
-      if (x < T.w) {
-        const std::uint32_t off = carry + incl - v;
-        prow[x] = pix_record(off, lo[k], num[k]);
-        // Row offset of the first pixel of each band.
-        if ((x & bmask) == 0 && (x >> T.band_shift) < T.nbands)
-          bstart[T.band_base + std::uint64_t(x >> T.band_shift) * T.h + y] = off;
-      }
+      if (x < T.w) prow[x] = pix_record(carry + incl - v, lo[k], num[k], val[k]);
       carry += static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
       vmax = max(vmax, v);
     }
@@ -187,54 +193,42 @@ __global__ __launch_bounds__(256) void k_tile_row_scan(const JobDesc* __restrict
   }
 }
 
-// Totals of one tile (tile_cells, tile_max) and the band corrections: an
-// exclusive scan of the band-row cell counts in band-major order, minus the
-// row offset of the band's first pixel.
+// Totals of one tile (cells, largest label count, most chunks in a row) and
+// the first cell of each of its rows: an exclusive scan of the row counts.
 constexpr int kCellsThreads = 1024;  // k_tile_cells: one block of 16 waves per tile
 __global__ __launch_bounds__(kCellsThreads) void k_tile_cells(const TileDesc* __restrict__ tiles,
                                                     const std::uint64_t* __restrict__ row_cells,
                                                     const std::uint32_t* __restrict__ row_max,
-                                                    const std::uint64_t* __restrict__ bstart,
-                                                    std::uint64_t* __restrict__ bcorr,
+                                                    std::uint32_t* __restrict__ rowbase,
                                                     std::uint64_t* __restrict__ tile_cells,
-                                                    std::uint32_t* __restrict__ tile_max) {
-  constexpr int kItems = 4;  // consecutive band rows per thread and pass
+                                                    std::uint32_t* __restrict__ tile_max,
+                                                    std::uint32_t* __restrict__ tile_row) {
   const TileDesc T = tiles[blockIdx.x];
   __shared__ std::uint64_t wsum[kCellsThreads / 64];
-  __shared__ std::uint32_t smax;
-  if (threadIdx.x == 0) smax = 0;
+  __shared__ std::uint32_t smax, srow;
+  if (threadIdx.x == 0) {
+    smax = 0;
+    srow = 0;
+  }
   __syncthreads();
-  for (int y = threadIdx.x; y < T.h; y += kCellsThreads) atomicMax(&smax, row_max[T.row_base + y]);
-  const int n = T.nbands * T.h;
   std::uint64_t carry = 0;
-  for (int base = 0; base < n; base += kCellsThreads * kItems) {
-    const int e0 = base + kItems * static_cast<int>(threadIdx.x);
-    std::uint64_t v[kItems], b0[kItems], sum = 0;
-#pragma unroll
-    for (int i = 0; i < kItems; ++i) {
-      const int e = e0 + i;
-      v[i] = 0;
-      b0[i] = 0;
-      if (e < n) {
-        const int b = e / T.h, y = e - b * T.h;
-        b0[i] = bstart[T.band_base + e];
-        const std::uint64_t b1 = b + 1 < T.nbands ? bstart[T.band_base + e + T.h] : row_cells[T.row_base + y];
-        v[i] = b1 - b0[i];
-      }
-      sum += v[i];
+  for (int base = 0; base < T.h; base += kCellsThreads) {
+    const int y = base + static_cast<int>(threadIdx.x);
+    std::uint64_t v = 0;
+    if (y < T.h) {
+      v = row_cells[T.row_base + y];
+      atomicMax(&smax, row_max[T.row_base + y]);
+      atomicMax(&srow, static_cast<std::uint32_t>(min(v / kLabelAlign, std::uint64_t{0xFFFFFFFFU})));
     }
     std::uint64_t total;
-    std::uint64_t before = carry + block_scan_incl<kCellsThreads / 64>(sum, wsum, total) - sum;
-#pragma unroll
-    for (int i = 0; i < kItems; ++i) {
-      if (e0 + i < n) bcorr[T.band_base + e0 + i] = before - b0[i];
-      before += v[i];
-    }
+    const std::uint64_t before = carry + block_scan_incl<kCellsThreads / 64>(v, wsum, total) - v;
+    if (y < T.h) rowbase[T.row_base + y] = static_cast<std::uint32_t>(before);
     carry += total;
   }
   if (threadIdx.x == 0) {
     tile_cells[blockIdx.x] = carry;
     tile_max[blockIdx.x] = smax;
+    tile_row[blockIdx.x] = srow;
   }
 }
 
@@ -279,25 +273,24 @@ __device__ __forceinline__ void scan_start(int s, int w, int h, int& x, int& y, 
 // invalid_cost when it does not, 0 for base pixels outside the base row's
 // valid interval.  One block per tile row; a thread per 16-label chunk writes
 // 16 bytes.  Rows of at most kPx pixels stage everything a chunk reads in
-// LDS (pixel cell offsets and lo, base Census, band corrections, a
-// chunk-to-pixel map, the partner Census window), so the chunk loop touches
+// LDS (pixel cell offsets and lo, base Census, a chunk-to-pixel map, the
+// partner Census window), so the chunk loop touches
 // global memory only to store; wider rows search their pixel records in
 // global memory.
 constexpr int kCostThreads = 256;
 __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict__ jobs, const TileDesc* __restrict__ tiles,
                                               const std::uint64_t* __restrict__ row_prefix, int ntiles,
-                                              const std::uint64_t* __restrict__ bcorr,
-                                              const std::uint64_t* __restrict__ pix, std::uint8_t* __restrict__ C) {
+                                              const std::uint32_t* __restrict__ rowbase,
+                                              const std::uint64_t* __restrict__ pix, std::uint8_t* __restrict__ C,
+                                              std::uint32_t* __restrict__ cmap) {
   // Sized for the tiles of the default options (at most 600 columns, 512
   // labels): 24 KB of LDS, six blocks per CU.
   constexpr int kPx = 640;          // row pixels staged in LDS
-  constexpr int kBands = kPx / 8;   // band corrections staged (8-column bands)
   constexpr int kMap = 2048;        // chunks mapped to their pixel
   constexpr int kWin = 1280;        // partner Census columns staged
   __shared__ std::uint32_t soff[kPx];
   __shared__ std::uint16_t slo[kPx];
   __shared__ std::uint64_t scl[kPx];
-  __shared__ std::uint64_t sbc[kBands];
   __shared__ std::uint16_t smap[kMap];
   __shared__ std::uint64_t swin[kWin];
   const std::uint64_t r = blockIdx.x;
@@ -310,7 +303,6 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
   const auto rows = gptr(J.rows4) + 4 * Y;
   const auto cl = gptr(J.cl) + std::size_t(Y) * J.cl_stride;
   const auto cr = gptr(J.cr) + std::size_t(Y) * J.cr_stride;
-  const std::uint64_t* bc = bcorr + T.band_base + y;
   const int pw1 = J.pwidth - 1;
   const bool mir = J.mirrored != 0;
   auto bcol = [&](int X) { return mir ? J.width - 1 - X : X; };  // column of cl
@@ -319,16 +311,15 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
   // tile and label in [0, D); every valid column lies in [c0, c1].
   const int c0 = max(0, T.x0 - J.dmin - (J.D - 1)), c1 = min(pw1, T.x0 + T.w - 1 - J.dmin);
   const bool windowed = c1 >= c0 && c1 - c0 < kWin;
-  const bool staged = T.w <= kPx && T.nbands <= kBands;
+  const bool staged = T.w <= kPx;
   const std::uint64_t last = rec[T.w - 1];
   // Staging: every global load of a thread is issued before the first LDS
   // store, so that the block waits for one memory latency, not one per
   // element (the launch has kCostThreads threads).
   constexpr int kWinIt = (kWin + kCostThreads - 1) / kCostThreads;
   constexpr int kPxIt = (kPx + kCostThreads - 1) / kCostThreads;
-  static_assert(kBands <= kCostThreads, "one band correction per thread");
   const int tid = static_cast<int>(threadIdx.x);
-  std::uint64_t wv[kWinIt], pv[kPxIt], cv[kPxIt], bv = 0;
+  std::uint64_t wv[kWinIt], pv[kPxIt], cv[kPxIt];
 #pragma unroll
   for (int i = 0; i < kWinIt; ++i) {
     const int k = tid + kCostThreads * i;
@@ -341,7 +332,6 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
       pv[i] = x < T.w ? rec[x] : 0;
       cv[i] = x < T.w ? cl[bcol(T.x0 + x)] : 0;
     }
-    if (tid < T.nbands) bv = bc[std::size_t(tid) * T.h];
   }
 #pragma unroll
   for (int i = 0; i < kWinIt; ++i) {
@@ -363,19 +353,19 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
         for (std::uint32_t k = off >> 4; k < e; ++k) smap[k] = static_cast<std::uint16_t>(x);
       }
     }
-    if (tid < T.nbands) sbc[tid] = bv;
   }
   __syncthreads();
   const std::uint32_t chunks = (pix_off(last) + static_cast<std::uint32_t>(pix_num(last))) >> 4;
   const int bfirst = rows[0], blast = rows[1], pfirst = rows[2], plast = rows[3];
   const std::uint32_t invalid = static_cast<std::uint32_t>(J.invalid_cost);
-  std::uint8_t* out = C + T.cell_base;
+  const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + y];
+  std::uint8_t* out = C + row_cell;
+  std::uint32_t* mout = cmap + row_cell / kLabelAlign;
   auto partner = [&](int xr) {
     return windowed ? swin[min(max(xr, c0), c1) - c0] : cr[pcol(min(max(xr, 0), pw1))];
   };
-  // Costs of chunk k of pixel xa (first cell off, first label lo, Census c),
-  // stored at the band row offset bco.
-  auto chunk = [&](std::uint32_t k, int xa, std::uint32_t off, int lo, std::uint64_t c, std::uint64_t bco) {
+  // Costs of chunk k of pixel xa (first cell off, first label lo, Census c).
+  auto chunk = [&](std::uint32_t k, int xa, std::uint32_t off, int lo, std::uint64_t c) {
     const int X = T.x0 + xa;
     const int jb = static_cast<int>(16 * k - off);
     const int xr0 = X - J.dmin - lo - jb;
@@ -394,7 +384,8 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
       }
       w[q] = v;
     }
-    *reinterpret_cast<uint4*>(out + bco + 16 * std::size_t(k)) = make_uint4(w[0], w[1], w[2], w[3]);
+    *reinterpret_cast<uint4*>(out + 16 * std::size_t(k)) = make_uint4(w[0], w[1], w[2], w[3]);
+    if (cmap != nullptr) mout[k] = static_cast<std::uint32_t>(xa) | static_cast<std::uint32_t>(jb / kLabelAlign) << 16;
   };
   if (staged) {
     const bool mapped = chunks <= static_cast<std::uint32_t>(kMap);
@@ -415,7 +406,7 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
           }
         }
       }
-      chunk(k, xa, soff[xa], slo[xa], scl[xa], sbc[xa >> T.band_shift]);
+      chunk(k, xa, soff[xa], slo[xa], scl[xa]);
     }
   } else {
     for (std::uint32_t k = threadIdx.x; k < chunks; k += blockDim.x) {
@@ -429,7 +420,7 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
         }
       }
       const std::uint64_t pr = rec[xa];
-      chunk(k, xa, pix_off(pr), pix_lo(pr), cl[bcol(T.x0 + xa)], bc[std::size_t(xa >> T.band_shift) * T.h]);
+      chunk(k, xa, pix_off(pr), pix_lo(pr), cl[bcol(T.x0 + xa)]);
     }
   }
 }
@@ -447,6 +438,14 @@ __device__ __forceinline__ std::uint32_t min8(std::uint32_t v) {
   v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, false)));
   v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xF, 0xF, false)));
   return v;
+}
+
+// Min over the four lanes of a quad (DPP quad swaps).
+__device__ __forceinline__ std::uint32_t quad_min(std::uint32_t v) {
+  const int i = static_cast<int>(v);
+  v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(i, i, 0xB1, 0xF, 0xF, false)));
+  const int j = static_cast<int>(v);
+  return min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(j, j, 0x4E, 0xF, 0xF, false)));
 }
 
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
@@ -505,12 +504,11 @@ static_assert(kMaxLabels / kLabelAlign <= 255, "label count / 16 must fit 8 bits
 __device__ __forceinline__ int step_lo(const StepIn& u) { return static_cast<int>(u.meta & 0xFFFFU); }
 __device__ __forceinline__ std::uint32_t step_p2_index(const StepIn& u) { return (u.meta >> 16) & 0xFFU; }
 __device__ __forceinline__ int step_num(const StepIn& u) { return static_cast<int>(u.meta >> 24) * kLabelAlign; }
-// Pixel record, band-row offset and intensity of step 8 b + l of a scanline,
-// held by lane l of its group: the loads of 8 steps are one batch.
+// Pixel record and row offset of step 8 b + l of a scanline, held by lane l of
+// its group: the loads of 8 steps are one batch.
 struct StepBatch {
   std::uint64_t rec;
   std::uint32_t rs;
-  std::uint16_t ip;  // widened where it is used, so no wait follows the load
 };
 // Segments 0 and 1 of a pixel, loaded one step ahead.
 struct StepSegs {
@@ -529,14 +527,14 @@ struct StepSegs {
 // its window of P + 2 values as aligned words (the window clamped into the
 // sentinels) and shifts them into place.  Segments 0 and 1 use data prefetched
 // kDist steps ahead; segments from 2 on (pixels of more than 96 labels) are
-// loaded in the step, one segment ahead.  The pixel records, band-row offsets
-// and intensities of a scanline are loaded 8 steps at a time (lane l of the
-// group loads step 8 b + l) and unpacked into an 8-slot ring in LDS, read one
-// step before the segment prefetch that needs them.
+// loaded in the step, one segment ahead.  The pixel records and row offsets
+// of a scanline are loaded 8 steps at a time (lane l of the group loads step
+// 8 b + l) and unpacked into an 8-slot ring in LDS, read one step before the
+// segment prefetch that needs them.
 template <int DX, int DY, bool kAcc>
 __global__ __launch_bounds__(64 * kWaves) void k_path(
     const JobDesc* __restrict__ jobs, const TileDesc* __restrict__ tiles, const std::uint64_t* __restrict__ gprefix,
-    int ntiles, std::uint64_t groups, const std::uint64_t* __restrict__ bcorr,
+    int ntiles, std::uint64_t groups, const std::uint32_t* __restrict__ rowbase,
     const std::uint64_t* __restrict__ pix, const std::uint8_t* __restrict__ C, std::uint16_t* __restrict__ S,
     std::uint16_t* __restrict__ scratch, int scratch_row, std::uint32_t* __restrict__ queue) {
   __shared__ __attribute__((aligned(16))) std::uint16_t lut[kWaves][256];
@@ -597,11 +595,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
 
   const std::uint32_t P1x2 = static_cast<std::uint32_t>(J.p1) * 0x10001U;
   const std::uint64_t* tpix = pix + T.px_base;
-  const std::uint64_t* tbc = bcorr + T.band_base;
-  const std::uint16_t* img = J.img;
-  const int img_stride = static_cast<int>(J.img_stride);
-  // Base columns of a mirrored job read the unmirrored image backwards.
-  const int img_x0 = J.mirrored != 0 ? J.width - 1 - T.x0 : T.x0, img_dx = J.mirrored != 0 ? -1 : 1;
+  const std::uint32_t* trow = rowbase + T.row_base;
   const std::uint8_t* Ct = C + T.cell_base;
   std::uint16_t* St = S + T.cell_base;
 
@@ -611,22 +605,22 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
     const int i = min(base + l8, len - 1);
     const int x = x0 + i * DX, y = y0 + i * DY;
     b.rec = ldb<std::uint64_t>(tpix, static_cast<std::uint32_t>(y * T.w + x) * 8U);
-    b.rs = ldb<std::uint32_t>(tbc, static_cast<std::uint32_t>((x >> T.band_shift) * T.h + y) * 8U);
-    b.ip = ldb<std::uint16_t>(img, static_cast<std::uint32_t>((T.y0 + y) * img_stride + img_x0 + img_dx * x) * 2U);
+    b.rs = ldb<std::uint32_t>(trow, static_cast<std::uint32_t>(y) * 4U);
   };
   // Unpacks a batch into the ring (slot l8 of the group); last_ip carries the
   // intensity of the batch's last step to the next batch's first.
   std::uint32_t last_ip = 0;
   auto write_batch = [&](const StepBatch& b) {
-    std::uint32_t prev = __shfl_up(b.ip, 1U, kLanesPerScan);
+    const std::uint32_t ip = static_cast<std::uint32_t>(pix_val(b.rec));
+    std::uint32_t prev = __shfl_up(ip, 1U, kLanesPerScan);
     prev = l8 == 0 ? last_ip : prev;
-    const std::uint32_t d = static_cast<std::uint32_t>(abs(static_cast<int>(b.ip) - static_cast<int>(prev))) >> 8;
+    const std::uint32_t d = static_cast<std::uint32_t>(abs(static_cast<int>(ip) - static_cast<int>(prev))) >> 8;
     ring[wave][l8][grp] = u32x2{b.rs + pix_off(b.rec), static_cast<std::uint32_t>(pix_lo(b.rec)) | d << 16 |
                                                            static_cast<std::uint32_t>(pix_num(b.rec) / kLabelAlign) << 24};
-    last_ip = __shfl(b.ip, kLanesPerScan - 1, kLanesPerScan);
+    last_ip = __shfl(ip, kLanesPerScan - 1, kLanesPerScan);
     __builtin_amdgcn_wave_barrier();
     // Keep the shuffles of b ahead of the loads that refill it: otherwise the
-    // new intensity lands in a temporary whose copy into b waits for the load.
+    // new record lands in a temporary whose copy into b waits for the load.
     __builtin_amdgcn_sched_barrier(0);
   };
   auto read_step = [&](int i, StepIn& u) {
@@ -900,18 +894,486 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
   }
 }
 
+// ------------------------------------------------------------------ full-range scans
+// The eight path scans of tiles whose pixels all have the same D labels (no
+// label ranges: single-level matches, the coarsest level of a hierarchy).
+// Nothing has to be aligned, so a scanline is LPS lanes (the power of two from
+// D / 16 on, lane q holding labels 16 q .. 16 q + 15 as packed pairs) and the
+// predecessor's path costs never leave their registers: the two neighbours
+// across lanes and the minimum over the labels are DPP moves.  A wave scans
+// 64 / LPS neighbouring scanlines in lockstep: columns of a tile row for the
+// vertical and diagonal paths (a diagonal scanline moves one column per row
+// and re-enters at the other side of the tile, as a new scanline, when it
+// leaves), rows of a tile column for the horizontal ones.  Each path stores
+// M = L - C, at most P2 and so one byte, into its own plane: no path waits
+// for another's sums, and all eight are one launch.
+//
+// Bound by the chain of a step at small sizes and by HBM at large ones (a byte
+// read and a byte written per label and path).  Aggregation of a 640x480 pair
+// with 64 labels: 0.92 ms with eight k_path launches, 0.19 ms here; 1024x768
+// with 128 labels: 3.4 ms, 0.92 ms.
+// Value of the lane below (above) in a wave; the first (last) lane keeps its own.
+template <int LPS>
+__device__ __forceinline__ std::uint32_t lane_below(std::uint32_t v) {
+  const int i = static_cast<int>(v);
+  return static_cast<std::uint32_t>(LPS <= 16 ? __builtin_amdgcn_update_dpp(i, i, 0x111, 0xF, 0xF, false)
+                                              : __builtin_amdgcn_update_dpp(i, i, 0x138, 0xF, 0xF, false));
+}
+template <int LPS>
+__device__ __forceinline__ std::uint32_t lane_above(std::uint32_t v) {
+  const int i = static_cast<int>(v);
+  return static_cast<std::uint32_t>(LPS <= 16 ? __builtin_amdgcn_update_dpp(i, i, 0x101, 0xF, 0xF, false)
+                                              : __builtin_amdgcn_update_dpp(i, i, 0x130, 0xF, 0xF, false));
+}
+template <int CTRL>
+__device__ __forceinline__ std::uint32_t dpp_min(std::uint32_t v) {
+  const int i = static_cast<int>(v);
+  return min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xF, 0xF, false)));
+}
+// Minimum over aligned groups of LPS lanes.
+template <int LPS>
+__device__ __forceinline__ std::uint32_t group_min(std::uint32_t v) {
+  if constexpr (LPS >= 2) v = dpp_min<0xB1>(v);   // quad_perm 1 0 3 2
+  if constexpr (LPS >= 4) v = dpp_min<0x4E>(v);   // quad_perm 2 3 0 1
+  if constexpr (LPS >= 8) v = dpp_min<0x141>(v);  // row_half_mirror
+  if constexpr (LPS >= 16) v = dpp_min<0x140>(v); // row_mirror
+  if constexpr (LPS >= 32) v = min(v, static_cast<std::uint32_t>(__shfl_xor(static_cast<int>(v), 16)));
+  return v;
+}
+
+template <int LPS>
+__global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
+  constexpr int S = 64 / LPS;
+  __shared__ std::uint16_t lut[256];
+  // The P2 table depends on the options only: the same for every job.
+  for (int k = threadIdx.x; k < 256; k += 64 * kWaves) lut[k] = A.jobs[0].lut[k];
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, sc = lane / LPS, q = lane % LPS;
+  const std::uint64_t item = std::uint64_t(blockIdx.x) * kWaves + wave;
+  if (item >= A.groups) return;
+  const auto gprefix = cptr(A.gprefix);
+  int t = 0;
+  for (int hi = A.ntiles - 1; t < hi;) {
+    const int mid = (t + hi + 1) >> 1;
+    if (gprefix[mid] <= item) {
+      t = mid;
+    } else {
+      hi = mid - 1;
+    }
+  }
+  const auto& T = cptr(A.tiles)[t];
+  const auto& J = cptr(A.jobs)[T.job];
+  const int tw = T.w, th = T.h, D = J.D;
+  int path = 0, g = static_cast<int>(item - gprefix[t]);
+  for (; path < kPaths - 1; ++path) {
+    const int n = ((path < 2 ? th : tw) + S - 1) / S;
+    if (g < n) break;
+    g -= n;
+  }
+  // Paths 0, 1: along rows; 2, 3: along columns; 4 .. 7: diagonals.  dx:
+  // columns a scanline moves per step; odd paths run from the last row
+  // (column) to the first.
+  const bool horiz = path < 2, rev = (path & 1) != 0;
+  const int dx = path < 4 ? 0 : (path == 4 || path == 7 ? 1 : -1);
+  const int nscan = horiz ? th : tw, steps = horiz ? tw : th;
+  const int s = min(g * S + sc, nscan - 1);
+  const bool on = g * S + sc < nscan && 16 * q < D;
+  const std::uint8_t* Ct = A.C + T.cell_base;
+  std::uint8_t* Mt = A.M + std::uint64_t(path) * A.mstride + T.cell_base;
+  const std::uint16_t* img = J.img;
+  const int img_stride = static_cast<int>(J.img_stride), iy0 = T.y0;
+  // Base columns of a mirrored job read the unmirrored image backwards.
+  const int ix0 = J.mirrored != 0 ? J.width - 1 - T.x0 : T.x0, idx = J.mirrored != 0 ? -1 : 1;
+  const std::uint32_t P1x2 = static_cast<std::uint32_t>(J.p1) * 0x10001U;
+  const std::uint32_t qoff = 16U * static_cast<std::uint32_t>(min(q, D / 16 - 1));
+  // Sentinels for the neighbours of the first and the last label, and for the labels of idle lanes.
+  const std::uint32_t left_inf = q == 0 ? 0xFFFFFFFFU : 0U, right_inf = 16 * (q + 1) >= D ? 0xFFFFFFFFU : 0U;
+
+  // Cell and intensity of a step's pixel; the column of the next one to load
+  // is kept up to date.
+  int xr = s;
+  struct In {
+    u32x4 c;
+    std::uint32_t cell;
+    std::uint16_t val;
+  };
+  auto load = [&](int i, In& d) {
+    const int r = rev ? steps - 1 - min(i, steps - 1) : min(i, steps - 1);
+    const int x = horiz ? r : xr, y = horiz ? s : r;
+    d.cell = static_cast<std::uint32_t>(y * tw + x) * static_cast<std::uint32_t>(D) + qoff;
+    d.c = ldb<u32x4>(Ct, d.cell);
+    d.val = ldb<std::uint16_t>(img, static_cast<std::uint32_t>((iy0 + y) * img_stride + ix0 + idx * x) * 2U);
+    if (!horiz) {
+      xr += dx;
+      xr = xr >= nscan ? 0 : (xr < 0 ? nscan - 1 : xr);
+    }
+  };
+  std::uint32_t L[8], pmin = 0, p2 = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) L[j] = 0xFFFFFFFFU;
+  int nfirst = 0;
+  auto step = [&](int i, const In& in, const In& next) __attribute__((always_inline)) {
+    const bool first = i == nfirst;
+    // The next pixel of a diagonal that leaves the tile starts a scanline.
+    nfirst += first ? (dx == 0 ? (1 << 30) : (i == 0 ? (dx > 0 ? nscan - s : s + 1) : nscan)) : 0;
+    const std::uint32_t mp = first ? 0U : pmin, pen = first ? 0U : pmin + p2;
+    const std::uint32_t PENx2 = pen * 0x10001U, MPx2 = mp * 0x10001U;
+    // P2 of the next step, read while this one computes.
+    const std::uint32_t ia = in.val, ib = next.val;
+    const std::uint32_t p2n = lut[(max(ia, ib) - min(ia, ib)) >> 8];
+    const std::uint32_t below = lane_below<LPS>(L[7]) | left_inf, above = lane_above<LPS>(L[0]) | right_inf;
+    std::uint32_t Q[9], M[8], m;
+    Q[0] = __builtin_amdgcn_alignbyte(L[0], below, 2U);
+#pragma unroll
+    for (int j = 1; j < 8; ++j) Q[j] = __builtin_amdgcn_alignbyte(L[j], L[j - 1], 2U);
+    Q[8] = __builtin_amdgcn_alignbyte(above, L[7], 2U);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const std::uint32_t Cx2 = __builtin_amdgcn_perm(0U, in.c[j >> 1], (j & 1) ? 0x0c030c02U : 0x0c010c00U);
+      const u16x2 nb =
+          __builtin_elementwise_add_sat(__builtin_elementwise_min(as_pair(Q[j]), as_pair(Q[j + 1])), as_pair(P1x2));
+      const u16x2 best = __builtin_elementwise_min(__builtin_elementwise_min(as_pair(L[j]), nb), as_pair(PENx2));
+      M[j] = as_u32(best - as_pair(MPx2));
+      L[j] = as_u32(as_pair(M[j]) + as_pair(Cx2));
+    }
+    m = L[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) m = as_u32(__builtin_elementwise_min(as_pair(m), as_pair(L[j])));
+    m = min(m & 0xFFFFU, m >> 16);
+    pmin = group_min<LPS>(on ? m : 0xFFFFU);
+    if (on) {
+      u32x4 o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = __builtin_amdgcn_perm(M[2 * j + 1], M[2 * j], 0x06040200U);
+      stb<u32x4>(Mt, in.cell, o);
+    }
+    p2 = p2n;
+  };
+  // Costs and intensities three steps ahead; the loop is unrolled over the
+  // four sets so that every index is a constant.
+  constexpr int N = 4;
+  In in[N];
+#pragma unroll
+  for (int j = 0; j < N - 1; ++j) load(j, in[j]);
+  for (int i = 0; i < steps; i += N) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (i + j < steps) {
+        load(i + j + N - 1, in[(j + N - 1) % N]);
+        step(i + j, in[j], in[(j + 1) % N]);
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------ row sweeps
+// The vertical and diagonal scans of tiles with label ranges.  A block sweeps
+// one tile row by row, downwards or upwards, and advances NP paths at once:
+// all three whose predecessors lie in the last row (NP = 3), so that a row's
+// costs are read and its sums written once for three paths, or one of them
+// (NP = 1, more blocks where there are few tiles).  A thread takes chunks (16
+// labels of a pixel) of the row, whatever pixel they belong to, so that wide
+// and narrow pixels keep the lanes equally busy; cmap holds each chunk's
+// column and place in its pixel.
+//
+// The last row's path costs of every path stay in LDS as uint16: pixel x's
+// labels from word 8 k + x + 1 on, k its first chunk, a word of sentinels
+// between neighbouring pixels (odd strides between one-chunk pixels: no bank
+// conflicts).  Pixels past the LDS rows (cap words, the end of rows with many
+// wide pixels) use rows of the same layout in a global scratch, one per
+// parity.  Each row is two phases between barriers: windows and minima of the
+// last row are read, the new costs stay in registers (kHeld chunks per thread;
+// later ones are past cap and go to scratch) until every thread has read, then
+// they replace the last row.  Costs, map and records are loaded one row ahead.
+//
+// Bound by VALU issue (about 180 instructions per chunk and path with three
+// paths) and the barriers.  The six paths of the 24 MP pair's finest level:
+// 19 ms by k_path; here 12 ms beside the two horizontal scans, on fewer CUs.
+constexpr int kSweepThreads = 1024;
+template <int NP>
+constexpr int kHeld = NP == 3 ? 2 : 4;
+
+// Barrier that orders LDS accesses only: loads in flight and stores of sums
+// stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int NP>
+__global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
+  constexpr int H = kHeld<NP>, N = kSweepThreads;
+  extern __shared__ __attribute__((aligned(16))) std::uint32_t lds[];
+  // info[3][wpad] (pixel records of three rows), pmin[2][NP][wpad], lut, item, rows[NP][cap + pad].
+  const int wpad = A.wpad, cap = A.cap, rstride = cap + kSweepRowPad;
+  u32x2* const info = reinterpret_cast<u32x2*>(lds);
+  std::uint32_t* const pmin = lds + 6 * wpad;
+  std::uint16_t* const lut = reinterpret_cast<std::uint16_t*>(pmin + 2 * NP * wpad);
+  std::uint32_t* const sitem = pmin + 2 * NP * wpad + 128;
+  std::uint32_t* const rows = sitem + 4;
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63;
+  const int wave0 = __builtin_amdgcn_readfirstlane(tid & ~63);  // first thread of the wave
+  if (tid < 256) lut[tid] = A.jobs[0].lut[tid];
+  auto* const scr = gptr_mut(A.scratch + std::uint64_t(blockIdx.x) * 2 * NP * A.swords);
+  constexpr int kUnits = NP == 3 ? 2 : 6;
+  for (;;) {
+    if (tid == 0) *sitem = atomicAdd(A.queue, 1U);
+    __syncthreads();
+    const std::uint32_t item = static_cast<std::uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(*sitem)));
+    if (item >= A.units) break;
+    const int t = cptr(A.order)[item / kUnits], u = static_cast<int>(item % kUnits);
+    const auto& T = cptr(A.tiles)[t];
+    const int w = T.w, h = T.h;
+    const bool rev = (u & 1) != 0;
+    // Columns from the predecessor: 0, 1, -1 (paths 2/3, 4/5, 6/7; upwards 0, -1, 1).
+    const int dx1 = (u >> 1) == 0 ? 0 : (((u >> 1) == 1) != rev ? 1 : -1);
+    auto path_dx = [&](int p) { return NP == 3 ? (p == 0 ? 0 : (p == 1 ? 1 : -1)) : dx1; };
+    const std::uint32_t P1x2 = static_cast<std::uint32_t>(cptr(A.jobs)[T.job].p1) * 0x10001U;
+    const std::uint32_t* rbase = A.rowbase + T.row_base;
+    const std::uint64_t* tpix = A.pix + T.px_base;
+    const std::uint8_t* Ct = A.C + T.cell_base;
+    const std::uint32_t* tmap = A.cmap + T.cell_base / kLabelAlign;
+    std::uint16_t* St = A.S[u] + T.cell_base;
+    const std::uint32_t tcells = T.cells;
+    auto row_y = [&](int i) { return rev ? h - 1 - i : i; };
+    // First cells of 64 rows at a time, one per lane; fcell(i) is that of row
+    // i, and of the row past the last one the other end of the volume.
+    std::uint32_t rb = 0;
+    auto load_rb = [&](int i0) {
+      rb = rbase[row_y(min(i0 + lane, h - 1))];
+      __builtin_amdgcn_s_waitcnt(kVmcnt0);
+    };
+    auto fcell = [&](int i) {
+      return i < h ? static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(rb), i & 63)) : tcells;
+    };
+    load_rb(0);
+    std::uint32_t first = fcell(0), next = h > 1 ? fcell(1) : tcells;
+    int K = static_cast<int>((rev ? tcells - first : next - first) >> 4);
+    // The record of column tid in row i (clamped: unused values).
+    auto load_pix = [&](int i) {
+      return ldb<u32x2>(tpix, static_cast<std::uint32_t>(row_y(min(i, h - 1)) * w + min(tid, w - 1)) * 8U);
+    };
+    u32x4 c[H];
+    std::uint32_t cm[H];
+    auto load_chunk = [&](int r, std::uint32_t f, int n) {
+      const std::uint32_t k = static_cast<std::uint32_t>(min(tid + N * r, n - 1));
+      c[r] = ldb<u32x4>(Ct, f + 16U * k);
+      cm[r] = ldb<std::uint32_t>(tmap, ((f >> 4) + k) * 4U);
+    };
+
+    // Where chunk m's window of path p lies, for pixel records `own` in row
+    // `info o` and predecessors in `info l`: bits 0-15 the window's first word
+    // in the LDS row, bits 16-28 P2, bit 29 the window starts on an odd label,
+    // bit 30 a predecessor exists, bit 31 the window needs the general read
+    // (past a sentinel on either side, or in scratch).
+    auto window = [&](std::uint32_t m, const u32x2& own, const u32x2* linfo, int p) {
+      const int x = static_cast<int>(m & 0xFFFFU), xp = x - path_dx(p);
+      const bool use = xp >= 0 && xp < w;
+      const int xq = use ? xp : 0;
+      const u32x2 pi = linfo[xq];
+      const std::uint32_t ia = own.y >> 16, ib = pi.y >> 16;
+      const std::uint32_t p2 = lut[(max(ia, ib) - min(ia, ib)) >> 8];
+      const int pw = static_cast<int>(pi.x >> 24) * 8, base = 8 * static_cast<int>(pi.x & 0xFFFFFFU) + xq + 1;
+      const int k0 = static_cast<int>(own.y & 0xFFFFU) + kLabelAlign * static_cast<int>(m >> 16) -
+                     static_cast<int>(pi.y & 0xFFFFU);
+      const bool far = static_cast<unsigned>(k0 + 1) > static_cast<unsigned>(2 * pw - 14) || base + pw >= cap;
+      const std::uint32_t at = use && !far ? static_cast<std::uint32_t>(base + ((k0 - 1) >> 1)) : 0U;
+      return at | p2 << 16 | (static_cast<std::uint32_t>(k0) & 1U) << 29 | (use ? 1U << 30 : 0U) |
+             (use && far ? 1U << 31 : 0U);
+    };
+    // A chunk's column, and what its row needs: bit 16 the pixel's first
+    // chunk, bit 17 its last, bit 18 the pixel's costs go to LDS.
+    auto place = [&](std::uint32_t m, const u32x2& own) {
+      const int x = static_cast<int>(m & 0xFFFFU), cc = static_cast<int>(m >> 16), n16 = static_cast<int>(own.x >> 24);
+      const bool in_lds = 8 * (static_cast<int>(own.x & 0xFFFFFFU) + n16) + x + 1 < cap;
+      return static_cast<std::uint32_t>(x) | (cc == 0 ? 1U << 16 : 0U) | (cc == n16 - 1 ? 1U << 17 : 0U) |
+             (in_lds ? 1U << 18 : 0U);
+    };
+    std::uint32_t pre[H][NP], flags[H];
+    // Windows and places of the held chunks of a row of n chunks.
+    auto prepare = [&](const u32x2* cinfo, const u32x2* linfo, int n, bool top) __attribute__((always_inline)) {
+#pragma unroll
+      for (int r = 0; r < H; ++r) {
+        flags[r] = 0;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) pre[r][p] = 0;
+        if (tid + N * r < n) {
+          const u32x2 own = cinfo[cm[r] & 0xFFFFU];
+          flags[r] = place(cm[r], own);
+#pragma unroll
+          for (int p = 0; p < NP; ++p) pre[r][p] = top ? 0U : window(cm[r], own, linfo, p);
+        }
+      }
+    };
+
+#pragma unroll
+    for (int r = 0; r < H; ++r) load_chunk(r, first, K);
+    const u32x2 p0 = load_pix(0);
+    u32x2 pr = load_pix(1);
+    if (tid < w) {
+      info[tid] = p0;
+#pragma unroll
+      for (int p = 0; p < NP; ++p) pmin[p * wpad + tid] = 0xFFFFU;
+    }
+    lds_barrier();
+    prepare(info, info, K, true);
+    int i0 = 0, i1 = 1, i2 = 2;  // info buffers of this, the next and the last row
+    for (int i = 0; i < h; ++i) {
+      std::uint32_t* const cmin = pmin + (i & 1) * NP * wpad;
+      std::uint32_t* const lmin = pmin + ((i & 1) ^ 1) * NP * wpad;
+      auto* const cscr = scr + (i & 1) * NP * A.swords;
+      const auto* const lscr = scr + ((i & 1) ^ 1) * NP * A.swords;
+      const u32x2* const cinfo = info + i0 * wpad;
+      const u32x2* const linfo = info + i2 * wpad;
+      // Chunks of the next row (of this one again after the last).
+      if (((i + 2) & 63) == 0) load_rb(i + 2);
+      const std::uint32_t after = fcell(i + 2);
+      const bool last = i + 1 >= h;
+      const std::uint32_t nfirst = last ? first : next;
+      const int nK = last ? K : static_cast<int>((rev ? first - next : after - next) >> 4);
+
+      // New path costs of chunk k (map entry m, windows pr, unpacked costs
+      // Cx2) into L, their sum to S, their minima to cmin.
+      auto chunk = [&](int k, std::uint32_t m, const std::uint32_t (&pp)[NP], const std::uint32_t (&Cx2)[8],
+                       std::uint32_t (&L)[NP][8]) __attribute__((always_inline)) {
+        const int x = static_cast<int>(m & 0xFFFFU);
+        std::uint32_t sum[8];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          const std::uint32_t v = pp[p];
+          const bool use = (v & (1U << 30)) != 0, far = (v & (1U << 31)) != 0;
+          const std::uint32_t pm = lmin[p * wpad + (use ? x - path_dx(p) : 0)];
+          const std::uint32_t* const lrow = rows + p * rstride;
+          std::uint32_t W[10], sh = ((v >> 29) & 1U) != 0 ? 0U : 16U;
+          const std::uint32_t* wp = lrow + (v & 0xFFFFU);
+#pragma unroll
+          for (int j = 0; j < 10; ++j) W[j] = wp[j];
+          if (__builtin_amdgcn_ballot_w64(far) != 0) {
+            if (far) {
+              const int xq = x - path_dx(p);
+              const u32x2 own = cinfo[x], pi = linfo[xq];
+              const int pw = static_cast<int>(pi.x >> 24) * 8, base = 8 * static_cast<int>(pi.x & 0xFFFFFFU) + xq + 1;
+              const int k0 = static_cast<int>(own.y & 0xFFFFU) + kLabelAlign * static_cast<int>(m >> 16) -
+                             static_cast<int>(pi.y & 0xFFFFU);
+              const int w0 = (k0 - 1) >> 1;
+              if (base + pw < cap) {
+#pragma unroll
+                for (int j = 0; j < 10; ++j) W[j] = lrow[base + min(max(w0 + j, -1), pw)];
+              } else {
+                const auto* sp = lscr + p * A.swords + base;
+#pragma unroll
+                for (int j = 0; j < 10; ++j) W[j] = sp[min(max(w0 + j, -1), pw)];
+                __builtin_amdgcn_s_waitcnt(kVmcnt0);
+              }
+            }
+          }
+          const std::uint32_t mpv = use ? pm : 0U, pen = use ? pm + ((v >> 16) & 0x1FFFU) : 0U;
+          const std::uint32_t PENx2 = pen * 0x10001U, MPx2 = mpv * 0x10001U;
+          std::uint32_t Q[9], mm = 0xFFFFFFFFU;
+#pragma unroll
+          for (int j = 0; j < 9; ++j) Q[j] = __builtin_amdgcn_alignbit(W[j + 1], W[j], sh);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const std::uint32_t p12 = __builtin_amdgcn_alignbyte(Q[j + 1], Q[j], 2U);
+            const u16x2 nb = __builtin_elementwise_add_sat(
+                __builtin_elementwise_min(as_pair(Q[j]), as_pair(Q[j + 1])), as_pair(P1x2));
+            const u16x2 best = __builtin_elementwise_min(__builtin_elementwise_min(as_pair(p12), nb), as_pair(PENx2));
+            L[p][j] = as_u32(best - as_pair(MPx2) + as_pair(Cx2[j]));
+            sum[j] = p == 0 ? L[p][j] : as_u32(as_pair(sum[j]) + as_pair(L[p][j]));
+            mm = as_u32(__builtin_elementwise_min(as_pair(mm), as_pair(L[p][j])));
+          }
+          atomicMin(&cmin[p * wpad + x], min(mm & 0xFFFFU, mm >> 16));
+        }
+        const std::uint32_t at = (first + 16U * static_cast<std::uint32_t>(k)) * 2U;
+        stb<u32x4>(St, at, u32x4{sum[0], sum[1], sum[2], sum[3]});
+        stb<u32x4>(St, at + 16U, u32x4{sum[4], sum[5], sum[6], sum[7]});
+      };
+      // A chunk's costs into a row, with the sentinels around its pixel.
+      auto put = [&](auto* row, int k, std::uint32_t f, const std::uint32_t (&L)[8]) __attribute__((always_inline)) {
+        auto* d = row + 8 * k + static_cast<int>(f & 0xFFFFU) + 1;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) d[j] = L[j];
+        if ((f & (1U << 16)) != 0) d[-1] = 0xFFFFFFFFU;
+        if ((f & (1U << 17)) != 0) d[8] = 0xFFFFFFFFU;
+      };
+      auto unpack = [&](const u32x4& cw, std::uint32_t (&Cx2)[8]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          Cx2[j] = __builtin_amdgcn_perm(0U, cw[j >> 1], (j & 1) ? 0x0c030c02U : 0x0c010c00U);
+      };
+      std::uint32_t L[H][NP][8];
+      bool spilled = false;
+#pragma unroll
+      for (int r = 0; r < H; ++r) {
+        // Waves without a chunk in this row and the next have nothing to do.
+        if (wave0 + N * r >= max(K, nK)) continue;
+        const int k = tid + N * r;
+        std::uint32_t Cx2[8];
+        unpack(c[r], Cx2);
+        const std::uint32_t m = cm[r];
+        load_chunk(r, nfirst, nK);
+        if (k < K) {
+          chunk(k, m, pre[r], Cx2, L[r]);
+          if ((flags[r] & (1U << 18)) == 0) {
+            spilled = true;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) put(cscr + p * A.swords, k, flags[r], L[r][p]);
+          }
+        }
+      }
+      // Chunks past the held ones lie past cap.
+      for (int k = tid + N * H; k < K; k += N) {
+        std::uint32_t Cx2[8], X[NP][8], pp[NP];
+        const std::uint32_t m = ldb<std::uint32_t>(tmap, ((first >> 4) + static_cast<std::uint32_t>(k)) * 4U);
+        unpack(ldb<u32x4>(Ct, first + 16U * static_cast<std::uint32_t>(k)), Cx2);
+        const u32x2 own = cinfo[m & 0xFFFFU];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) pp[p] = i == 0 ? 0U : window(m, own, linfo, p);
+        chunk(k, m, pp, Cx2, X);
+        spilled = true;
+        const std::uint32_t f = place(m, own);
+#pragma unroll
+        for (int p = 0; p < NP; ++p) put(cscr + p * A.swords, k, f, X[p]);
+      }
+      if (tid < w) info[i1 * wpad + tid] = pr;
+      pr = load_pix(i + 2);
+      // Scratch rows have to be in place before another wave reads them.
+      if (__builtin_amdgcn_ballot_w64(spilled) != 0) __builtin_amdgcn_s_waitcnt(kVmcnt0);
+      lds_barrier();
+#pragma unroll
+      for (int r = 0; r < H; ++r) {
+        if ((flags[r] & (1U << 18)) != 0) {
+#pragma unroll
+          for (int p = 0; p < NP; ++p) put(rows + p * rstride, tid + N * r, flags[r], L[r][p]);
+        }
+      }
+      if (tid < w) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) lmin[p * wpad + tid] = 0xFFFFU;
+      }
+      prepare(info + i1 * wpad, cinfo, nK, false);
+      lds_barrier();
+      const int t0 = i2;
+      i2 = i0;
+      i0 = i1;
+      i1 = t0;
+      first = nfirst;
+      next = after;
+      K = nK;
+    }
+  }
+}
+
 // ------------------------------------------------------------------ partial sums
 // Sum of the path-cost slices of scans that ran side by side (uint16
 // wrap-around, so the grouping of the 8 paths does not matter).
-struct SumSrc {
-  const std::uint16_t* p[4];
-};
-__global__ __launch_bounds__(256) void k_sum_u16(std::uint16_t* __restrict__ dst, SumSrc src, int nsrc,
-                                                 std::uint64_t n8) {
+__global__ __launch_bounds__(256) void k_sum_u16(std::uint16_t* __restrict__ dst, SumSrc src, std::uint64_t n8) {
   const std::uint64_t i = std::uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n8) return;
   uint4 acc = reinterpret_cast<const uint4*>(src.p[0])[i];
-  for (int k = 1; k < nsrc; ++k) {
+  for (int k = 1; k < src.n; ++k) {
     const uint4 v = reinterpret_cast<const uint4*>(src.p[k])[i];
     acc.x = as_u32(as_pair(acc.x) + as_pair(v.x));
     acc.y = as_u32(as_pair(acc.y) + as_pair(v.y));
@@ -940,13 +1402,6 @@ __device__ __forceinline__ float subpixel_offset(int method, float sm, float s0,
 // [32 i + 8 q, 32 i + 8 q + 8) of chunk i, so a quad reads 64 contiguous
 // bytes per chunk; the first two chunks stay in registers for the second
 // pass of the winner-takes-all (sgm_kernels.cpp:405-426).
-__device__ __forceinline__ std::uint32_t quad_min(std::uint32_t v) {
-  const int i = static_cast<int>(v);
-  v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(i, i, 0xB1, 0xF, 0xF, false)));
-  const int j = static_cast<int>(v);
-  return min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(j, j, 0x4E, 0xF, 0xF, false)));
-}
-
 // Minimum of (value << 16 | label) over the 8 labels of a chunk word group,
 // labels k0..k0+7: the lowest value, the first label on ties.
 __device__ __forceinline__ std::uint32_t key_min(const uint4& q, int k0, std::uint32_t m) {
@@ -1001,15 +1456,15 @@ __device__ __forceinline__ std::uint32_t group_value(const uint4& q, int k0, int
   return e >= 0 && e < 8 ? v : 0xFFFFFFFFU;
 }
 
+template <bool kBytes>
 __global__ __launch_bounds__(256) void k_select(const JobDesc* __restrict__ jobs, const TileDesc* __restrict__ tiles,
                                                 const std::uint64_t* __restrict__ row_prefix, int ntiles,
-                                                const std::uint64_t* __restrict__ bcorr,
-                                                const std::uint64_t* __restrict__ pix,
-                                                SumSrc S, int nslices, SelectParams p,
+                                                const std::uint32_t* __restrict__ rowbase,
+                                                const std::uint64_t* __restrict__ pix, SumSrc S, SelectParams p,
                                                 float* __restrict__ tdisp, float* __restrict__ tconf,
                                                 std::int16_t* __restrict__ tlab) {
   constexpr int kStage = 1024;  // row pixels whose first cell and range are staged in LDS
-  __shared__ std::uint64_t scell[kStage];
+  __shared__ std::uint32_t soff[kStage];
   __shared__ std::uint32_t srange[kStage];
   extern __shared__ std::uint32_t keys[];
   const std::uint64_t r = blockIdx.x;
@@ -1022,11 +1477,33 @@ __global__ __launch_bounds__(256) void k_select(const JobDesc* __restrict__ jobs
   const int lf = rows[0], ll = rows[1], rf = rows[2], rl = rows[3];
   const int xb = min(max(lf - T.x0, 0), T.w);
   const int xe = min(max(ll + 1 - T.x0, xb), T.w);
-  const std::uint64_t* bc = bcorr + T.band_base + y;
-  // Aggregated costs: the sum of the slices of scans that ran side by side.
+  const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + y];
+  const int slices = T.cell_base < S.xcells ? kPaths : S.n;
+  // Aggregated costs of 8 labels: 8 C plus the eight paths' bytes M (L = C + M),
+  // or the sum of the slices of scans that ran side by side.
   auto ld8 = [&](std::uint64_t c) {
+    if constexpr (kBytes) {
+      u32x2 v[kPaths + 1];
+#pragma unroll
+      for (int i = 0; i < kPaths; ++i) v[i] = *reinterpret_cast<const u32x2*>(S.m + i * S.mstride + c);
+      v[kPaths] = *reinterpret_cast<const u32x2*>(S.c + c);
+      std::uint32_t w[4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        // Even and odd labels as packed 16-bit sums (at most 16 x 255).
+        std::uint32_t even = (v[kPaths][h] & 0x00FF00FFU) << 3, odd = ((v[kPaths][h] >> 8) & 0x00FF00FFU) << 3;
+#pragma unroll
+        for (int i = 0; i < kPaths; ++i) {
+          even += v[i][h] & 0x00FF00FFU;
+          odd += (v[i][h] >> 8) & 0x00FF00FFU;
+        }
+        w[2 * h] = __builtin_amdgcn_perm(odd, even, 0x05040100U);
+        w[2 * h + 1] = __builtin_amdgcn_perm(odd, even, 0x07060302U);
+      }
+      return make_uint4(w[0], w[1], w[2], w[3]);
+    }
     uint4 a = *reinterpret_cast<const uint4*>(S.p[0] + c);
-    for (int i = 1; i < nslices; ++i) {
+    for (int i = 1; i < slices; ++i) {
       const uint4 v = *reinterpret_cast<const uint4*>(S.p[i] + c);
       a.x = as_u32(as_pair(a.x) + as_pair(v.x));
       a.y = as_u32(as_pair(a.y) + as_pair(v.y));
@@ -1036,8 +1513,14 @@ __global__ __launch_bounds__(256) void k_select(const JobDesc* __restrict__ jobs
     return a;
   };
   auto ld1 = [&](std::uint64_t c) {
+    if constexpr (kBytes) {
+      std::uint32_t a = 8U * S.c[c];
+#pragma unroll
+      for (int i = 0; i < kPaths; ++i) a += S.m[i * S.mstride + c];
+      return a;
+    }
     std::uint32_t a = S.p[0][c];
-    for (int i = 1; i < nslices; ++i) a += S.p[i][c];
+    for (int i = 1; i < slices; ++i) a += S.p[i][c];
     return a & 0xFFFFU;
   };
   const std::uint64_t px = T.px_base + std::uint64_t(y) * T.w;
@@ -1048,38 +1531,34 @@ __global__ __launch_bounds__(256) void k_select(const JobDesc* __restrict__ jobs
   if (staged) {
     // Every load of a thread before its first LDS store (256 threads).
     constexpr int kIt = kStage / 256;
-    std::uint64_t rv[kIt], bv[kIt];
+    std::uint64_t rv[kIt];
 #pragma unroll
     for (int i = 0; i < kIt; ++i) {
       const int x = static_cast<int>(threadIdx.x) + 256 * i;
       rv[i] = x < T.w ? pix[px + x] : 0;
-      bv[i] = x < T.w ? bc[std::size_t(x >> T.band_shift) * T.h] : 0;
     }
 #pragma unroll
     for (int i = 0; i < kIt; ++i) {
       const int x = static_cast<int>(threadIdx.x) + 256 * i;
       if (x < T.w) {
-        scell[x] = bv[i] + pix_off(rv[i]);
-        srange[x] = static_cast<std::uint32_t>(rv[i] >> 32);
+        soff[x] = pix_off(rv[i]);
+        srange[x] = static_cast<std::uint32_t>(pix_lo(rv[i])) | static_cast<std::uint32_t>(pix_num(rv[i])) << 16;
       }
     }
     __syncthreads();
   }
   // First cell, lo and label count of pixel x.
   auto pixel = [&](int x, int& lo, int& n) {
-    std::uint64_t cell;
-    std::uint32_t range;
     if (staged) {
-      cell = scell[x];
-      range = srange[x];
-    } else {
-      const std::uint64_t rec = pix[px + x];
-      cell = bc[std::size_t(x >> T.band_shift) * T.h] + pix_off(rec);
-      range = static_cast<std::uint32_t>(rec >> 32);
+      const std::uint32_t range = srange[x];
+      lo = static_cast<int>(range & 0xFFFFU);
+      n = static_cast<int>(range >> 16);
+      return row_cell + soff[x];
     }
-    lo = static_cast<int>(range & 0xFFFFU);
-    n = static_cast<int>(range >> 16);
-    return T.cell_base + cell;
+    const std::uint64_t rec = pix[px + x];
+    lo = pix_lo(rec);
+    n = pix_num(rec);
+    return row_cell + pix_off(rec);
   };
 
   if (p.diagonal_lr) {
@@ -1091,9 +1570,13 @@ __global__ __launch_bounds__(256) void k_select(const JobDesc* __restrict__ jobs
       int lo, num;
       const std::uint64_t s = pixel(x, lo, num);
       for (int k0 = 8 * q; k0 < num; k0 += 32) {
+        const uint4 g = ld8(s + k0);
+        const std::uint32_t w[4] = {g.x, g.y, g.z, g.w};
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          atomicMin(&keys[x - (lo + k0 + e) + D - 1], (ld1(s + k0 + e) << 16) | std::uint32_t(x));
+        for (int e = 0; e < 8; ++e) {
+          const std::uint32_t v = (w[e >> 1] >> ((e & 1) * 16)) & 0xFFFFU;
+          atomicMin(&keys[x - (lo + k0 + e) + D - 1], (v << 16) | std::uint32_t(x));
+        }
       }
     }
     __syncthreads();
@@ -1306,7 +1789,7 @@ std::uint64_t path_blocks() {
 
 template <int DX, int DY>
 void path_launch(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* gp, int ntiles,
-                 std::uint64_t groups, const std::uint64_t* rs, const std::uint64_t* pix, const std::uint8_t* C,
+                 std::uint64_t groups, const std::uint32_t* rs, const std::uint64_t* pix, const std::uint8_t* C,
                  std::uint16_t* S, std::uint16_t* scratch, int scratch_row, std::uint32_t* queue, std::uint64_t slots,
                  bool accumulate, hipStream_t s) {
   // Persistent waves: at most `slots` (scratch rows), at most one per group.
@@ -1326,24 +1809,24 @@ void path_launch(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t
 
 void launch_tile_row_scan(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
                           std::uint64_t total_rows, std::uint64_t* pix, std::uint64_t* row_cells,
-                          std::uint32_t* row_max, std::uint64_t* bstart, hipStream_t s) {
+                          std::uint32_t* row_max, hipStream_t s) {
   if (total_rows == 0) return;
   k_tile_row_scan<<<dim3(static_cast<unsigned>((total_rows + 3) / 4)), 256, 0, s>>>(jobs, tiles, row_prefix, ntiles,
-                                                                                    total_rows, pix, row_cells, row_max,
-                                                                                    bstart);
+                                                                                    total_rows, pix, row_cells, row_max);
 }
 
 void launch_tile_cells(const TileDesc* tiles, int ntiles, const std::uint64_t* row_cells, const std::uint32_t* row_max,
-                       const std::uint64_t* bstart, std::uint64_t* bcorr, std::uint64_t* tile_cells,
-                       std::uint32_t* tile_max, hipStream_t s) {
-  k_tile_cells<<<dim3(ntiles), kCellsThreads, 0, s>>>(tiles, row_cells, row_max, bstart, bcorr, tile_cells, tile_max);
+                       std::uint32_t* rowbase, std::uint64_t* tile_cells, std::uint32_t* tile_max,
+                       std::uint32_t* tile_row, hipStream_t s) {
+  k_tile_cells<<<dim3(ntiles), kCellsThreads, 0, s>>>(tiles, row_cells, row_max, rowbase, tile_cells, tile_max, tile_row);
 }
 
 void launch_cost(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
-                 std::uint64_t total_rows, const std::uint64_t* bcorr, const std::uint64_t* pix, std::uint8_t* C,
-                 hipStream_t s) {
+                 std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix, std::uint8_t* C,
+                 std::uint32_t* cmap, hipStream_t s) {
   if (total_rows == 0) return;
-  k_cost<<<dim3(static_cast<unsigned>(total_rows)), kCostThreads, 0, s>>>(jobs, tiles, row_prefix, ntiles, bcorr, pix, C);
+  k_cost<<<dim3(static_cast<unsigned>(total_rows)), kCostThreads, 0, s>>>(jobs, tiles, row_prefix, ntiles, rowbase, pix,
+                                                                         C, cmap);
 }
 
 int path_scratch_row(int max_num) { return kPad + (max_num + 15) / 16 * 16 + kPad; }
@@ -1362,7 +1845,7 @@ std::size_t path_scratch_elems(std::uint64_t slots, int max_num) {
 }
 
 void launch_sgm_path(int path, const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* gp, int ntiles,
-                     std::uint64_t groups, const std::uint64_t* rs, const std::uint64_t* pix, const std::uint8_t* C,
+                     std::uint64_t groups, const std::uint32_t* rs, const std::uint64_t* pix, const std::uint8_t* C,
                      std::uint16_t* S, std::uint16_t* scratch, std::uint64_t slots, int max_num,
                      std::uint32_t* queue, bool accumulate, hipStream_t s) {
   if (groups == 0) return;
@@ -1379,24 +1862,75 @@ void launch_sgm_path(int path, const JobDesc* jobs, const TileDesc* tiles, const
   }
 }
 
-void launch_select(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
-                   std::uint64_t total_rows, const std::uint64_t* row_start, const std::uint64_t* col_off,
-                   const std::uint16_t* const* S, int nslices, SelectParams p, int max_w, int max_D, float* tdisp,
-                   float* tconf, std::int16_t* tlab, hipStream_t s) {
-  if (total_rows == 0 || nslices < 1 || nslices > 4) return;
-  SumSrc ss{};
-  for (int k = 0; k < nslices; ++k) ss.p[k] = S[k];
-  const std::size_t lds = p.diagonal_lr ? std::size_t(max_w + max_D) * sizeof(std::uint32_t) : 0;
-  k_select<<<dim3(static_cast<unsigned>(total_rows)), 256, lds, s>>>(jobs, tiles, row_prefix, ntiles, row_start,
-                                                                      col_off, ss, nslices, p, tdisp, tconf, tlab);
+int full_lanes(int D) {
+  int lps = 2;
+  while (lps * kLabelAlign < D) lps *= 2;
+  return lps <= 32 ? lps : 0;
 }
 
-void launch_sum_u16(std::uint16_t* dst, const std::uint16_t* const* src, int nsrc, std::uint64_t n, hipStream_t s) {
+void launch_full(const FullArgs& a, int lps, hipStream_t s) {
+  if (a.groups == 0) return;
+  const dim3 grid(static_cast<unsigned>((a.groups + kWaves - 1) / kWaves));
+  switch (lps) {
+    case 2: k_full<2><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 4: k_full<4><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 8: k_full<8><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 16: k_full<16><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    default: k_full<32><<<grid, 64 * kWaves, 0, s>>>(a); break;
+  }
+}
+
+SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks) {
+  SweepPlan p{};
+  if (max_w > kSweepThreads) return p;
+  int dev = 0, cus = 0, lds = 0;
+  (void)hipGetDevice(&dev);
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  (void)hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+  const int fixed = 4 * (6 * max_w + 2 * np * max_w + 128 + 4);
+  const int held = np == 3 ? kHeld<3> : kHeld<1>;
+  const int need = static_cast<int>(std::min<std::uint64_t>(8 * std::uint64_t(max_chunks) + std::uint64_t(max_w) + 2, 1 << 20));
+  p.wpad = max_w;
+  p.cap = std::min({(lds - fixed) / (4 * np) - kSweepRowPad, 8 * kSweepThreads * held, need});
+  if (p.cap < 1024) return p;
+  p.lds_bytes = fixed + 4 * np * (p.cap + kSweepRowPad);
+  p.swords = p.cap >= need ? 0 : need + 16;
+  p.blocks = std::max(cus, 1);
+  p.ok = true;
+  return p;
+}
+
+void launch_sweep(const SweepArgs& a, int np, const SweepPlan& p, std::uint64_t blocks, hipStream_t s) {
+  if (a.units == 0) return;
+  const dim3 grid(static_cast<unsigned>(std::min<std::uint64_t>(a.units, blocks)));
+  // Dynamic LDS past 64 KB has to be asked for once per kernel and device.
+  const auto* fn = np == 3 ? reinterpret_cast<const void*>(&k_sweep<3>) : reinterpret_cast<const void*>(&k_sweep<1>);
+  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, p.lds_bytes) != hipSuccess) return;
+  if (np == 3) {
+    k_sweep<3><<<grid, kSweepThreads, p.lds_bytes, s>>>(a);
+  } else {
+    k_sweep<1><<<grid, kSweepThreads, p.lds_bytes, s>>>(a);
+  }
+}
+
+void launch_select(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
+                   std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix, const SumSrc& src,
+                   SelectParams p, int max_w, int max_D, float* tdisp, float* tconf, std::int16_t* tlab,
+                   hipStream_t s) {
+  if (total_rows == 0) return;
+  const std::size_t lds = p.diagonal_lr ? std::size_t(max_w + max_D) * sizeof(std::uint32_t) : 0;
+  const dim3 grid(static_cast<unsigned>(total_rows));
+  if (src.m != nullptr) {
+    k_select<true><<<grid, 256, lds, s>>>(jobs, tiles, row_prefix, ntiles, rowbase, pix, src, p, tdisp, tconf, tlab);
+  } else {
+    k_select<false><<<grid, 256, lds, s>>>(jobs, tiles, row_prefix, ntiles, rowbase, pix, src, p, tdisp, tconf, tlab);
+  }
+}
+
+void launch_sum_u16(std::uint16_t* dst, const SumSrc& src, std::uint64_t n, hipStream_t s) {
   const std::uint64_t n8 = (n + 7) / 8;
-  if (n8 == 0 || nsrc <= 0 || nsrc > 4) return;
-  SumSrc ss{};
-  for (int k = 0; k < nsrc; ++k) ss.p[k] = src[k];
-  k_sum_u16<<<dim3(static_cast<unsigned>((n8 + 255) / 256)), 256, 0, s>>>(dst, ss, nsrc, n8);
+  if (n8 == 0 || src.n <= 0) return;
+  k_sum_u16<<<dim3(static_cast<unsigned>((n8 + 255) / 256)), 256, 0, s>>>(dst, src, n8);
 }
 
 void launch_pack_rows(const std::int32_t* base, const std::int32_t* partner, int h, std::int32_t* rows4,

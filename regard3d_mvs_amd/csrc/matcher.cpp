@@ -490,8 +490,6 @@ std::size_t estimated_tile_bytes(std::uint64_t cells64, int w_, int h_, int righ
          (w + static_cast<std::size_t>(right_width) + 16) * (h + 6) * 8;
 }
 
-int path_scanlines(int p, int w, int h) { return p < 2 ? h : (p < 4 ? w : w + h - 1); }
-
 // Tile layout of a set of jobs: the tiles of all jobs share the layout pass,
 // and chunks of consecutive tiles share the cost pass, the 8 path launches
 // and the selection launch.
@@ -503,9 +501,13 @@ struct Aggregation {
   std::vector<Grid> grids;
   std::vector<int> tile_base;
   std::vector<std::uint64_t> tcells;
-  DBuf<std::uint64_t> bcorr, pix;  // bcorr: band corrections (TileDesc)
+  DBuf<std::uint32_t> rowbase;  // first cell of every tile row
+  DBuf<std::uint64_t> pix;
   std::uint64_t total_rows = 0, total_px = 0, total_cells = 0, max_tile_cells = 0;
-  int max_w = 1, max_D = 16, max_num = 16;
+  int max_w = 1, max_h = 1, max_D = 16, max_num = 16;
+  std::uint32_t max_row_chunks = 1;
+  int p2max = 0;
+  std::vector<int> full;  // per job: its labels if every pixel has all of them, else 0
 };
 
 // Aggregated volume S of tiles [t0, t1) of a layout; the chunk's tile
@@ -516,23 +518,38 @@ struct Chunk {
   DView<TileDesc> dtiles;
   DView<std::uint64_t> drow_prefix;
   std::uint64_t rows = 0, cells = 0, px = 0;
-  // Aggregated costs: S plus the slices of path scans that ran side by side
-  // on other streams (the sum mod 2^16 of all of them).
-  DBuf<std::uint16_t> S;
-  std::vector<DBuf<std::uint16_t>> slices;
-  std::vector<const std::uint16_t*> parts() const {
-    std::vector<const std::uint16_t*> v{S.get()};
-    for (const auto& b : slices) v.push_back(b.get());
+  // Aggregated costs: the paths' planes and the costs C, or slices of S (the
+  // sum mod 2^16 of all of them), `stride` elements apart.
+  DBuf<std::uint8_t> C, planes;
+  DBuf<std::uint16_t> S, X;
+  std::uint64_t stride = 0;
+  int slices = 0;
+  // Tiles swept path by path hold the chunk's first xcells cells; their
+  // further paths have slices of their own, xstride elements apart in X.
+  std::uint64_t xcells = 0, xstride = 0;
+  SumSrc source() const {
+    SumSrc v{};
+    if (planes.get() != nullptr) {
+      v.m = planes.get();
+      v.mstride = stride;
+      v.c = C.get();
+      return v;
+    }
+    for (v.n = 0; v.n < slices; ++v.n) v.p[v.n] = S.get() + std::uint64_t(v.n) * stride;
+    if (xcells > 0) {
+      v.xcells = xcells;
+      for (int k = slices; k < kPaths; ++k) v.p[k] = X.get() + std::uint64_t(k - slices) * xstride;
+    }
     return v;
   }
 };
 
-// band_shift: log2 of the volume band width (TileDesc); 31 stores every tile
-// row contiguously (the packed order of detail::sgm_cost_volume).
-Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& o, int band_shift = 3) {
+Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& o) {
   Aggregation A;
   const int nj = static_cast<int>(jobs.size());
   const auto lut = p2_table(o);
+  A.p2max = *std::max_element(lut.begin(), lut.end());
+  for (const Job& J : jobs) A.full.push_back(J.ranges == nullptr ? J.D : 0);
   std::vector<JobDesc> jd(static_cast<std::size_t>(nj));
   for (int j = 0; j < nj; ++j) {
     const Job& J = jobs[std::size_t(j)];
@@ -572,10 +589,11 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
   std::vector<std::uint32_t> tmax;
   DView<TileDesc> dtiles;
   DView<std::uint64_t> drow_prefix;
-  DBuf<std::uint64_t>& bcorr = A.bcorr;
-  DBuf<std::uint64_t> bstart;
+  std::vector<std::uint32_t> trow;
+  DBuf<std::uint32_t>& rowbase = A.rowbase;
   DBuf<std::uint64_t>& pix = A.pix;
-  DBuf<std::uint64_t> row_cells, tile_counts;  // tile_counts: cells [nt], then the max label counts (uint32)
+  // tile_counts: cells [nt], then (uint32) the largest label counts [nt] and the most chunks in a row [nt]
+  DBuf<std::uint64_t> row_cells, tile_counts;
   DBuf<std::uint32_t> row_max;
   std::uint64_t& total_rows = A.total_rows;
   std::uint64_t& total_px = A.total_px;
@@ -586,7 +604,6 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
     row_prefix.clear();
     total_rows = 0;
     total_px = 0;
-    std::uint64_t total_bands = 0;
     for (int j = 0; j < nj; ++j) {
       const Job& J = jobs[std::size_t(j)];
       grids[std::size_t(j)] = layout(J.base->w, J.base->h, tsize[std::size_t(j)], ext);
@@ -601,13 +618,9 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
           t.job = j;
           t.px_base = total_px;
           t.row_base = total_rows;
-          t.band_shift = band_shift;
-          t.nbands = band_shift >= 30 ? 1 : (t.w + (1 << band_shift) - 1) >> band_shift;
-          t.band_base = total_bands;
           row_prefix.push_back(total_rows);
           total_px += std::uint64_t(t.w) * std::uint64_t(t.h);
           total_rows += std::uint64_t(t.h);
-          total_bands += std::uint64_t(t.nbands) * std::uint64_t(t.h);
           td.push_back(t);
         }
       }
@@ -625,16 +638,16 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
     pix = DBuf<std::uint64_t>(c.arena, total_px);
     row_cells = DBuf<std::uint64_t>(c.arena, total_rows);
     row_max = DBuf<std::uint32_t>(c.arena, total_rows);
-    bstart = DBuf<std::uint64_t>(c.arena, total_bands);
-    bcorr = DBuf<std::uint64_t>(c.arena, total_bands);
+    rowbase = DBuf<std::uint32_t>(c.arena, total_rows);
     tile_counts = DBuf<std::uint64_t>(c.arena, 2 * std::size_t(nt));
     launch_tile_row_scan(A.djobs.get(), dtiles.get(), drow_prefix.get(), nt, total_rows, pix.get(), row_cells.get(),
-                         row_max.get(), bstart.get(), c.stream);
+                         row_max.get(), c.stream);
     check_launch();
-    launch_tile_cells(dtiles.get(), nt, row_cells.get(), row_max.get(), bstart.get(), bcorr.get(), tile_counts.get(),
-                      reinterpret_cast<std::uint32_t*>(tile_counts.get() + nt), c.stream);
+    auto* const tail = reinterpret_cast<std::uint32_t*>(tile_counts.get() + nt);
+    launch_tile_cells(dtiles.get(), nt, row_cells.get(), row_max.get(), rowbase.get(), tile_counts.get(), tail,
+                      tail + nt, c.stream);
     check_launch();
-    // Cells and largest label count of every tile, in one download (into a
+    // Counts of every tile, in one download (into a
     // pinned block, so that the host waits in the stream synchronisation).
     std::vector<std::uint64_t> counts(2 * std::size_t(nt), 0);
     {
@@ -654,7 +667,10 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
     }
     tcells.assign(counts.begin(), counts.begin() + nt);
     tmax.resize(std::size_t(nt));
-    std::memcpy(tmax.data(), counts.data() + nt, sizeof(std::uint32_t) * nt);
+    trow.resize(std::size_t(nt));
+    const auto* const ctail = reinterpret_cast<const std::uint32_t*>(counts.data() + nt);
+    std::copy_n(ctail, nt, tmax.begin());
+    std::copy_n(ctail + nt, nt, trow.begin());
     // Halve the tile size of a job while its largest tile exceeds the memory
     // budget (stereo_matcher.cpp:643-648).
     bool changed = false;
@@ -680,11 +696,13 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
   int& max_D = A.max_D;
   for (int t = 0; t < nt; ++t) {
     td[std::size_t(t)].cell_base = total_cells;
+    td[std::size_t(t)].cells = static_cast<std::uint32_t>(tcells[std::size_t(t)]);
     A.max_tile_cells = std::max(A.max_tile_cells, tcells[std::size_t(t)]);
     td[std::size_t(t)].max_num = static_cast<std::int32_t>(tmax[std::size_t(t)]);
     total_cells += tcells[std::size_t(t)];
     max_num = std::max<int>(max_num, static_cast<int>(tmax[std::size_t(t)]));
     max_w = std::max(max_w, td[std::size_t(t)].w);
+    A.max_h = std::max(A.max_h, td[std::size_t(t)].h);
   }
   for (const Job& J : jobs) max_D = std::max(max_D, J.D);
   if (max_num > kMaxLabels)
@@ -695,35 +713,106 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
     fail(R3DG_ERROR_INVALID_ARGUMENT, "stereo: a tile of " + std::to_string(A.max_tile_cells) +
                                           " cells exceeds the 2^31 cells a tile volume may hold on the GPU; "
                                           "use a smaller tile_size or memory_budget");
+  A.max_row_chunks = *std::max_element(trow.begin(), trow.end());
+  if (A.max_row_chunks >= kMaxRowChunks)
+    fail(R3DG_ERROR_INVALID_ARGUMENT, "stereo: a tile row of 2^28 cells or more is not supported on the GPU; use a "
+                                      "smaller tile_size");
   upload(c, A.dtiles, td);
   layout_timer.reset();
   return A;
 }
 
-// Costs and the 8 path scans of tiles [t0, t1) (their rows are consecutive).
-// With `sum_slices` the slices of side-by-side scans are added into S.
-Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, bool sum_slices) {
+int path_scanlines(int p, int w, int h) { return p < 2 ? h : (p < 4 ? w : w + h - 1); }
+
+// How a chunk of tiles is aggregated.  kFull: all its pixels have all labels
+// (k_full: a plane of bytes per path, 9 bytes per cell with the costs).
+// kSweep: row sweeps for the vertical and diagonal paths, path scans for the
+// horizontal ones (k_sweep, k_path: at least 7 bytes per cell).  kScan: a path
+// scan per path, summed in S (3 bytes per cell), where the memory left holds
+// no more or the other kernels do not apply.
+enum class Aggregate { kFull, kSweep, kScan };
+
+// Sweeps of one path each instead of three where the tiles are fewer than
+// this: their blocks would leave most of the device idle.
+constexpr int kSweepTiles = 96;
+
+// Costs and the 8 paths of tiles [t0, t1) (their rows are consecutive).  With
+// `sum_slices` the slices of side-by-side scans are added into the first.
+Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind, bool sum_slices) {
   Chunk ch;
   ch.t0 = t0;
   ch.t1 = t1;
   const int nt = t1 - t0;
   std::vector<TileDesc> td(A.td.begin() + t0, A.td.begin() + t1);
   std::vector<std::uint64_t> row_prefix(static_cast<std::size_t>(nt));
-  const std::uint64_t cell0 = td.front().cell_base, row0 = td.front().row_base;
+  const std::uint64_t row0 = td.front().row_base;
   int max_num = 16;
   for (int t = 0; t < nt; ++t) {
     TileDesc& T = td[std::size_t(t)];
-    T.cell_base -= cell0;
     row_prefix[std::size_t(t)] = T.row_base - row0;
     ch.cells += A.tcells[std::size_t(t0 + t)];
     ch.rows += std::uint64_t(T.h);
     ch.px += std::uint64_t(T.w) * std::uint64_t(T.h);
     max_num = std::max(max_num, T.max_num);
   }
-  // Group prefixes of the 8 paths (kScanPerWave scanlines per wave).
-  std::vector<std::uint64_t> gp(8 * (std::size_t(nt) + 1), 0);
+  // Volumes in the order of the tiles' work, largest first, so that the sweeps
+  // end with short ones.
+  std::vector<std::int32_t> order(static_cast<std::size_t>(nt));
+  for (int t = 0; t < nt; ++t) order[std::size_t(t)] = t;
+  std::stable_sort(order.begin(), order.end(), [&](std::int32_t a, std::int32_t b) {
+    return A.tcells[std::size_t(t0 + a)] > A.tcells[std::size_t(t0 + b)];
+  });
+  std::uint64_t base = 0;
+  for (const std::int32_t t : order) {
+    td[std::size_t(t)].cell_base = base;
+    base += A.tcells[std::size_t(t0 + t)];
+  }
+  ch.stride = (ch.cells + kSPad + 127) / 128 * 128;
+  const auto free_bytes = [&] { return c.arena.budget() > c.arena.live() ? c.arena.budget() - c.arena.live() : 0; };
+
+  // Sweeps of one path (i = 0) for the first `heavy` tiles in order, of three
+  // (i = 1) for the rest.  Heavy are all tiles where there are few, else those
+  // whose mean row exceeds the LDS rows of a three-path sweep: one block would
+  // still sweep them when the others are done.  Scratch rows (for rows with
+  // more wide pixels than LDS holds) for as many blocks at once as a sixteenth
+  // of the memory left holds rows for.
+  struct Sweep {
+    SweepPlan plan;
+    std::uint64_t units, blocks, block_words;
+    DBuf<std::uint32_t> scratch;
+  };
+  std::array<Sweep, 2> sw{};
+  int heavy = 0;
+  if (kind == Aggregate::kSweep) {
+    sw[0].plan = sweep_plan(1, A.max_w, A.max_row_chunks);
+    sw[1].plan = sweep_plan(3, A.max_w, A.max_row_chunks);
+    const auto mean_words = [&](std::int32_t t) {
+      const TileDesc& T = td[std::size_t(t)];
+      return A.tcells[std::size_t(t0 + t)] / std::uint64_t(T.h) / 2 + std::uint64_t(T.w);
+    };
+    while (heavy < nt && (nt < kSweepTiles || mean_words(order[std::size_t(heavy)]) > std::uint64_t(sw[1].plan.cap))) ++heavy;
+    std::uint64_t hcells = 0;
+    for (int k = 0; k < heavy; ++k) hcells += A.tcells[std::size_t(t0 + order[std::size_t(k)])];
+    if (8 * ch.cells + 8 * hcells > free_bytes() / 2) heavy = 0;
+    sw[0].units = std::uint64_t(heavy) * 6;
+    sw[1].units = std::uint64_t(nt - heavy) * 2;
+    for (int i = 0; i < 2; ++i) {
+      Sweep& s = sw[std::size_t(i)];
+      s.block_words = 2 * (i == 0 ? 1 : 3) * std::uint64_t(s.plan.swords);
+      s.blocks = std::min<std::uint64_t>(std::uint64_t(s.plan.blocks), s.units);
+      if (s.block_words > 0) s.blocks = std::min(s.blocks, free_bytes() / 64 / s.block_words);
+      if (s.units > 0 && (!s.plan.ok || s.blocks < 1)) kind = Aggregate::kScan;
+    }
+  }
+  const bool sweep = kind == Aggregate::kSweep, full = kind == Aggregate::kFull;
+  // Path scans: all eight, or the horizontal two beside the sweeps.
+  const int npaths = full ? 0 : (sweep ? 2 : kPaths);
+  // Group prefixes of the path scans (kScanPerWave scanlines per wave), of the
+  // full-range scans, and the tiles in the order of their work, largest first,
+  // so that the sweeps end with short ones.
+  std::vector<std::uint64_t> gp(std::size_t(npaths) * (std::size_t(nt) + 1), 0);
   std::uint64_t max_groups = 0, sum_groups = 0;
-  for (int p = 0; p < 8; ++p) {
+  for (int p = 0; p < npaths; ++p) {
     std::uint64_t* g = gp.data() + std::size_t(p) * (std::size_t(nt) + 1);
     for (int t = 0; t < nt; ++t)
       g[t + 1] = g[t] + std::uint64_t((path_scanlines(p, td[std::size_t(t)].w, td[std::size_t(t)].h) +
@@ -731,122 +820,216 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, bool sum_slice
     max_groups = std::max(max_groups, g[nt]);
     sum_groups += g[nt];
   }
-  // Tiles, row prefix, group prefixes and the 8 work-queue counters (zero)
-  // in one upload.
-  DView<std::uint64_t> dgp;
+  std::vector<std::uint64_t> fp;
+  int lps = 0;
+  if (full) {
+    for (const TileDesc& T : td) lps = std::max(lps, full_lanes(A.full[std::size_t(T.job)]));
+    const int per = 64 / lps;
+    fp.assign(std::size_t(nt) + 1, 0);
+    for (int t = 0; t < nt; ++t) {
+      const TileDesc& T = td[std::size_t(t)];
+      fp[std::size_t(t) + 1] = fp[std::size_t(t)] + std::uint64_t(2 * ((T.h + per - 1) / per) + 6 * ((T.w + per - 1) / per));
+    }
+  }
+  // Everything the launches read, and the work-queue counters (zero: the
+  // paths', then the sweeps'), in one upload.
+  DView<std::uint64_t> dgp, dfp;
+  DView<std::int32_t> dorder;
   DView<std::uint32_t> queues;
   {
     UploadPack pk;
-    const std::size_t ot = pk.add(td), orp = pk.add(row_prefix), og = pk.add(gp), oq = pk.zeros(8 * sizeof(std::uint32_t));
+    const std::size_t ot = pk.add(td), orp = pk.add(row_prefix), og = pk.add(gp), of = pk.add(fp), oo = pk.add(order);
+    const std::size_t oq = pk.zeros((kPaths + 2) * sizeof(std::uint32_t));
     upload(c, ch.meta, pk.host);
     ch.dtiles = view<TileDesc>(ch.meta, ot);
     ch.drow_prefix = view<std::uint64_t>(ch.meta, orp);
     dgp = view<std::uint64_t>(ch.meta, og);
+    dfp = view<std::uint64_t>(ch.meta, of);
+    dorder = view<std::int32_t>(ch.meta, oo);
     queues = view<std::uint32_t>(ch.meta, oq);
   }
-  ch.S = DBuf<std::uint16_t>(c.arena, ch.cells + kSPad);
-  // Scratch rows of the persistent waves (pixels wider than the LDS rows) and
-  // the work-queue counters of the 8 launches.
-  // (a multiple of 4: launches use whole blocks of 4 waves, one slot each)
+  ch.C = DBuf<std::uint8_t>(c.arena, ch.cells + kSPad);
+  DBuf<std::uint32_t> cmap;
+  // Scratch rows of the path scans' persistent waves (pixels wider than the
+  // LDS rows; a multiple of 4: launches use whole blocks of 4 waves, one slot
+  // each).
   const std::uint64_t resident = path_slots();
   const std::uint64_t slots = (std::min(resident, std::max<std::uint64_t>(max_groups, 1)) + 3) / 4 * 4;
-  // The scans run side by side on 2 or 3 streams (3 where their groups
-  // average less than the device holds), each stream summing its paths into a
-  // slice of its own, when the slices and their scratch rows fit the budget:
-  // a launch's last groups then overlap the next launch on another stream.
-  // Not 4: a process gets 4 hardware queues and 4 such streams were traced
-  // on 3 of them, so that one queue ran 4 launches in turn (measured: the
-  // 1080p pair's aggregation 5.0 ms with 4 streams, 4.7 ms with 3).
-  const std::uint64_t mean_groups = std::max<std::uint64_t>((sum_groups + 7) / 8, 1);
-  int ways = static_cast<int>(std::clamp<std::uint64_t>((resident + mean_groups - 1) / mean_groups, 2, 3));
-  const std::uint64_t slice_bytes =
-      (ch.cells + kSPad) * sizeof(std::uint16_t) + path_scratch_elems(slots, max_num) * sizeof(std::uint16_t);
-  const std::uint64_t free_bytes = c.arena.budget() > c.arena.live() ? c.arena.budget() - c.arena.live() : 0;
-  while (ways > 1 && std::uint64_t(ways - 1) * slice_bytes + (ch.cells + kSPad) > free_bytes / 2) --ways;
-  std::vector<DBuf<std::uint16_t>>& slices = ch.slices;
-  for (int w = 1; w < ways; ++w) slices.emplace_back(c.arena, ch.cells + kSPad);
-  DBuf<std::uint16_t> scratch(c.arena, std::size_t(ways) * path_scratch_elems(slots, max_num));
+  // Streams of the path scans.  Alone they run side by side on 2 or 3 streams
+  // (3 where their groups average less than the device holds), each stream
+  // summing its paths into a slice of its own, when the slices and their
+  // scratch rows fit the budget: a launch's last groups then overlap the next
+  // launch on another stream.  Not 4: a process gets 4 hardware queues and 4
+  // such streams were traced on 3 of them, so that one queue ran 4 launches in
+  // turn (measured: the 1080p pair's aggregation 5.0 ms with 4 streams, 4.7 ms
+  // with 3).  Beside the sweeps the two horizontal scans take one stream and
+  // one slice, or a stream and a slice each where the tiles are few.
+  int ways = 0;
+  if (full) {
+    ch.planes = DBuf<std::uint8_t>(c.arena, kPaths * ch.stride);
+  } else if (sweep) {
+    ways = heavy == nt ? 2 : 1;
+    ch.slices = 2 + ways;
+    ch.S = DBuf<std::uint16_t>(c.arena, std::size_t(ch.slices) * ch.stride);
+    if (heavy > 0) {
+      ch.xcells = heavy < nt ? td[std::size_t(order[std::size_t(heavy)])].cell_base : ch.cells;
+      ch.xstride = (ch.xcells + kSPad + 127) / 128 * 128;
+      ch.X = DBuf<std::uint16_t>(c.arena, std::size_t(kPaths - ch.slices) * ch.xstride);
+    }
+    cmap = DBuf<std::uint32_t>(c.arena, ch.cells / kLabelAlign + 1);
+    for (Sweep& s : sw)
+      if (s.units > 0 && s.block_words > 0) s.scratch = DBuf<std::uint32_t>(c.arena, s.blocks * s.block_words);
+  } else {
+    const std::uint64_t mean_groups = std::max<std::uint64_t>((sum_groups + 7) / 8, 1);
+    ways = static_cast<int>(std::clamp<std::uint64_t>((resident + mean_groups - 1) / mean_groups, 2, 3));
+    const std::uint64_t slice_bytes = (ch.stride + path_scratch_elems(slots, max_num)) * sizeof(std::uint16_t);
+    const std::uint64_t room = free_bytes() - std::min(free_bytes(), 2 * ch.stride);
+    while (ways > 1 && std::uint64_t(ways - 1) * slice_bytes > room / 2) --ways;
+    ch.slices = ways;
+    ch.S = DBuf<std::uint16_t>(c.arena, std::size_t(ways) * ch.stride);
+  }
+
+  const std::size_t scratch_elems = npaths > 0 ? path_scratch_elems(slots, max_num) : 0;
+  DBuf<std::uint16_t> scratch(c.arena, std::max<std::size_t>(std::size_t(ways) * scratch_elems, 1));
 
   // Matching costs of every cell (timed with the other cost preparation).
-  DBuf<std::uint8_t> C(c.arena, ch.cells + kSPad);
   {
     const StageTimer timer(c, R3DG_STAGE_PREPARE);
-    launch_cost(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), nt, ch.rows, A.bcorr.get(), A.pix.get(),
-                C.get(), c.stream);
+    launch_cost(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), nt, ch.rows, A.rowbase.get(), A.pix.get(),
+                ch.C.get(), cmap.get(), c.stream);
     check_launch();
   }
-  // Aggregation: 8 path launches over the chunk's tiles; path p runs on
-  // stream p % ways and adds into that stream's slice.
-  {
-    const StageTimer timer(c, R3DG_STAGE_AGGREGATE);
-    std::array<hipStream_t, 4> st{c.stream, nullptr, nullptr, nullptr};
-    std::array<hipEvent_t, 4> ev{};
-    if (ways > 1) {
-      ev[0] = c.event();
-      hip_check(hipEventRecord(ev[0], c.stream), "hipEventRecord");
-      for (int w = 1; w < ways; ++w) {
-        st[std::size_t(w)] = c.side_stream(w - 1);
-        hip_check(hipStreamWaitEvent(st[std::size_t(w)], ev[0], 0), "hipStreamWaitEvent");
-      }
-    }
-    for (int p = 0; p < 8; ++p) {
-      const int w = p % ways;
-      const std::size_t o8 = std::size_t(p) * (std::size_t(nt) + 1);
-      std::uint16_t* S = w == 0 ? ch.S.get() : slices[std::size_t(w - 1)].get();
-      launch_sgm_path(p, A.djobs.get(), ch.dtiles.get(), dgp.get() + o8, nt, gp[o8 + std::size_t(nt)],
-                      A.bcorr.get(), A.pix.get(), C.get(), S, scratch.get() + std::size_t(w) * path_scratch_elems(slots, max_num),
-                      slots, max_num, queues.get() + p, p >= ways, st[std::size_t(w)]);
-      check_launch();
-    }
-    if (ways > 1) {
-      for (int w = 1; w < ways; ++w) {
-        ev[std::size_t(w)] = c.event();
-        hip_check(hipEventRecord(ev[std::size_t(w)], st[std::size_t(w)]), "hipEventRecord");
-        hip_check(hipStreamWaitEvent(c.stream, ev[std::size_t(w)], 0), "hipStreamWaitEvent");
-      }
-      if (sum_slices) {
-        const std::vector<const std::uint16_t*> src = ch.parts();
-        launch_sum_u16(ch.S.get(), src.data(), ways, ch.cells, c.stream);
-        check_launch();
-        slices.clear();
-      }
-      for (int w = 0; w < ways; ++w) c.event_pool.push_back(ev[std::size_t(w)]);
+  const StageTimer timer(c, R3DG_STAGE_AGGREGATE);
+  if (full) {
+    FullArgs fa{};
+    fa.jobs = A.djobs.get();
+    fa.tiles = ch.dtiles.get();
+    fa.gprefix = dfp.get();
+    fa.ntiles = nt;
+    fa.groups = fp.back();
+    fa.C = ch.C.get();
+    fa.M = ch.planes.get();
+    fa.mstride = ch.stride;
+    launch_full(fa, lps, c.stream);
+    check_launch();
+    c.agg_launches += 1;
+    // Per cell and path its cost read and its byte stored; per tile pixel and
+    // path its intensity.
+    c.agg_bytes += 16 * ch.cells + 16 * ch.px;
+    return ch;
+  }
+  // The context's stream takes the first sweeps; the path scans and the other
+  // sweeps run beside them on side streams.
+  const bool both = sweep && heavy > 0 && heavy < nt;
+  const int side = sweep ? ways + (both ? 1 : 0) : ways - 1;
+  std::array<hipStream_t, 4> st{c.stream, nullptr, nullptr, nullptr};
+  std::array<hipEvent_t, 4> ev{};
+  if (side > 0) {
+    ev[0] = c.event();
+    hip_check(hipEventRecord(ev[0], c.stream), "hipEventRecord");
+    for (int w = 1; w <= side; ++w) {
+      st[std::size_t(w)] = c.side_stream(w - 1);
+      hip_check(hipStreamWaitEvent(st[std::size_t(w)], ev[0], 0), "hipStreamWaitEvent");
     }
   }
-  c.agg_launches += 8;
-  // Algorithmic bytes of the 8 launches: per cell C read 8 x 1, S written
-  // 8 x 2 and read 8 - ways times x 2 (the first scan of each stream only
-  // writes its slice); per tile pixel and path its record (8) and intensity (2).
-  c.agg_bytes += std::uint64_t(40 - 2 * ways) * ch.cells + 80 * ch.px;
+  for (int i = 0; i < 2 && sweep; ++i) {
+    Sweep& s = sw[std::size_t(i)];
+    if (s.units == 0) continue;
+    SweepArgs sa{};
+    sa.jobs = A.djobs.get();
+    sa.tiles = ch.dtiles.get();
+    sa.order = dorder.get() + (i == 0 ? 0 : heavy);
+    sa.units = static_cast<std::uint32_t>(s.units);
+    sa.rowbase = A.rowbase.get();
+    sa.pix = A.pix.get();
+    sa.cmap = cmap.get();
+    sa.C = ch.C.get();
+    // Downwards into slice 0, upwards into slice 1; the diagonals of one-path
+    // sweeps into X.
+    for (int u = 0; u < 6; ++u)
+      sa.S[u] = u < 2 ? ch.S.get() + std::uint64_t(u) * ch.stride
+                      : ch.X.get() + std::uint64_t(u - 2) * ch.xstride;
+    sa.scratch = s.scratch.get();
+    sa.queue = queues.get() + kPaths + i;
+    sa.wpad = s.plan.wpad;
+    sa.cap = s.plan.cap;
+    sa.swords = s.plan.swords;
+    launch_sweep(sa, i == 0 ? 1 : 3, s.plan, s.blocks, st[std::size_t(both && i == 1 ? side : 0)]);
+    check_launch();
+    c.agg_launches += 1;
+  }
+  const int slice0 = sweep ? ch.slices - ways : 0;
+  for (int p = 0; p < npaths; ++p) {
+    const int w = p % ways;
+    const std::size_t o8 = std::size_t(p) * (std::size_t(nt) + 1);
+    launch_sgm_path(p, A.djobs.get(), ch.dtiles.get(), dgp.get() + o8, nt, gp[o8 + std::size_t(nt)], A.rowbase.get(),
+                    A.pix.get(), ch.C.get(), ch.S.get() + std::uint64_t(slice0 + w) * ch.stride,
+                    scratch.get() + std::size_t(w) * scratch_elems, slots, max_num, queues.get() + p, p >= ways,
+                    st[std::size_t(sweep ? w + 1 : w)]);
+    check_launch();
+  }
+  for (int w = 1; w <= side; ++w) {
+    ev[std::size_t(w)] = c.event();
+    hip_check(hipEventRecord(ev[std::size_t(w)], st[std::size_t(w)]), "hipEventRecord");
+    hip_check(hipStreamWaitEvent(c.stream, ev[std::size_t(w)], 0), "hipStreamWaitEvent");
+  }
+  for (int w = 0; w <= side && side > 0; ++w) c.event_pool.push_back(ev[std::size_t(w)]);
+  if (sum_slices && ch.slices > 1) {
+    launch_sum_u16(ch.S.get(), ch.source(), ch.cells, c.stream);
+    check_launch();
+    ch.slices = 1;
+  }
+  c.agg_launches += std::uint64_t(npaths);
+  // Per cell the cost bytes read, S written and read back (the first scan of
+  // each slice only writes it) and the sweeps' map; per tile pixel and pass
+  // over it its record.
+  if (sweep) {
+    const std::uint64_t scans = (2 + 2 + (ways == 1 ? 2 + 2 + 2 : 2 + 2)) * ch.cells + 16 * ch.px;
+    c.agg_bytes += scans + (2 + 4) * ch.cells + ch.cells / 2 + 16 * ch.px +
+                   (ch.xcells > 0 ? (4 + 8 + 1) * ch.xcells : 0);
+  } else {
+    c.agg_bytes += std::uint64_t(40 - 2 * ways) * ch.cells + 64 * ch.px;
+  }
   return ch;
 }
 
-// Tile ranges whose volumes (S, costs, scratch) fit the device memory left
-// in the context's budget, one chunk when everything fits.
-std::vector<std::array<int, 2>> chunk_tiles(const Context& c, const Aggregation& A) {
+// Consecutive tiles aggregated together, sized to the device memory left in
+// the context's budget (one range when everything fits): at most a twentieth
+// of it in cells where planes or sweep slices are kept, at most a quarter (S,
+// C and room for scratch rows and per-tile data) where only path scans fit;
+// at most 4 G cells, enough to fill the device, so that the volume blocks are
+// reused from range to range rather than freed and mapped again.
+struct TileRange {
+  int t0, t1;
+  Aggregate kind;
+};
+std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
   const std::uint64_t free_bytes = c.arena.budget() > c.arena.live() ? c.arena.budget() - c.arena.live() : 0;
-  // 3 bytes per cell (S and C) with room for scratch rows and per-tile data;
-  // at most 4 G cells, enough to fill the device, so that the volume blocks
-  // are reused from chunk to chunk rather than freed and mapped again.
-  const std::uint64_t cap = std::max(A.max_tile_cells, std::min(free_bytes / 4, std::uint64_t{4} << 30));
-  std::vector<std::array<int, 2>> out;
+  const bool roomy = A.max_tile_cells <= free_bytes / 20;
+  const bool planes = roomy && A.p2max <= kMaxByteP2;
+  const std::uint64_t cap =
+      std::max(A.max_tile_cells, std::min(free_bytes / (roomy ? 20 : 4), std::uint64_t{4} << 30));
+  std::vector<TileRange> out;
   const int nt = static_cast<int>(A.td.size());
-  int t0 = 0;
   std::uint64_t cells = 0;
   for (int t = 0; t < nt; ++t) {
-    if (t > t0 && cells + A.tcells[std::size_t(t)] > cap) {
-      out.push_back({t0, t});
-      t0 = t;
+    const auto job = std::size_t(A.td[std::size_t(t)].job);
+    const Aggregate kind = !roomy ? Aggregate::kScan
+                           : planes && A.full[job] > 0 && full_lanes(A.full[job]) > 0 ? Aggregate::kFull
+                                                                                      : Aggregate::kSweep;
+    const std::uint64_t n = A.tcells[std::size_t(t)];
+    if (out.empty() || out.back().kind != kind || cells + n > cap) {
+      out.push_back({t, t, kind});
       cells = 0;
     }
-    cells += A.tcells[std::size_t(t)];
+    cells += n;
+    out.back().t1 = t + 1;
   }
-  if (nt > 0) out.push_back({t0, nt});
   return out;
 }
 
 // match_tiles (stereo_matcher.cpp:613-771) for several jobs at once.
-std::vector<TilesOut> match_tiles(Context& c, std::vector<Job>& jobs, const r3dg_options& o, SelectParams sp) {
+std::vector<TilesOut> match_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& o, SelectParams sp) {
   const int nj = static_cast<int>(jobs.size());
   Aggregation A = layout_jobs(c, jobs, o);
   const std::uint64_t total_px = A.total_px;
@@ -855,15 +1038,13 @@ std::vector<TilesOut> match_tiles(Context& c, std::vector<Job>& jobs, const r3dg
   DBuf<float> tdisp(c.arena, std::max<std::uint64_t>(total_px, 1)), tconf(c.arena, std::max<std::uint64_t>(total_px, 1));
   DBuf<std::int16_t> tlab;
   if (any_labels) tlab = DBuf<std::int16_t>(c.arena, std::max<std::uint64_t>(total_px, 1));
-  for (const auto& [t0, t1] : chunk_tiles(c, A)) {
+  for (const auto& [t0, t1, kind] : chunk_tiles(c, A)) {
     poll_cancel(c);
-    Chunk ch = aggregate_tiles(c, A, t0, t1, false);
+    Chunk ch = aggregate_tiles(c, A, t0, t1, kind, false);
     // Selection into per-tile maps.
     const StageTimer timer(c, R3DG_STAGE_SELECT);
-    const std::vector<const std::uint16_t*> parts = ch.parts();
-    launch_select(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), t1 - t0, ch.rows, A.bcorr.get(),
-                  A.pix.get(), parts.data(), static_cast<int>(parts.size()), sp, A.max_w, A.max_D, tdisp.get(),
-                  tconf.get(), tlab.get(), c.stream);
+    launch_select(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), t1 - t0, ch.rows, A.rowbase.get(),
+                  A.pix.get(), ch.source(), sp, A.max_w, A.max_D, tdisp.get(), tconf.get(), tlab.get(), c.stream);
     check_launch();
   }
   std::vector<TilesOut> out(static_cast<std::size_t>(nj));
@@ -909,6 +1090,21 @@ std::vector<TilesOut> match_tiles(Context& c, std::vector<Job>& jobs, const r3dg
   }
   // dgrids returns to the arena here; later uses of the same memory are
   // ordered after the blends on the context's stream.
+  return out;
+}
+
+// The same, the jobs whose pixels have all labels taken first: they and the
+// others are aggregated by different kernels.
+std::vector<TilesOut> match_tiles(Context& c, std::vector<Job>& jobs, const r3dg_options& o, SelectParams sp) {
+  std::vector<std::size_t> at;
+  for (const bool full : {true, false}) {
+    for (std::size_t j = 0; j < jobs.size(); ++j)
+      if ((jobs[j].ranges == nullptr) == full) at.push_back(j);
+  }
+  std::vector<Job> sorted;
+  for (const std::size_t j : at) sorted.push_back(std::move(jobs[j]));
+  std::vector<TilesOut> got = match_jobs(c, sorted, o, sp), out(jobs.size());
+  for (std::size_t k = 0; k < at.size(); ++k) out[at[k]] = std::move(got[k]);
   return out;
 }
 
@@ -2770,9 +2966,9 @@ int32_t r3dg_cost_volume(r3dg_ctx* h, r3dg_image left, r3dg_image right, int32_t
     jobs[0].ranges = has ? &rg : nullptr;
     jobs[0].dmin = disparity_min;
     jobs[0].D = D;
-    Aggregation A = layout_jobs(c, jobs, one, 31);  // rows contiguous: the reference's packed order
+    Aggregation A = layout_jobs(c, jobs, one);
     if (A.total_cells != out_cells) fail(R3DG_ERROR_INTERNAL, "cost_volume: cell count mismatch");
-    const Chunk ch = aggregate_tiles(c, A, 0, static_cast<int>(A.td.size()), true);
+    const Chunk ch = aggregate_tiles(c, A, 0, static_cast<int>(A.td.size()), Aggregate::kScan, true);
     const hipMemcpyKind kind = out_memory == R3DG_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     if (out_cells > 0) hip_check(hipMemcpyAsync(out, ch.S.get(), out_cells * 2, kind, c.stream), "download");
     sync(c);

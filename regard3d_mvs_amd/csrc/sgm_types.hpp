@@ -8,15 +8,16 @@
 // and one launch can cover the tiles of many jobs (both directions of a level,
 // or every pair of a batch).
 //
-// HBM layout of the aggregated costs S (uint16) and the costs C (uint8): every
-// tile owns a contiguous volume at cell_base, stored band by band (TileDesc
-// below); a pixel's labels follow each other, at the cell offset held in its
-// pixel record pix[px_base + y*w + x] (the TileLabels ranges of
-// stereo_matcher.cpp:172-224).  Label counts are multiples of 16, so every
-// pixel's labels start on a 32-byte boundary of S.
+// HBM layout of the costs C (uint8), of the paths' planes (uint8) and of the
+// aggregated costs S (uint16): every tile owns a contiguous volume at
+// cell_base, its rows one after the other (rowbase[row_base + y] is row y's
+// first cell), a row's pixels in order; a pixel's labels follow each other, at
+// the offset held in its pixel record pix[px_base + y*w + x] (the TileLabels
+// ranges of stereo_matcher.cpp:172-224).  Label counts are multiples of 16, so
+// every pixel's labels are whole chunks of 16 cells.
 //
-// Pixel record (uint64): bits 0-31 cell offset inside the tile row, bits 32-47
-// first label `lo`, bits 48-63 label count `num`.
+// Pixel record (uint64): bits 0-23 chunk offset inside the tile row, bits
+// 24-31 label count / 16, bits 32-47 first label `lo`, bits 48-63 intensity.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,14 +27,19 @@
 namespace r3dg {
 
 constexpr int kLabelAlign = 16;
-constexpr int kMaxLabels = 4000;  // per pixel and level: the path kernel keeps label count / 16 in 8 bits
+constexpr int kMaxLabels = 4000;           // per pixel and level: a record keeps label count / 16 in 8 bits
+constexpr std::uint32_t kMaxRowChunks = 1U << 24;  // a record keeps a row's chunk offsets in 24 bits
+constexpr int kPaths = 8;
+constexpr int kMaxByteP2 = 255;  // largest P2 with which a path's M = L - C is a byte
 
-__host__ __device__ constexpr std::uint64_t pix_record(std::uint32_t off, int lo, int num) {
-  return std::uint64_t(off) | (std::uint64_t(std::uint16_t(lo)) << 32) | (std::uint64_t(std::uint16_t(num)) << 48);
+__host__ __device__ constexpr std::uint64_t pix_record(std::uint64_t off, int lo, int num, int val) {
+  return ((off / kLabelAlign) & 0xFFFFFFU) | (std::uint64_t((num / kLabelAlign) & 0xFF) << 24) |
+         (std::uint64_t(std::uint16_t(lo)) << 32) | (std::uint64_t(std::uint16_t(val)) << 48);
 }
-__host__ __device__ constexpr std::uint32_t pix_off(std::uint64_t r) { return std::uint32_t(r); }
+__host__ __device__ constexpr std::uint32_t pix_off(std::uint64_t r) { return std::uint32_t(r & 0xFFFFFFU) * kLabelAlign; }
+__host__ __device__ constexpr int pix_num(std::uint64_t r) { return int((r >> 24) & 0xFFU) * kLabelAlign; }
 __host__ __device__ constexpr int pix_lo(std::uint64_t r) { return int((r >> 32) & 0xFFFFU); }
-__host__ __device__ constexpr int pix_num(std::uint64_t r) { return int((r >> 48) & 0xFFFFU); }
+__host__ __device__ constexpr int pix_val(std::uint64_t r) { return int(r >> 48); }
 constexpr int kMaxLevels = 13;
 
 struct JobDesc {
@@ -65,10 +71,6 @@ struct JobDesc {
   std::uint16_t lut[256];    // P2 by 8-bit intensity step (stereo_matcher.cpp:69-79)
 };
 
-// Cells of a tile are stored band by band: columns [b << band_shift,
-// (b + 1) << band_shift) of every row, rows in order, then the next band.
-// Pixel (x, y)'s labels start at cell_base + bcorr[band_base + (x >> band_shift)
-// * h + y] + off(x, y), off being the pixel record's offset in its row.
 struct TileDesc {
   std::int32_t x0, y0, w, h;  // in the job's base image
   std::int32_t job;
@@ -76,9 +78,8 @@ struct TileDesc {
   std::uint64_t cell_base;    // first cell of the tile in S
   std::uint64_t px_base;      // first tile pixel in per-pixel arrays
   std::uint64_t row_base;     // first tile row in per-row arrays
-  std::int32_t band_shift;    // log2 of the band width (31: one band per row)
-  std::int32_t nbands;
-  std::uint64_t band_base;    // first (band, row) entry in bcorr
+  std::uint32_t cells;        // cells of the tile
+  std::uint32_t reserved;
 };
 
 // Tile grid of one job for blending (stereo_matcher.cpp:688-766): tile (i, j)
