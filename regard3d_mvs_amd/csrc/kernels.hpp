@@ -125,7 +125,7 @@ void launch_tile_cells(const TileDesc* tiles, int ntiles, const std::uint64_t* r
 constexpr int kLanesPerScan = 8;
 constexpr int kScanPerWave = 64 / kLanesPerScan;
 // Matching costs (u8) of every tile cell into C (same cell indexing as S);
-// cmap (may be null) receives per chunk of 16 cells its column (bits 0-15) and
+// cmap receives per chunk of 16 cells its column (bits 0-15) and
 // its place in the pixel (bits 16-31).
 void launch_cost(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
                  std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix, std::uint8_t* C,
@@ -206,9 +206,9 @@ struct SumSrc {
 void launch_sum_u16(std::uint16_t* dst, const SumSrc& src, std::uint64_t cells, hipStream_t s);
 // WTA + sub-pixel + checks of every tile row into per-tile-pixel results.
 void launch_select(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
-                   std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix, const SumSrc& src,
-                   SelectParams p, int max_w, int max_D, float* tdisp, float* tconf, std::int16_t* tlab,
-                   hipStream_t s);
+                   std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix,
+                   const std::uint32_t* cmap, const SumSrc& src, SelectParams p, int max_w, int max_D, float* tdisp,
+                   float* tconf, std::int16_t* tlab, hipStream_t s);
 // Packs two valid-interval arrays ([h][2] each) into rows4 ([h][4]).
 void launch_pack_rows(const std::int32_t* base, const std::int32_t* partner, int h, std::int32_t* rows4,
                       hipStream_t s);

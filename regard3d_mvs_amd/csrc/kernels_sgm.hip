@@ -385,7 +385,7 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
       w[q] = v;
     }
     *reinterpret_cast<uint4*>(out + 16 * std::size_t(k)) = make_uint4(w[0], w[1], w[2], w[3]);
-    if (cmap != nullptr) mout[k] = static_cast<std::uint32_t>(xa) | static_cast<std::uint32_t>(jb / kLabelAlign) << 16;
+    mout[k] = static_cast<std::uint32_t>(xa) | static_cast<std::uint32_t>(jb / kLabelAlign) << 16;
   };
   if (staged) {
     const bool mapped = chunks <= static_cast<std::uint32_t>(kMap);
@@ -438,14 +438,6 @@ __device__ __forceinline__ std::uint32_t min8(std::uint32_t v) {
   v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, false)));
   v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xF, 0xF, false)));
   return v;
-}
-
-// Min over the four lanes of a quad (DPP quad swaps).
-__device__ __forceinline__ std::uint32_t quad_min(std::uint32_t v) {
-  const int i = static_cast<int>(v);
-  v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(i, i, 0xB1, 0xF, 0xF, false)));
-  const int j = static_cast<int>(v);
-  return min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(j, j, 0x4E, 0xF, 0xF, false)));
 }
 
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
@@ -1397,99 +1389,77 @@ __device__ __forceinline__ float subpixel_offset(int method, float sm, float s0,
   return delta < -0.5F ? -0.5F : (0.5F < delta ? 0.5F : delta);
 }
 
-// select_disparities (stereo_matcher.cpp:446-525) for one tile row per block,
-// four lanes (a quad) per pixel.  Lane q of a quad holds labels
-// [32 i + 8 q, 32 i + 8 q + 8) of chunk i, so a quad reads 64 contiguous
-// bytes per chunk; the first two chunks stay in registers for the second
-// pass of the winner-takes-all (sgm_kernels.cpp:405-426).
-// Minimum of (value << 16 | label) over the 8 labels of a chunk word group,
-// labels k0..k0+7: the lowest value, the first label on ties.
-__device__ __forceinline__ std::uint32_t key_min(const uint4& q, int k0, std::uint32_t m) {
-  const std::uint32_t w[4] = {q.x, q.y, q.z, q.w};
+// Minimum of (value << 16 | label) over the 16 packed values of a chunk whose
+// first label is k0: the lowest value, the first label on ties.
+__device__ __forceinline__ std::uint32_t chunk_key(const std::uint32_t (&V)[8], std::uint32_t k0) {
+  std::uint32_t m = 0xFFFFFFFFU;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const std::uint32_t v = (w[e >> 1] >> ((e & 1) * 16)) & 0xFFFFU;
-    m = min(m, (v << 16) | static_cast<std::uint32_t>(k0 + e));
+  for (int j = 0; j < 8; ++j) {
+    m = min(m, (V[j] << 16) | (k0 + 2U * j));
+    m = min(m, (V[j] & 0xFFFF0000U) | (k0 + 2U * j + 1U));
   }
   return m;
 }
 
-// Inserts the keys (value << 16 | label) of labels k0..k0+7 into the sorted
-// four smallest keys t0 <= t1 <= t2 <= t3.
-__device__ __forceinline__ void top4(const uint4& q, int k0, std::uint32_t& t0, std::uint32_t& t1,
-                                     std::uint32_t& t2, std::uint32_t& t3) {
-  const std::uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    std::uint32_t c = (((w[e >> 1] >> ((e & 1) * 16)) & 0xFFFFU) << 16) | static_cast<std::uint32_t>(k0 + e);
-    std::uint32_t a = min(t0, c);
-    c = max(t0, c);
-    t0 = a;
-    a = min(t1, c);
-    c = max(t1, c);
-    t1 = a;
-    a = min(t2, c);
-    c = max(t2, c);
-    t2 = a;
-    t3 = min(t3, c);
-  }
-}
-
-// Lowest value of labels k0..k0+7 outside [kb - 1, kb + 1].
-__device__ __forceinline__ std::uint32_t outside_min(const uint4& q, int k0, int kb, std::uint32_t m) {
-  const std::uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const std::uint32_t v = (w[e >> 1] >> ((e & 1) * 16)) & 0xFFFFU;
-    const int k = k0 + e;
-    m = k + 1 < kb || k > kb + 1 ? min(m, v) : m;
-  }
-  return m;
-}
-
-// Label k of a lane's group of 8 starting at k0 (0xFFFFFFFF when the group
-// does not hold k).
-__device__ __forceinline__ std::uint32_t group_value(const uint4& q, int k0, int k) {
-  const int e = k - k0;
-  const std::uint64_t a = (std::uint64_t(q.y) << 32) | q.x, b = (std::uint64_t(q.w) << 32) | q.z;
-  const std::uint32_t v = static_cast<std::uint32_t>((e < 4 ? a : b) >> ((e & 3) * 16)) & 0xFFFFU;
-  return e >= 0 && e < 8 ? v : 0xFFFFFFFFU;
-}
-
+// select_disparities (stereo_matcher.cpp:446-525): the winner-takes-all
+// (sgm_kernels.cpp:405-426) of one tile row (of kSelPx columns of it) per
+// block.  A thread takes chunks (16 labels of a pixel) of the row, whatever
+// pixel they belong to, and keeps their summed costs in registers: first the
+// chunks' best (cost, label) keys meet in LDS, then each chunk gives its best
+// cost outside the winner's neighbours and, where it holds them, the costs
+// next to the winner; last a thread per pixel fits and checks.  Chunks past
+// the kSelHeld a thread keeps are summed again for the second step.
+//
+// HBM-bound: the chunk's slices or planes once, 12 bytes per pixel (5.3 TB/s
+// with eight slices).  With a quad of lanes per pixel, 8 labels a lane, half
+// the lanes idled on pixels of 16 labels: selection of 1024x768 with 128
+// labels 1.17 ms, 0.70 ms here; of the 24 MP pair 5.75 ms, 5.38 ms.
+constexpr int kSelThreads = 256, kSelPx = 1024, kSelHeld = 4;
 template <bool kBytes>
-__global__ __launch_bounds__(256) void k_select(const JobDesc* __restrict__ jobs, const TileDesc* __restrict__ tiles,
+__global__ __launch_bounds__(kSelThreads) void k_select(const JobDesc* __restrict__ jobs,
+                                                const TileDesc* __restrict__ tiles,
                                                 const std::uint64_t* __restrict__ row_prefix, int ntiles,
                                                 const std::uint32_t* __restrict__ rowbase,
-                                                const std::uint64_t* __restrict__ pix, SumSrc S, SelectParams p,
+                                                const std::uint64_t* __restrict__ pix,
+                                                const std::uint32_t* __restrict__ cmap, SumSrc S, SelectParams p,
                                                 float* __restrict__ tdisp, float* __restrict__ tconf,
                                                 std::int16_t* __restrict__ tlab) {
-  constexpr int kStage = 1024;  // row pixels whose first cell and range are staged in LDS
-  __shared__ std::uint32_t soff[kStage];
-  __shared__ std::uint32_t srange[kStage];
+  __shared__ std::uint32_t best[kSelPx], second[kSelPx];
+  __shared__ std::uint16_t below[kSelPx], above[kSelPx];  // costs next to the winner
   extern __shared__ std::uint32_t keys[];
   const std::uint64_t r = blockIdx.x;
   const int t = find_tile_wave(row_prefix, ntiles, r);
   const TileDesc T = tiles[t];
+  const int x0 = static_cast<int>(blockIdx.y) * kSelPx, x1 = min(x0 + kSelPx, T.w);
+  if (x0 >= T.w) return;
   const JobDesc& J = jobs[T.job];
   const int y = static_cast<int>(r - row_prefix[t]);
-  const int Y = T.y0 + y;
+  const int Y = T.y0 + y, tid = static_cast<int>(threadIdx.x);
   const auto rows = gptr(J.rows4) + 4 * Y;
   const int lf = rows[0], ll = rows[1], rf = rows[2], rl = rows[3];
   const int xb = min(max(lf - T.x0, 0), T.w);
   const int xe = min(max(ll + 1 - T.x0, xb), T.w);
   const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + y];
+  const std::uint64_t px = T.px_base + std::uint64_t(y) * T.w;
   const int slices = T.cell_base < S.xcells ? kPaths : S.n;
-  // Aggregated costs of 8 labels: 8 C plus the eight paths' bytes M (L = C + M),
-  // or the sum of the slices of scans that ran side by side.
-  auto ld8 = [&](std::uint64_t c) {
+  const int D = J.D;
+  const std::uint32_t* rmap = cmap + row_cell / kLabelAlign;
+  // Chunks of the block's columns.
+  const std::uint64_t rec0 = pix[px + x0], rec1 = pix[px + x1 - 1];
+  const int ka = static_cast<int>(pix_off(rec0) / kLabelAlign);
+  const int kb = static_cast<int>((pix_off(rec1) + pix_num(rec1)) / kLabelAlign);
+
+  // Aggregated costs of chunk k: 8 C plus the eight paths' bytes M (L = C +
+  // M), or the sum of the slices of scans that ran side by side.
+  auto load = [&](int k, std::uint32_t (&V)[8]) __attribute__((always_inline)) {
+    const std::uint64_t cell = row_cell + 16 * std::uint64_t(k);
     if constexpr (kBytes) {
-      u32x2 v[kPaths + 1];
+      u32x4 v[kPaths + 1];
 #pragma unroll
-      for (int i = 0; i < kPaths; ++i) v[i] = *reinterpret_cast<const u32x2*>(S.m + i * S.mstride + c);
-      v[kPaths] = *reinterpret_cast<const u32x2*>(S.c + c);
-      std::uint32_t w[4];
+      for (int i = 0; i < kPaths; ++i) v[i] = *reinterpret_cast<const u32x4*>(S.m + i * S.mstride + cell);
+      v[kPaths] = *reinterpret_cast<const u32x4*>(S.c + cell);
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < 4; ++h) {
         // Even and odd labels as packed 16-bit sums (at most 16 x 255).
         std::uint32_t even = (v[kPaths][h] & 0x00FF00FFU) << 3, odd = ((v[kPaths][h] >> 8) & 0x00FF00FFU) << 3;
 #pragma unroll
@@ -1497,161 +1467,137 @@ __global__ __launch_bounds__(256) void k_select(const JobDesc* __restrict__ jobs
           even += v[i][h] & 0x00FF00FFU;
           odd += (v[i][h] >> 8) & 0x00FF00FFU;
         }
-        w[2 * h] = __builtin_amdgcn_perm(odd, even, 0x05040100U);
-        w[2 * h + 1] = __builtin_amdgcn_perm(odd, even, 0x07060302U);
+        V[2 * h] = __builtin_amdgcn_perm(odd, even, 0x05040100U);
+        V[2 * h + 1] = __builtin_amdgcn_perm(odd, even, 0x07060302U);
       }
-      return make_uint4(w[0], w[1], w[2], w[3]);
-    }
-    uint4 a = *reinterpret_cast<const uint4*>(S.p[0] + c);
-    for (int i = 1; i < slices; ++i) {
-      const uint4 v = *reinterpret_cast<const uint4*>(S.p[i] + c);
-      a.x = as_u32(as_pair(a.x) + as_pair(v.x));
-      a.y = as_u32(as_pair(a.y) + as_pair(v.y));
-      a.z = as_u32(as_pair(a.z) + as_pair(v.z));
-      a.w = as_u32(as_pair(a.w) + as_pair(v.w));
-    }
-    return a;
-  };
-  auto ld1 = [&](std::uint64_t c) {
-    if constexpr (kBytes) {
-      std::uint32_t a = 8U * S.c[c];
+    } else {
+      const u32x4* a = reinterpret_cast<const u32x4*>(S.p[0] + cell);
+      const u32x4 lo = a[0], hi = a[1];
 #pragma unroll
-      for (int i = 0; i < kPaths; ++i) a += S.m[i * S.mstride + c];
-      return a;
-    }
-    std::uint32_t a = S.p[0][c];
-    for (int i = 1; i < slices; ++i) a += S.p[i][c];
-    return a & 0xFFFFU;
-  };
-  const std::uint64_t px = T.px_base + std::uint64_t(y) * T.w;
-  const int D = J.D;
-  const int q = threadIdx.x & 3;
-  constexpr int kPerPass = 256 / 4;
-  const bool staged = T.w <= kStage;
-  if (staged) {
-    // Every load of a thread before its first LDS store (256 threads).
-    constexpr int kIt = kStage / 256;
-    std::uint64_t rv[kIt];
+      for (int j = 0; j < 4; ++j) {
+        V[j] = lo[j];
+        V[j + 4] = hi[j];
+      }
+      for (int i = 1; i < slices; ++i) {
+        const u32x4* b = reinterpret_cast<const u32x4*>(S.p[i] + cell);
+        const u32x4 bl = b[0], bh = b[1];
 #pragma unroll
-    for (int i = 0; i < kIt; ++i) {
-      const int x = static_cast<int>(threadIdx.x) + 256 * i;
-      rv[i] = x < T.w ? pix[px + x] : 0;
-    }
-#pragma unroll
-    for (int i = 0; i < kIt; ++i) {
-      const int x = static_cast<int>(threadIdx.x) + 256 * i;
-      if (x < T.w) {
-        soff[x] = pix_off(rv[i]);
-        srange[x] = static_cast<std::uint32_t>(pix_lo(rv[i])) | static_cast<std::uint32_t>(pix_num(rv[i])) << 16;
+        for (int j = 0; j < 4; ++j) {
+          V[j] = as_u32(as_pair(V[j]) + as_pair(bl[j]));
+          V[j + 4] = as_u32(as_pair(V[j + 4]) + as_pair(bh[j]));
+        }
       }
     }
-    __syncthreads();
-  }
-  // First cell, lo and label count of pixel x.
-  auto pixel = [&](int x, int& lo, int& n) {
-    if (staged) {
-      const std::uint32_t range = srange[x];
-      lo = static_cast<int>(range & 0xFFFFU);
-      n = static_cast<int>(range >> 16);
-      return row_cell + soff[x];
-    }
-    const std::uint64_t rec = pix[px + x];
-    lo = pix_lo(rec);
-    n = pix_num(rec);
-    return row_cell + pix_off(rec);
   };
 
+  for (int i = tid; i < x1 - x0; i += kSelThreads) {
+    best[i] = 0xFFFFFFFFU;
+    second[i] = 0xFFFFU;
+  }
   if (p.diagonal_lr) {
     // Right-image WTA along x - label (sgm_kernels.cpp:427-435): the first
     // (in x order) minimum of each diagonal, as a (cost, x) key minimum.
-    for (int i = threadIdx.x; i < T.w + D; i += blockDim.x) keys[i] = 0xFFFFFFFFU;
+    for (int i = tid; i < T.w + D; i += kSelThreads) keys[i] = 0xFFFFFFFFU;
     __syncthreads();
-    for (int x = xb + (threadIdx.x >> 2); x < xe; x += kPerPass) {
-      int lo, num;
-      const std::uint64_t s = pixel(x, lo, num);
-      for (int k0 = 8 * q; k0 < num; k0 += 32) {
-        const uint4 g = ld8(s + k0);
-        const std::uint32_t w[4] = {g.x, g.y, g.z, g.w};
+    const std::uint64_t recl = pix[px + T.w - 1];
+    const int kn = static_cast<int>((pix_off(recl) + pix_num(recl)) / kLabelAlign);
+    for (int k = tid; k < kn; k += kSelThreads) {
+      const std::uint32_t m = rmap[k];
+      const int x = static_cast<int>(m & 0xFFFFU);
+      if (x < xb || x >= xe) continue;
+      std::uint32_t V[8];
+      load(k, V);
+      const int d0 = x - pix_lo(pix[px + x]) - kLabelAlign * static_cast<int>(m >> 16) + D - 1;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const std::uint32_t v = (w[e >> 1] >> ((e & 1) * 16)) & 0xFFFFU;
-          atomicMin(&keys[x - (lo + k0 + e) + D - 1], (v << 16) | std::uint32_t(x));
-        }
+      for (int j = 0; j < 8; ++j) {
+        atomicMin(&keys[d0 - 2 * j], (V[j] << 16) | static_cast<std::uint32_t>(x));
+        atomicMin(&keys[d0 - 2 * j - 1], (V[j] & 0xFFFF0000U) | static_cast<std::uint32_t>(x));
       }
     }
-    __syncthreads();
   }
+  __syncthreads();
 
-  for (int base = 0; base < T.w; base += kPerPass) {
-    const int x = base + (threadIdx.x >> 2);
-    if (x >= T.w) continue;  // whole quads leave together
+  std::uint32_t V[kSelHeld][8], m[kSelHeld];
+#pragma unroll
+  for (int i = 0; i < kSelHeld; ++i) {
+    const int k = ka + tid + kSelThreads * i;
+    m[i] = k < kb ? rmap[k] : 0U;
+  }
+#pragma unroll
+  for (int i = 0; i < kSelHeld; ++i) {
+    const int k = ka + tid + kSelThreads * i;
+    if (k < kb) {
+      load(k, V[i]);
+      atomicMin(&best[(m[i] & 0xFFFFU) - x0], chunk_key(V[i], (m[i] >> 16) * kLabelAlign));
+    }
+  }
+  for (int k = ka + tid + kSelThreads * kSelHeld; k < kb; k += kSelThreads) {
+    std::uint32_t X[8];
+    const std::uint32_t mm = rmap[k];
+    load(k, X);
+    atomicMin(&best[(mm & 0xFFFFU) - x0], chunk_key(X, (mm >> 16) * kLabelAlign));
+  }
+  __syncthreads();
+  // Best cost of a chunk outside the winner and its neighbours (labels w - 1
+  // .. w + 1, halves a .. a + 2 of the chunk: words a / 2 and a / 2 + 1).
+  auto outside = [&](std::uint32_t mm, const std::uint32_t (&X)[8]) __attribute__((always_inline)) {
+    const int x = static_cast<int>(mm & 0xFFFFU) - x0;
+    const int a = static_cast<int>(best[x] & 0xFFFFU) - 1 - static_cast<int>(mm >> 16) * kLabelAlign, j0 = a >> 1;
+    std::uint32_t w0 = 0xFFFFFFFFU, w1 = 0xFFFFFFFFU, lowest = 0xFFFFFFFFU;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const bool e0 = j == j0, e1 = j == j0 + 1;
+      w0 = e0 ? X[j] : w0;
+      w1 = e1 ? X[j] : w1;
+      lowest = as_u32(__builtin_elementwise_min(as_pair(lowest), as_pair(e0 || e1 ? 0xFFFFFFFFU : X[j])));
+    }
+    const bool odd = (a & 1) != 0;
+    // Costs at w - 1 and w + 1 where this chunk holds them.
+    if (j0 >= 0 && j0 < 8) below[x] = static_cast<std::uint16_t>(odd ? w0 >> 16 : w0);
+    if (j0 + 1 >= 0 && j0 + 1 < 8) above[x] = static_cast<std::uint16_t>(odd ? w1 >> 16 : w1);
+    lowest = as_u32(__builtin_elementwise_min(as_pair(lowest), as_pair(w0 | (odd ? 0xFFFF0000U : 0xFFFFFFFFU))));
+    lowest = as_u32(__builtin_elementwise_min(as_pair(lowest), as_pair(w1 | (odd ? 0xFFFFFFFFU : 0x0000FFFFU))));
+    atomicMin(&second[x], min(lowest & 0xFFFFU, lowest >> 16));
+  };
+#pragma unroll
+  for (int i = 0; i < kSelHeld; ++i) {
+    if (ka + tid + kSelThreads * i < kb) outside(m[i], V[i]);
+  }
+  for (int k = ka + tid + kSelThreads * kSelHeld; k < kb; k += kSelThreads) {
+    std::uint32_t X[8];
+    load(k, X);
+    outside(rmap[k], X);
+  }
+  __syncthreads();
+
+  for (int x = x0 + tid; x < x1; x += kSelThreads) {
     float d = kInf, conf = 0.0F;
     std::int16_t lab = INT16_MIN;
     if (x >= xb && x < xe) {
-      const int X = T.x0 + x;
-      int lo, n;
-      const std::uint64_t s = pixel(x, lo, n);
-      // Labels are a multiple of 16 per pixel, so each lane's group of 8 is
-      // either wholly inside the pixel's labels or wholly past them.
-      const int k0 = 8 * q, k1 = 32 + 8 * q;
-      uint4 g0 = make_uint4(0xFFFFFFFFU, 0xFFFFFFFFU, 0xFFFFFFFFU, 0xFFFFFFFFU), g1 = g0;
-      if (k0 < n) g0 = ld8(s + k0);
-      if (k1 < n) g1 = ld8(s + k1);
-      std::uint32_t m = 0xFFFFFFFFU;
-      if (k0 < n) m = key_min(g0, k0, m);
-      if (k1 < n) m = key_min(g1, k1, m);
-      // Labels from 64 on are read once: the lane keeps its four smallest
-      // keys among them (t0 <= t1 <= t2 <= t3).  At most three labels are
-      // excluded from the second minimum (kb - 1, kb, kb + 1), so the first
-      // of these keys outside that interval holds the lane's second minimum
-      // over its labels from 64 on.
-      std::uint32_t t0 = 0xFFFFFFFFU, t1 = t0, t2 = t0, t3 = t0;
-      for (int k = 64 + 8 * q; k < n; k += 32) top4(ld8(s + k), k, t0, t1, t2, t3);
-      m = quad_min(min(m, t0));
-      const int kb = static_cast<int>(m & 0xFFFFU);
-      std::uint32_t second = 0xFFFFU;
-      if (k0 < n) second = outside_min(g0, k0, kb, second);
-      if (k1 < n) second = outside_min(g1, k1, kb, second);
-      auto outside = [&](std::uint32_t t) {
-        const int k = static_cast<int>(t & 0xFFFFU);
-        return k + 1 < kb || k > kb + 1;
-      };
-      const std::uint32_t tw = outside(t0) ? t0 : (outside(t1) ? t1 : (outside(t2) ? t2 : t3));
-      second = min(second, tw >> 16);
-      second = quad_min(second);
-      // Costs at kb - 1 and kb + 1 from the registers of the quad when they
-      // lie in the first 64 labels.
-      const std::uint32_t sm = quad_min(min(group_value(g0, k0, kb - 1), group_value(g1, k1, kb - 1)));
-      const std::uint32_t sp = quad_min(min(group_value(g0, k0, kb + 1), group_value(g1, k1, kb + 1)));
-      if (q != 0) continue;
-      const std::uint32_t bcost = m >> 16;
-      const int best = lo + kb;
-      const int j = kb;
-      const int xr = X - J.dmin - best;
+      const std::uint64_t rec = pix[px + x];
+      const int lo = pix_lo(rec), n = pix_num(rec);
+      const std::uint32_t key = best[x - x0], sec = second[x - x0], bcost = key >> 16;
+      const int j = static_cast<int>(key & 0xFFFFU), label = lo + j;
+      const int xr = T.x0 + x - J.dmin - label;
       bool ok = !(xr < rf || xr > rl);
       if (ok && ((j == 0 && lo > 0) || (j == n - 1 && lo + n < D))) ok = false;
       if (ok && p.diagonal_lr) {
-        const std::uint32_t key = keys[x - best + D - 1];
-        const int rbest = static_cast<int>(key & 0xFFFFU) - (x - best);
-        if (abs(rbest - best) > p.lr_max_diff) ok = false;
+        const std::uint32_t rkey = keys[x - label + D - 1];
+        const int rbest = static_cast<int>(rkey & 0xFFFFU) - (x - label);
+        if (abs(rbest - label) > p.lr_max_diff) ok = false;
       }
       const float best_cost = static_cast<float>(bcost);
-      if (ok && p.uniqueness > 0.0F && second != 0xFFFFU &&
-          best_cost > (1.0F - p.uniqueness) * static_cast<float>(second))
+      if (ok && p.uniqueness > 0.0F && sec != 0xFFFFU && best_cost > (1.0F - p.uniqueness) * static_cast<float>(sec))
         ok = false;
       if (ok) {
         float delta = 0.0F;
-        if (j > 0 && j < n - 1) {
-          const std::uint32_t vm = j - 1 < 64 ? sm : ld1(s + j - 1);
-          const std::uint32_t vp = j + 1 < 64 ? sp : ld1(s + j + 1);
-          delta = subpixel_offset(p.subpixel, static_cast<float>(vm), best_cost, static_cast<float>(vp));
-        }
-        d = static_cast<float>(J.dmin + best) + delta;
-        conf = second != 0xFFFFU && second > 0 ? 1.0F - best_cost / static_cast<float>(second) : 0.0F;
-        lab = static_cast<std::int16_t>(J.dmin + best);
+        if (j > 0 && j < n - 1)
+          delta = subpixel_offset(p.subpixel, static_cast<float>(below[x - x0]), best_cost,
+                                  static_cast<float>(above[x - x0]));
+        d = static_cast<float>(J.dmin + label) + delta;
+        conf = sec != 0xFFFFU && sec > 0 ? 1.0F - best_cost / static_cast<float>(sec) : 0.0F;
+        lab = static_cast<std::int16_t>(J.dmin + label);
       }
-    } else if (q != 0) {
-      continue;
     }
     tdisp[px + x] = d;
     if (J.confidence) tconf[px + x] = conf;
@@ -1914,16 +1860,18 @@ void launch_sweep(const SweepArgs& a, int np, const SweepPlan& p, std::uint64_t 
 }
 
 void launch_select(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
-                   std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix, const SumSrc& src,
-                   SelectParams p, int max_w, int max_D, float* tdisp, float* tconf, std::int16_t* tlab,
+                   std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix,
+                   const std::uint32_t* cmap, const SumSrc& src, SelectParams p, int max_w, int max_D, float* tdisp, float* tconf, std::int16_t* tlab,
                    hipStream_t s) {
   if (total_rows == 0) return;
   const std::size_t lds = p.diagonal_lr ? std::size_t(max_w + max_D) * sizeof(std::uint32_t) : 0;
-  const dim3 grid(static_cast<unsigned>(total_rows));
+  const dim3 grid(static_cast<unsigned>(total_rows), static_cast<unsigned>((max_w + kSelPx - 1) / kSelPx));
   if (src.m != nullptr) {
-    k_select<true><<<grid, 256, lds, s>>>(jobs, tiles, row_prefix, ntiles, rowbase, pix, src, p, tdisp, tconf, tlab);
+    k_select<true><<<grid, kSelThreads, lds, s>>>(jobs, tiles, row_prefix, ntiles, rowbase, pix, cmap, src, p, tdisp,
+                                                  tconf, tlab);
   } else {
-    k_select<false><<<grid, 256, lds, s>>>(jobs, tiles, row_prefix, ntiles, rowbase, pix, src, p, tdisp, tconf, tlab);
+    k_select<false><<<grid, kSelThreads, lds, s>>>(jobs, tiles, row_prefix, ntiles, rowbase, pix, cmap, src, p, tdisp,
+                                                   tconf, tlab);
   }
 }
 

@@ -521,6 +521,7 @@ struct Chunk {
   // Aggregated costs: the paths' planes and the costs C, or slices of S (the
   // sum mod 2^16 of all of them), `stride` elements apart.
   DBuf<std::uint8_t> C, planes;
+  DBuf<std::uint32_t> cmap;  // per chunk of 16 cells its column and place in the pixel
   DBuf<std::uint16_t> S, X;
   std::uint64_t stride = 0;
   int slices = 0;
@@ -849,7 +850,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     queues = view<std::uint32_t>(ch.meta, oq);
   }
   ch.C = DBuf<std::uint8_t>(c.arena, ch.cells + kSPad);
-  DBuf<std::uint32_t> cmap;
+  ch.cmap = DBuf<std::uint32_t>(c.arena, ch.cells / kLabelAlign + 1);
   // Scratch rows of the path scans' persistent waves (pixels wider than the
   // LDS rows; a multiple of 4: launches use whole blocks of 4 waves, one slot
   // each).
@@ -876,7 +877,6 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
       ch.xstride = (ch.xcells + kSPad + 127) / 128 * 128;
       ch.X = DBuf<std::uint16_t>(c.arena, std::size_t(kPaths - ch.slices) * ch.xstride);
     }
-    cmap = DBuf<std::uint32_t>(c.arena, ch.cells / kLabelAlign + 1);
     for (Sweep& s : sw)
       if (s.units > 0 && s.block_words > 0) s.scratch = DBuf<std::uint32_t>(c.arena, s.blocks * s.block_words);
   } else {
@@ -896,7 +896,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   {
     const StageTimer timer(c, R3DG_STAGE_PREPARE);
     launch_cost(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), nt, ch.rows, A.rowbase.get(), A.pix.get(),
-                ch.C.get(), cmap.get(), c.stream);
+                ch.C.get(), ch.cmap.get(), c.stream);
     check_launch();
   }
   const StageTimer timer(c, R3DG_STAGE_AGGREGATE);
@@ -942,7 +942,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     sa.units = static_cast<std::uint32_t>(s.units);
     sa.rowbase = A.rowbase.get();
     sa.pix = A.pix.get();
-    sa.cmap = cmap.get();
+    sa.cmap = ch.cmap.get();
     sa.C = ch.C.get();
     // Downwards into slice 0, upwards into slice 1; the diagonals of one-path
     // sweeps into X.
@@ -1044,7 +1044,7 @@ std::vector<TilesOut> match_jobs(Context& c, std::vector<Job>& jobs, const r3dg_
     // Selection into per-tile maps.
     const StageTimer timer(c, R3DG_STAGE_SELECT);
     launch_select(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), t1 - t0, ch.rows, A.rowbase.get(),
-                  A.pix.get(), ch.source(), sp, A.max_w, A.max_D, tdisp.get(), tconf.get(), tlab.get(), c.stream);
+                  A.pix.get(), ch.cmap.get(), ch.source(), sp, A.max_w, A.max_D, tdisp.get(), tconf.get(), tlab.get(), c.stream);
     check_launch();
   }
   std::vector<TilesOut> out(static_cast<std::size_t>(nj));
