@@ -138,10 +138,26 @@ void launch_cost(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t
 std::uint64_t path_slots();
 std::size_t path_scratch_elems(std::uint64_t slots, int max_num);
 int path_scratch_row(int max_num);
-void launch_sgm_path(int path, const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* group_prefix, int ntiles,
-                     std::uint64_t groups, const std::uint32_t* rowbase, const std::uint64_t* pix,
-                     const std::uint8_t* C, std::uint16_t* S, std::uint16_t* scratch, std::uint64_t slots, int max_num,
-                     std::uint32_t* queue, bool accumulate, hipStream_t s);
+// What a path scan does with its path costs L: kFirstSum stores them into S
+// (uint16), kAddSum adds them to S, kByteM (horizontal paths) stores the bytes
+// M = L - C, at most P2.
+enum PathMode { kFirstSum, kAddSum, kByteM };
+struct PathArgs {
+  const JobDesc* jobs;
+  const TileDesc* tiles;
+  const std::uint64_t* gprefix;  // [ntiles + 1]: scanline groups before a tile
+  int ntiles;
+  std::uint64_t groups;
+  const std::uint32_t* rowbase;
+  const std::uint64_t* pix;
+  const std::uint8_t* C;
+  void* out;
+  std::uint16_t* scratch;
+  std::uint64_t slots;
+  int max_num;
+  std::uint32_t* queue;
+};
+void launch_sgm_path(int path, const PathArgs& a, int mode, hipStream_t s);
 // The eight paths of tiles whose pixels all have their job's D labels, each
 // into its own plane of bytes M = L - C (at most P2, which must be at most
 // 255).  A wave takes 64 / lps scanlines (rows for paths 0 and 1, columns for
@@ -161,8 +177,8 @@ int full_lanes(int D);
 void launch_full(const FullArgs& a, int lps, hipStream_t s);
 // The vertical and diagonal paths (2 .. 7) of tiles of at most 1024 columns,
 // row by row: np = 3 takes the three paths downwards (upwards) of a tile at
-// once and stores their sum in slice 0 (1) of S, np = 1 stores path 2 + u in
-// slice u.  Units (2 or 6 per tile) are taken from `queue`, a zeroed counter,
+// once and stores their sum in out[0] (out[1]) as uint16, np = 1 stores path
+// 2 + u in out[u], as uint16 or (`bytes`) as M = L - C.  Units (2 or 6 per tile) are taken from `queue`, a zeroed counter,
 // in the order of `order`.
 struct SweepArgs {
   const JobDesc* jobs;
@@ -173,7 +189,7 @@ struct SweepArgs {
   const std::uint64_t* pix;
   const std::uint32_t* cmap;
   const std::uint8_t* C;
-  std::uint16_t* S[6];           // the slice of each unit of a tile
+  void* out[6];                  // volume of each unit of a tile
   std::uint32_t* scratch;        // per block 2 np swords
   std::uint32_t* queue;
   int wpad, cap, swords;         // SweepPlan
@@ -187,18 +203,22 @@ struct SweepPlan {
 };
 constexpr int kSweepRowPad = 8;  // words after an LDS row that a window may read
 SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks);
-void launch_sweep(const SweepArgs& a, int np, const SweepPlan& p, std::uint64_t blocks, hipStream_t s);
+void launch_sweep(const SweepArgs& a, int np, bool bytes, const SweepPlan& p, std::uint64_t blocks, hipStream_t s);
 // Extra elements S, C and a plane hold past their last cell.
 constexpr std::size_t kSPad = 64;
-// Aggregated costs: the paths' planes and the costs (m, c), or else n slices
-// of scans that ran side by side (S is their sum mod 2^16), all of p for the
-// tiles whose cells lie below xcells.
+// Aggregated costs of a chunk of tiles.  With planes (m not null) paths 0 and
+// 1 are the byte planes m, m + mstride of M = L - C for all cells; the others
+// are the planes mx + (path - 2) mxstride for the tiles whose cells lie below
+// xcells and the uint16 slices p[0], p[1] for the rest; c holds C.  Without,
+// S is the sum mod 2^16 of n slices, of all of p below xcells.
 struct SumSrc {
   const std::uint16_t* p[kPaths];
   int n;
   std::uint64_t xcells;
   const std::uint8_t* m;
   std::uint64_t mstride;
+  const std::uint8_t* mx;
+  std::uint64_t mxstride;
   const std::uint8_t* c;
 };
 // dst[i] = (p[0][i] + ... + p[n - 1][i]) mod 2^16 for i < cells rounded up to a

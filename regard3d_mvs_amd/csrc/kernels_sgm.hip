@@ -523,12 +523,13 @@ struct StepSegs {
 // of a scanline are loaded 8 steps at a time (lane l of the group loads step
 // 8 b + l) and unpacked into an 8-slot ring in LDS, read one step before the
 // segment prefetch that needs them.
-template <int DX, int DY, bool kAcc>
+template <int DX, int DY, int MODE>
 __global__ __launch_bounds__(64 * kWaves) void k_path(
     const JobDesc* __restrict__ jobs, const TileDesc* __restrict__ tiles, const std::uint64_t* __restrict__ gprefix,
     int ntiles, std::uint64_t groups, const std::uint32_t* __restrict__ rowbase,
-    const std::uint64_t* __restrict__ pix, const std::uint8_t* __restrict__ C, std::uint16_t* __restrict__ S,
+    const std::uint64_t* __restrict__ pix, const std::uint8_t* __restrict__ C, void* __restrict__ out_volume,
     std::uint16_t* __restrict__ scratch, int scratch_row, std::uint32_t* __restrict__ queue) {
+  constexpr bool kAcc = MODE == kAddSum, kByte = MODE == kByteM;
   __shared__ __attribute__((aligned(16))) std::uint16_t lut[kWaves][256];
   __shared__ __attribute__((aligned(16))) std::uint32_t rows[kWaves][kScanPerWave][2][kRow / 2];
   __shared__ __attribute__((aligned(16))) u32x2 ring[kWaves][8][kScanPerWave];
@@ -589,7 +590,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
   const std::uint64_t* tpix = pix + T.px_base;
   const std::uint32_t* trow = rowbase + T.row_base;
   const std::uint8_t* Ct = C + T.cell_base;
-  std::uint16_t* St = S + T.cell_base;
+  std::uint16_t* St = static_cast<std::uint16_t*>(out_volume) + T.cell_base;  // not kByte
+  std::uint8_t* Mt = static_cast<std::uint8_t*>(out_volume) + T.cell_base;    // kByte
 
   // Batch of steps [base, base + 8): lane l8 loads step base + l8 (steps past
   // the scanline repeat its last pixel; they are never active).
@@ -703,7 +705,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
       return static_cast<std::uint32_t>(min(max(j0 + delta, -(P + 1)), n + 1) - 1 + kPad) * 2U;
     };
     // New path costs of P labels from their window words W (shift sh) and costs.
-    auto recur = [&](auto Pc, const std::uint32_t* W, std::uint32_t sh, const std::uint32_t* c, std::uint32_t* L) {
+    // M: L - C.
+    auto recur = [&](auto Pc, const std::uint32_t* W, std::uint32_t sh, const std::uint32_t* c, std::uint32_t* L,
+                     std::uint32_t* M) {
       constexpr int P = decltype(Pc)::value;
       std::uint32_t Q[P / 2 + 1];
 #pragma unroll
@@ -713,12 +717,14 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
         const std::uint32_t Cx2 = __builtin_amdgcn_perm(0U, c[k >> 1], (k & 1) ? 0x0c030c02U : 0x0c010c00U);
         if (first) {
           L[k] = Cx2;
+          M[k] = 0;
         } else {
           const std::uint32_t p12 = __builtin_amdgcn_alignbyte(Q[k + 1], Q[k], 2U);
           const u16x2 nb =
               __builtin_elementwise_add_sat(__builtin_elementwise_min(as_pair(Q[k]), as_pair(Q[k + 1])), as_pair(P1x2));
           const u16x2 best = __builtin_elementwise_min(__builtin_elementwise_min(as_pair(p12), nb), as_pair(PENx2));
-          L[k] = as_u32(best - as_pair(MPx2) + as_pair(Cx2));
+          M[k] = as_u32(best - as_pair(MPx2));
+          L[k] = as_u32(as_pair(M[k]) + as_pair(Cx2));
         }
       }
     };
@@ -745,7 +751,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
     // next step does not read (the sentinels after the labels are written
     // later in the step, and reads stop inside them), and a wide pixel's row
     // is read from scratch.
-    auto emit = [&](auto Pc, auto kLow, int j0, const std::uint32_t* L, const std::uint32_t* sv) {
+    auto emit = [&](auto Pc, auto kLow, int j0, const std::uint32_t* L, const std::uint32_t* M, const std::uint32_t* sv) {
       constexpr int P = decltype(Pc)::value;
       const bool on = act && j0 < num;
       const int w0 = (kPad + j0) >> 1;
@@ -768,7 +774,13 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
       }
       if (on) {
         const std::uint32_t off = (cell + static_cast<std::uint32_t>(j0)) * 2U;
-        if constexpr (P == 4) {
+        if constexpr (kByte && P == 4) {
+          stb<std::uint32_t>(Mt, cell + static_cast<std::uint32_t>(j0), __builtin_amdgcn_perm(M[1], M[0], 0x06040200U));
+        } else if constexpr (kByte) {
+          stb<u32x2>(Mt, cell + static_cast<std::uint32_t>(j0),
+                     u32x2{__builtin_amdgcn_perm(M[1], M[0], 0x06040200U),
+                           __builtin_amdgcn_perm(M[3], M[2], 0x06040200U)});
+        } else if constexpr (P == 4) {
           stb<u32x2>(St, off, u32x2{out[0], out[1]});
         } else {
           stb<u32x4>(St, off, u32x4{out[0], out[1], out[2], out[3]});
@@ -795,17 +807,17 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
     };
     auto seg8 = [&](int s, const SegIn<8>& d) {
       const int j0 = seg_first<8>(s, l8);
-      std::uint32_t W[6], sh, L[4];
+      std::uint32_t W[6], sh, L[4], M[4];
       window(P8{}, j0, W, sh);
-      recur(P8{}, W, sh, d.c, L);
-      emit(P8{}, std::true_type{}, j0, L, d.s);
+      recur(P8{}, W, sh, d.c, L, M);
+      emit(P8{}, std::true_type{}, j0, L, M, d.s);
     };
     auto seg4 = [&](const SegIn<4>& d) {
       const int j0 = seg_first<4>(0, l8);
-      std::uint32_t W[4], sh, L[2];
+      std::uint32_t W[4], sh, L[2], M[2];
       window(P4{}, j0, W, sh);
-      recur(P4{}, W, sh, d.c, L);
-      emit(P4{}, std::true_type{}, j0, L, d.s);
+      recur(P4{}, W, sh, d.c, L, M);
+      emit(P4{}, std::true_type{}, j0, L, M, d.s);
     };
     // Segments from 2 on (pixels of more than 96 labels): costs, S and the
     // scratch window of every lane (used where prev_wide) loaded one segment
@@ -824,14 +836,14 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
       };
       auto run = [&](int s, const Ahead& x) {
         const int j0 = seg_first<8>(s, l8);
-        std::uint32_t W[6], sh, L[4];
+        std::uint32_t W[6], sh, L[4], M[4];
         lds_window(P8{}, j0, W, sh);
         const std::uint32_t gsh = wpos(8, j0, prev_num);
 #pragma unroll
         for (int k = 0; k < 6; ++k) W[k] = prev_wide ? x.G[k] : W[k];
         sh = prev_wide ? gsh : sh;
-        recur(P8{}, W, sh, x.d.c, L);
-        emit(P8{}, std::false_type{}, j0, L, x.d.s);
+        recur(P8{}, W, sh, x.d.c, L, M);
+        emit(P8{}, std::false_type{}, j0, L, M, x.d.s);
       };
       load(2, A);
       for (int s = 2; s < segmax; s += 2) {
@@ -1094,8 +1106,9 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int NP>
+template <int NP, bool kByte>
 __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
+  static_assert(NP == 1 || !kByte, "a byte holds L - C of one path");
   constexpr int H = kHeld<NP>, N = kSweepThreads;
   extern __shared__ __attribute__((aligned(16))) std::uint32_t lds[];
   // info[3][wpad] (pixel records of three rows), pmin[2][NP][wpad], lut, item, rows[NP][cap + pad].
@@ -1127,7 +1140,8 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
     const std::uint64_t* tpix = A.pix + T.px_base;
     const std::uint8_t* Ct = A.C + T.cell_base;
     const std::uint32_t* tmap = A.cmap + T.cell_base / kLabelAlign;
-    std::uint16_t* St = A.S[u] + T.cell_base;
+    std::uint16_t* St = static_cast<std::uint16_t*>(A.out[u]) + T.cell_base;  // not kByte
+    std::uint8_t* Mt = static_cast<std::uint8_t*>(A.out[u]) + T.cell_base;    // kByte
     const std::uint32_t tcells = T.cells;
     auto row_y = [&](int i) { return rev ? h - 1 - i : i; };
     // First cells of 64 rows at a time, one per lane; fcell(i) is that of row
@@ -1272,15 +1286,23 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
             const u16x2 nb = __builtin_elementwise_add_sat(
                 __builtin_elementwise_min(as_pair(Q[j]), as_pair(Q[j + 1])), as_pair(P1x2));
             const u16x2 best = __builtin_elementwise_min(__builtin_elementwise_min(as_pair(p12), nb), as_pair(PENx2));
-            L[p][j] = as_u32(best - as_pair(MPx2) + as_pair(Cx2[j]));
-            sum[j] = p == 0 ? L[p][j] : as_u32(as_pair(sum[j]) + as_pair(L[p][j]));
+            const u16x2 M = best - as_pair(MPx2);
+            L[p][j] = as_u32(M + as_pair(Cx2[j]));
+            sum[j] = kByte ? as_u32(M) : (p == 0 ? L[p][j] : as_u32(as_pair(sum[j]) + as_pair(L[p][j])));
             mm = as_u32(__builtin_elementwise_min(as_pair(mm), as_pair(L[p][j])));
           }
           atomicMin(&cmin[p * wpad + x], min(mm & 0xFFFFU, mm >> 16));
         }
-        const std::uint32_t at = (first + 16U * static_cast<std::uint32_t>(k)) * 2U;
-        stb<u32x4>(St, at, u32x4{sum[0], sum[1], sum[2], sum[3]});
-        stb<u32x4>(St, at + 16U, u32x4{sum[4], sum[5], sum[6], sum[7]});
+        const std::uint32_t at = first + 16U * static_cast<std::uint32_t>(k);
+        if constexpr (kByte) {
+          u32x4 o;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) o[j] = __builtin_amdgcn_perm(sum[2 * j + 1], sum[2 * j], 0x06040200U);
+          stb<u32x4>(Mt, at, o);
+        } else {
+          stb<u32x4>(St, 2U * at, u32x4{sum[0], sum[1], sum[2], sum[3]});
+          stb<u32x4>(St, 2U * at + 16U, u32x4{sum[4], sum[5], sum[6], sum[7]});
+        }
       };
       // A chunk's costs into a row, with the sentinels around its pixel.
       auto put = [&](auto* row, int k, std::uint32_t f, const std::uint32_t (&L)[8]) __attribute__((always_inline)) {
@@ -1441,7 +1463,8 @@ __global__ __launch_bounds__(kSelThreads) void k_select(const JobDesc* __restric
   const int xe = min(max(ll + 1 - T.x0, xb), T.w);
   const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + y];
   const std::uint64_t px = T.px_base + std::uint64_t(y) * T.w;
-  const int slices = T.cell_base < S.xcells ? kPaths : S.n;
+  const bool split = T.cell_base < S.xcells;  // a slice or plane per path
+  const int slices = split ? kPaths : S.n;
   const int D = J.D;
   const std::uint32_t* rmap = cmap + row_cell / kLabelAlign;
   // Chunks of the block's columns.
@@ -1449,44 +1472,56 @@ __global__ __launch_bounds__(kSelThreads) void k_select(const JobDesc* __restric
   const int ka = static_cast<int>(pix_off(rec0) / kLabelAlign);
   const int kb = static_cast<int>((pix_off(rec1) + pix_num(rec1)) / kLabelAlign);
 
-  // Aggregated costs of chunk k: 8 C plus the eight paths' bytes M (L = C +
-  // M), or the sum of the slices of scans that ran side by side.
+  // Aggregated costs of chunk k.  With planes a path's bytes are M = L - C:
+  // 8 C and the eight planes' sum, or 2 C, the horizontal paths' planes and
+  // the sweeps' slices; else the sum of the slices.
   auto load = [&](int k, std::uint32_t (&V)[8]) __attribute__((always_inline)) {
     const std::uint64_t cell = row_cell + 16 * std::uint64_t(k);
-    if constexpr (kBytes) {
-      u32x4 v[kPaths + 1];
-#pragma unroll
-      for (int i = 0; i < kPaths; ++i) v[i] = *reinterpret_cast<const u32x4*>(S.m + i * S.mstride + cell);
-      v[kPaths] = *reinterpret_cast<const u32x4*>(S.c + cell);
-#pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        // Even and odd labels as packed 16-bit sums (at most 16 x 255).
-        std::uint32_t even = (v[kPaths][h] & 0x00FF00FFU) << 3, odd = ((v[kPaths][h] >> 8) & 0x00FF00FFU) << 3;
-#pragma unroll
-        for (int i = 0; i < kPaths; ++i) {
-          even += v[i][h] & 0x00FF00FFU;
-          odd += (v[i][h] >> 8) & 0x00FF00FFU;
-        }
-        V[2 * h] = __builtin_amdgcn_perm(odd, even, 0x05040100U);
-        V[2 * h + 1] = __builtin_amdgcn_perm(odd, even, 0x07060302U);
-      }
-    } else {
-      const u32x4* a = reinterpret_cast<const u32x4*>(S.p[0] + cell);
-      const u32x4 lo = a[0], hi = a[1];
+    auto add_slice = [&](const std::uint16_t* q) __attribute__((always_inline)) {
+      const u32x4* b = reinterpret_cast<const u32x4*>(q + cell);
+      const u32x4 bl = b[0], bh = b[1];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        V[j] = lo[j];
-        V[j + 4] = hi[j];
+        V[j] = as_u32(as_pair(V[j]) + as_pair(bl[j]));
+        V[j + 4] = as_u32(as_pair(V[j + 4]) + as_pair(bh[j]));
       }
-      for (int i = 1; i < slices; ++i) {
-        const u32x4* b = reinterpret_cast<const u32x4*>(S.p[i] + cell);
-        const u32x4 bl = b[0], bh = b[1];
+    };
+    if constexpr (kBytes) {
+      // Sum of n planes and n C: even and odd labels as packed 16-bit sums (at
+      // most 16 x 255).
+      auto planes = [&](auto Nc) __attribute__((always_inline)) {
+        constexpr int n = decltype(Nc)::value;
+        u32x4 v[n + 1];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          V[j] = as_u32(as_pair(V[j]) + as_pair(bl[j]));
-          V[j + 4] = as_u32(as_pair(V[j + 4]) + as_pair(bh[j]));
+        for (int i = 0; i < n; ++i) {
+          const std::uint8_t* q = i < 2 ? S.m + i * S.mstride : S.mx + (i - 2) * S.mxstride;
+          v[i] = *reinterpret_cast<const u32x4*>(q + cell);
         }
+        v[n] = *reinterpret_cast<const u32x4*>(S.c + cell);
+        constexpr int kShift = n == 8 ? 3 : 1;
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          std::uint32_t even = (v[n][h] & 0x00FF00FFU) << kShift, odd = ((v[n][h] >> 8) & 0x00FF00FFU) << kShift;
+#pragma unroll
+          for (int i = 0; i < n; ++i) {
+            even += v[i][h] & 0x00FF00FFU;
+            odd += (v[i][h] >> 8) & 0x00FF00FFU;
+          }
+          V[2 * h] = __builtin_amdgcn_perm(odd, even, 0x05040100U);
+          V[2 * h + 1] = __builtin_amdgcn_perm(odd, even, 0x07060302U);
+        }
+      };
+      if (split) {
+        planes(std::integral_constant<int, kPaths>{});
+      } else {
+        planes(std::integral_constant<int, 2>{});
+        add_slice(S.p[0]);
+        add_slice(S.p[1]);
       }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) V[j] = 0;
+      for (int i = 0; i < slices; ++i) add_slice(S.p[i]);
     }
   };
 
@@ -1727,27 +1762,34 @@ std::uint64_t resident_blocks(K kernel) {
   return std::uint64_t(std::max(cus, 1)) * std::uint64_t(std::max(per_cu, 1));
 }
 
-template <int DX, int DY, bool kAcc>
+template <int DX, int DY, int MODE>
 std::uint64_t path_blocks() {
-  static const std::uint64_t n = resident_blocks(k_path<DX, DY, kAcc>);
+  static const std::uint64_t n = resident_blocks(k_path<DX, DY, MODE>);
   return n;
 }
 
-template <int DX, int DY>
-void path_launch(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* gp, int ntiles,
-                 std::uint64_t groups, const std::uint32_t* rs, const std::uint64_t* pix, const std::uint8_t* C,
-                 std::uint16_t* S, std::uint16_t* scratch, int scratch_row, std::uint32_t* queue, std::uint64_t slots,
-                 bool accumulate, hipStream_t s) {
+template <int DX, int DY, int MODE>
+void path_launch(const PathArgs& a, hipStream_t s) {
   // Persistent waves: at most `slots` (scratch rows), at most one per group.
-  const std::uint64_t waves = std::min(groups, slots);
-  if (accumulate) {
-    const std::uint64_t blocks = std::min((waves + kWaves - 1) / kWaves, path_blocks<DX, DY, true>());
-    k_path<DX, DY, true><<<dim3(static_cast<unsigned>(blocks)), 64 * kWaves, 0, s>>>(
-        jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, scratch_row, queue);
+  const std::uint64_t waves = std::min(a.groups, a.slots);
+  const std::uint64_t blocks = std::min((waves + kWaves - 1) / kWaves, path_blocks<DX, DY, MODE>());
+  k_path<DX, DY, MODE><<<dim3(static_cast<unsigned>(blocks)), 64 * kWaves, 0, s>>>(
+      a.jobs, a.tiles, a.gprefix, a.ntiles, a.groups, a.rowbase, a.pix, a.C, a.out, a.scratch, path_scratch_row(a.max_num),
+      a.queue);
+}
+
+template <int DX, int DY>
+void path_launch(const PathArgs& a, int mode, hipStream_t s) {
+  if constexpr (DY == 0) {
+    if (mode == kByteM) {
+      path_launch<DX, DY, kByteM>(a, s);
+      return;
+    }
+  }
+  if (mode == kAddSum) {
+    path_launch<DX, DY, kAddSum>(a, s);
   } else {
-    const std::uint64_t blocks = std::min((waves + kWaves - 1) / kWaves, path_blocks<DX, DY, false>());
-    k_path<DX, DY, false><<<dim3(static_cast<unsigned>(blocks)), 64 * kWaves, 0, s>>>(
-        jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, scratch_row, queue);
+    path_launch<DX, DY, kFirstSum>(a, s);
   }
 }
 
@@ -1778,11 +1820,12 @@ void launch_cost(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t
 int path_scratch_row(int max_num) { return kPad + (max_num + 15) / 16 * 16 + kPad; }
 
 std::uint64_t path_slots() {
-  std::uint64_t b = path_blocks<1, 0, true>();
-  b = std::max(b, path_blocks<1, 0, false>());
-  b = std::max(b, path_blocks<0, 1, true>());
-  b = std::max(b, path_blocks<1, 1, true>());
-  b = std::max(b, path_blocks<-1, 1, true>());
+  std::uint64_t b = path_blocks<1, 0, kAddSum>();
+  b = std::max(b, path_blocks<1, 0, kFirstSum>());
+  b = std::max(b, path_blocks<1, 0, kByteM>());
+  b = std::max(b, path_blocks<0, 1, kAddSum>());
+  b = std::max(b, path_blocks<1, 1, kAddSum>());
+  b = std::max(b, path_blocks<-1, 1, kAddSum>());
   return b * kWaves;
 }
 
@@ -1790,21 +1833,17 @@ std::size_t path_scratch_elems(std::uint64_t slots, int max_num) {
   return std::size_t(slots) * kScanPerWave * 2 * std::size_t(path_scratch_row(max_num));
 }
 
-void launch_sgm_path(int path, const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* gp, int ntiles,
-                     std::uint64_t groups, const std::uint32_t* rs, const std::uint64_t* pix, const std::uint8_t* C,
-                     std::uint16_t* S, std::uint16_t* scratch, std::uint64_t slots, int max_num,
-                     std::uint32_t* queue, bool accumulate, hipStream_t s) {
-  if (groups == 0) return;
-  const int srow = path_scratch_row(max_num);
+void launch_sgm_path(int path, const PathArgs& a, int mode, hipStream_t s) {
+  if (a.groups == 0) return;
   switch (path) {
-    case 0: path_launch<1, 0>(jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, srow, queue, slots, accumulate, s); break;
-    case 1: path_launch<-1, 0>(jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, srow, queue, slots, accumulate, s); break;
-    case 2: path_launch<0, 1>(jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, srow, queue, slots, accumulate, s); break;
-    case 3: path_launch<0, -1>(jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, srow, queue, slots, accumulate, s); break;
-    case 4: path_launch<1, 1>(jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, srow, queue, slots, accumulate, s); break;
-    case 5: path_launch<-1, -1>(jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, srow, queue, slots, accumulate, s); break;
-    case 6: path_launch<-1, 1>(jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, srow, queue, slots, accumulate, s); break;
-    default: path_launch<1, -1>(jobs, tiles, gp, ntiles, groups, rs, pix, C, S, scratch, srow, queue, slots, accumulate, s); break;
+    case 0: path_launch<1, 0>(a, mode, s); break;
+    case 1: path_launch<-1, 0>(a, mode, s); break;
+    case 2: path_launch<0, 1>(a, mode, s); break;
+    case 3: path_launch<0, -1>(a, mode, s); break;
+    case 4: path_launch<1, 1>(a, mode, s); break;
+    case 5: path_launch<-1, -1>(a, mode, s); break;
+    case 6: path_launch<-1, 1>(a, mode, s); break;
+    default: path_launch<1, -1>(a, mode, s); break;
   }
 }
 
@@ -1846,16 +1885,26 @@ SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks) {
   return p;
 }
 
-void launch_sweep(const SweepArgs& a, int np, const SweepPlan& p, std::uint64_t blocks, hipStream_t s) {
-  if (a.units == 0) return;
+namespace {
+template <int NP, bool kByte>
+void sweep_launch(const SweepArgs& a, const SweepPlan& p, std::uint64_t blocks, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(std::min<std::uint64_t>(a.units, blocks)));
-  // Dynamic LDS past 64 KB has to be asked for once per kernel and device.
-  const auto* fn = np == 3 ? reinterpret_cast<const void*>(&k_sweep<3>) : reinterpret_cast<const void*>(&k_sweep<1>);
-  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, p.lds_bytes) != hipSuccess) return;
+  // Dynamic LDS past 64 KB has to be asked for (a failure is the launch's).
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep<NP, kByte>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, p.lds_bytes) != hipSuccess)
+    return;
+  k_sweep<NP, kByte><<<grid, kSweepThreads, p.lds_bytes, s>>>(a);
+}
+}  // namespace
+
+void launch_sweep(const SweepArgs& a, int np, bool bytes, const SweepPlan& p, std::uint64_t blocks, hipStream_t s) {
+  if (a.units == 0) return;
   if (np == 3) {
-    k_sweep<3><<<grid, kSweepThreads, p.lds_bytes, s>>>(a);
+    sweep_launch<3, false>(a, p, blocks, s);
+  } else if (bytes) {
+    sweep_launch<1, true>(a, p, blocks, s);
   } else {
-    k_sweep<1><<<grid, kSweepThreads, p.lds_bytes, s>>>(a);
+    sweep_launch<1, false>(a, p, blocks, s);
   }
 }
 

@@ -518,27 +518,26 @@ struct Chunk {
   DView<TileDesc> dtiles;
   DView<std::uint64_t> drow_prefix;
   std::uint64_t rows = 0, cells = 0, px = 0;
-  // Aggregated costs: the paths' planes and the costs C, or slices of S (the
-  // sum mod 2^16 of all of them), `stride` elements apart.
-  DBuf<std::uint8_t> C, planes;
+  // Aggregated costs (SumSrc): `planes` byte planes of M, `stride` apart, and
+  // slices of S, `stride` elements apart.  Tiles aggregated path by path hold
+  // the chunk's first xcells cells; their other paths have planes or slices
+  // of their own, xstride apart, in MX or X.
+  DBuf<std::uint8_t> C, M, MX;
   DBuf<std::uint32_t> cmap;  // per chunk of 16 cells its column and place in the pixel
   DBuf<std::uint16_t> S, X;
-  std::uint64_t stride = 0;
-  int slices = 0;
-  // Tiles swept path by path hold the chunk's first xcells cells; their
-  // further paths have slices of their own, xstride elements apart in X.
-  std::uint64_t xcells = 0, xstride = 0;
+  std::uint64_t stride = 0, xcells = 0, xstride = 0;
+  int planes = 0, slices = 0;
   SumSrc source() const {
     SumSrc v{};
-    if (planes.get() != nullptr) {
-      v.m = planes.get();
-      v.mstride = stride;
-      v.c = C.get();
-      return v;
-    }
     for (v.n = 0; v.n < slices; ++v.n) v.p[v.n] = S.get() + std::uint64_t(v.n) * stride;
-    if (xcells > 0) {
-      v.xcells = xcells;
+    v.xcells = xcells;
+    if (planes > 0) {
+      v.m = M.get();
+      v.mstride = stride;
+      v.mx = planes == kPaths ? M.get() + 2 * stride : MX.get();
+      v.mxstride = planes == kPaths ? stride : xstride;
+      v.c = C.get();
+    } else if (xcells > 0) {
       for (int k = slices; k < kPaths; ++k) v.p[k] = X.get() + std::uint64_t(k - slices) * xstride;
     }
     return v;
@@ -794,7 +793,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     while (heavy < nt && (nt < kSweepTiles || mean_words(order[std::size_t(heavy)]) > std::uint64_t(sw[1].plan.cap))) ++heavy;
     std::uint64_t hcells = 0;
     for (int k = 0; k < heavy; ++k) hcells += A.tcells[std::size_t(t0 + order[std::size_t(k)])];
-    if (8 * ch.cells + 8 * hcells > free_bytes() / 2) heavy = 0;
+    if (10 * ch.cells + 8 * hcells > free_bytes() / 2) heavy = 0;
     sw[0].units = std::uint64_t(heavy) * 6;
     sw[1].units = std::uint64_t(nt - heavy) * 2;
     for (int i = 0; i < 2; ++i) {
@@ -806,6 +805,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     }
   }
   const bool sweep = kind == Aggregate::kSweep, full = kind == Aggregate::kFull;
+  const bool bytes = sweep && A.p2max <= kMaxByteP2;  // a path's M = L - C fits a byte
   // Path scans: all eight, or the horizontal two beside the sweeps.
   const int npaths = full ? 0 : (sweep ? 2 : kPaths);
   // Group prefixes of the path scans (kScanPerWave scanlines per wave), of the
@@ -863,19 +863,31 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   // launch on another stream.  Not 4: a process gets 4 hardware queues and 4
   // such streams were traced on 3 of them, so that one queue ran 4 launches in
   // turn (measured: the 1080p pair's aggregation 5.0 ms with 4 streams, 4.7 ms
-  // with 3).  Beside the sweeps the two horizontal scans take one stream and
-  // one slice, or a stream and a slice each where the tiles are few.
+  // with 3).  Beside the sweeps the two horizontal scans take a stream each,
+  // one between them beside two sweep launches.
   int ways = 0;
   if (full) {
-    ch.planes = DBuf<std::uint8_t>(c.arena, kPaths * ch.stride);
+    ch.planes = kPaths;
+    ch.M = DBuf<std::uint8_t>(c.arena, kPaths * ch.stride);
+    ch.xcells = ch.cells;
   } else if (sweep) {
-    ways = heavy == nt ? 2 : 1;
-    ch.slices = 2 + ways;
-    ch.S = DBuf<std::uint16_t>(c.arena, std::size_t(ch.slices) * ch.stride);
+    ways = heavy == 0 || heavy == nt ? 2 : 1;
     if (heavy > 0) {
       ch.xcells = heavy < nt ? td[std::size_t(order[std::size_t(heavy)])].cell_base : ch.cells;
       ch.xstride = (ch.xcells + kSPad + 127) / 128 * 128;
-      ch.X = DBuf<std::uint16_t>(c.arena, std::size_t(kPaths - ch.slices) * ch.xstride);
+    }
+    if (bytes) {
+      ch.planes = 2;
+      ch.M = DBuf<std::uint8_t>(c.arena, 2 * ch.stride);
+      if (heavy > 0) ch.MX = DBuf<std::uint8_t>(c.arena, std::size_t(kPaths - 2) * ch.xstride);
+      if (heavy < nt) {
+        ch.slices = 2;
+        ch.S = DBuf<std::uint16_t>(c.arena, 2 * ch.stride);
+      }
+    } else {
+      ch.slices = 4;
+      ch.S = DBuf<std::uint16_t>(c.arena, 4 * ch.stride);
+      if (heavy > 0) ch.X = DBuf<std::uint16_t>(c.arena, std::size_t(kPaths - 4) * ch.xstride);
     }
     for (Sweep& s : sw)
       if (s.units > 0 && s.block_words > 0) s.scratch = DBuf<std::uint32_t>(c.arena, s.blocks * s.block_words);
@@ -908,7 +920,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     fa.ntiles = nt;
     fa.groups = fp.back();
     fa.C = ch.C.get();
-    fa.M = ch.planes.get();
+    fa.M = ch.M.get();
     fa.mstride = ch.stride;
     launch_full(fa, lps, c.stream);
     check_launch();
@@ -944,28 +956,53 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     sa.pix = A.pix.get();
     sa.cmap = ch.cmap.get();
     sa.C = ch.C.get();
-    // Downwards into slice 0, upwards into slice 1; the diagonals of one-path
-    // sweeps into X.
-    for (int u = 0; u < 6; ++u)
-      sa.S[u] = u < 2 ? ch.S.get() + std::uint64_t(u) * ch.stride
-                      : ch.X.get() + std::uint64_t(u - 2) * ch.xstride;
+    // Three paths at once: downwards into slice 0, upwards into slice 1.  One
+    // path: a plane each, or the slices 0 and 1 and (diagonals) those of X.
+    for (int u = 0; u < 6; ++u) {
+      if (i == 0 && bytes) {
+        sa.out[u] = ch.MX.get() + std::uint64_t(u) * ch.xstride;
+      } else {
+        sa.out[u] = u < 2 ? ch.S.get() + std::uint64_t(u) * ch.stride
+                          : ch.X.get() + std::uint64_t(u - 2) * ch.xstride;
+      }
+    }
     sa.scratch = s.scratch.get();
     sa.queue = queues.get() + kPaths + i;
     sa.wpad = s.plan.wpad;
     sa.cap = s.plan.cap;
     sa.swords = s.plan.swords;
-    launch_sweep(sa, i == 0 ? 1 : 3, s.plan, s.blocks, st[std::size_t(both && i == 1 ? side : 0)]);
+    launch_sweep(sa, i == 0 ? 1 : 3, bytes, s.plan, s.blocks, st[std::size_t(both && i == 1 ? side : 0)]);
     check_launch();
     c.agg_launches += 1;
   }
-  const int slice0 = sweep ? ch.slices - ways : 0;
+  PathArgs pa{};
+  pa.jobs = A.djobs.get();
+  pa.tiles = ch.dtiles.get();
+  pa.ntiles = nt;
+  pa.rowbase = A.rowbase.get();
+  pa.pix = A.pix.get();
+  pa.C = ch.C.get();
+  pa.slots = slots;
+  pa.max_num = max_num;
   for (int p = 0; p < npaths; ++p) {
     const int w = p % ways;
     const std::size_t o8 = std::size_t(p) * (std::size_t(nt) + 1);
-    launch_sgm_path(p, A.djobs.get(), ch.dtiles.get(), dgp.get() + o8, nt, gp[o8 + std::size_t(nt)], A.rowbase.get(),
-                    A.pix.get(), ch.C.get(), ch.S.get() + std::uint64_t(slice0 + w) * ch.stride,
-                    scratch.get() + std::size_t(w) * scratch_elems, slots, max_num, queues.get() + p, p >= ways,
-                    st[std::size_t(sweep ? w + 1 : w)]);
+    pa.gprefix = dgp.get() + o8;
+    pa.groups = gp[o8 + std::size_t(nt)];
+    pa.scratch = scratch.get() + std::size_t(w) * scratch_elems;
+    pa.queue = queues.get() + p;
+    int mode = kFirstSum;
+    if (bytes) {
+      mode = kByteM;
+      pa.out = ch.M.get() + std::uint64_t(p) * ch.stride;
+    } else if (sweep) {
+      pa.out = ch.S.get() + std::uint64_t(2 + p) * ch.stride;
+    } else {
+      // Path p adds into its stream's slice.
+      mode = p >= ways ? kAddSum : kFirstSum;
+      pa.out = ch.S.get() + std::uint64_t(w) * ch.stride;
+    }
+    launch_sgm_path(p, pa, mode, st[std::size_t(sweep ? w + 1 : w)]);
     check_launch();
   }
   for (int w = 1; w <= side; ++w) {
@@ -984,9 +1021,9 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   // each slice only writes it) and the sweeps' map; per tile pixel and pass
   // over it its record.
   if (sweep) {
-    const std::uint64_t scans = (2 + 2 + (ways == 1 ? 2 + 2 + 2 : 2 + 2)) * ch.cells + 16 * ch.px;
-    c.agg_bytes += scans + (2 + 4) * ch.cells + ch.cells / 2 + 16 * ch.px +
-                   (ch.xcells > 0 ? (4 + 8 + 1) * ch.xcells : 0);
+    const std::uint64_t out = bytes ? 1 : 2, light = ch.cells - ch.xcells;
+    c.agg_bytes += 2 * (1 + out) * ch.cells + light * (2 + 4) + light / 2 + ch.xcells * (6 + 6 * out) + 3 * ch.xcells / 2 +
+                   48 * ch.px;
   } else {
     c.agg_bytes += std::uint64_t(40 - 2 * ways) * ch.cells + 64 * ch.px;
   }
