@@ -55,6 +55,7 @@ void launch_rectify_f32(const float* src, std::int64_t ss, const RectifyGeom& g,
                         std::uint8_t* valid, std::int64_t vs, hipStream_t s);
 // combine_pairs (mvs/multi_stereo.cpp:74-216): one pair of a view (device
 // pointers) and the grid with the options.
+constexpr double kMaxDivisor = 1e100;  // of quotients that share a reciprocal
 struct CombinePair {
   double g[9];       // grid pixel -> rectified pixel, row-major
   double fb, offset;
@@ -64,6 +65,8 @@ struct CombinePair {
   const float* conf;  // may be null
   std::int64_t cs;
   int dw, dh, cw, ch;
+  double umax, vmax;  // dw - 0.5, dh - 0.5
+  int shared;         // the grid's divisors and fb stay where quotients may share a reciprocal
 };
 struct CombineGrid {
   double inv_k[9], rot_t[9], center[3];

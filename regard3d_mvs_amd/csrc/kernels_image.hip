@@ -486,6 +486,26 @@ __global__ void k_median3x3(const float* __restrict__ in, int w, int h, float* _
   out[std::int64_t(y) * w + x] = m;
 }
 
+// ------------------------------------------------------------------ shared divisors
+// Several quotients by one divisor c, each the correctly rounded one that /
+// gives: the reciprocal y is refined once (Newton), every quotient then takes a
+// product and Markstein's correction q + y (a - c q) with an exact remainder,
+// 3 instructions in place of 11.  For c between 1e-10 and kMaxDivisor and |a|
+// from 1e-290 to 1e200, or 0, no step leaves the normal range.  A smaller |a|
+// gives a quotient below 1e-280 all the same, a larger one a quotient above
+// 1e100 or a NaN.
+struct Divisor {
+  double c, y;
+  __device__ __forceinline__ explicit Divisor(double d) : c(d), y(__builtin_amdgcn_rcp(d)) {
+    y = __builtin_fma(y, __builtin_fma(-c, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-c, y, 1.0), y);
+  }
+  __device__ __forceinline__ double under(double a) const {
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-c, q, a), y, q);
+  }
+};
+
 // ------------------------------------------------------------------ rectification
 // rectify_image (rectify/rectification.cpp:288-350), one thread per target
 // pixel: the ray (x - cx) / fx, (y - cy) / fy, 1 of the target camera turned
@@ -603,122 +623,178 @@ __global__ __launch_bounds__(256) void k_rectify(const T* __restrict__ src, std:
 }
 
 // ------------------------------------------------------------------ combining pairs
-// sample_disparity (multi_stereo.cpp:44-72): bilinear when the four
-// neighbours are finite and within one pixel of each other, else the nearest
-// pixel; +inf outside.
-__device__ float sample_disparity(const float* __restrict__ d, std::int64_t s, int w, int h, double u, double v) {
-  if (!(u > -0.5 && v > -0.5 && u < w - 0.5 && v < h - 0.5)) return kInf;
-  const int x0 = min(max(static_cast<int>(floor(u)), 0), w - 1);
-  const int y0 = min(max(static_cast<int>(floor(v)), 0), h - 1);
-  const int x1 = min(x0 + 1, w - 1), y1 = min(y0 + 1, h - 1);
-  const float d00 = d[y0 * s + x0], d10 = d[y0 * s + x1], d01 = d[y1 * s + x0], d11 = d[y1 * s + x1];
-  if (finite(d00) && finite(d10) && finite(d01) && finite(d11)) {
-    const float lo = smin(smin(smin(d00, d10), d01), d11);
-    const float hi = smax(smax(smax(d00, d10), d01), d11);
-    if (hi - lo <= 1.0F) {
-      const double ex = u - x0, ey = v - y0;
-      const float fx = static_cast<float>(ex < 0.0 ? 0.0 : (1.0 < ex ? 1.0 : ex));
-      const float fy = static_cast<float>(ey < 0.0 ? 0.0 : (1.0 < ey ? 1.0 : ey));
-      const float top = d00 + fx * (d10 - d00);
-      const float bottom = d01 + fx * (d11 - d01);
-      return top + fy * (bottom - top);
-    }
-  }
-  const int xn = min(max(static_cast<int>(lround(u)), 0), w - 1);
-  const int yn = min(max(static_cast<int>(lround(v)), 0), h - 1);
-  return d[yn * s + xn];
-}
-
 // Unit vector a / |a| (Eigen's normalized(): unchanged when |a| = 0).
 __device__ __forceinline__ void unit3(double* a) {
   const double n2 = a[0] * a[0] + a[1] * a[1] + a[2] * a[2];
   if (n2 > 0.0) {
     const double n = sqrt(n2);
-    a[0] = a[0] / n;
-    a[1] = a[1] / n;
-    a[2] = a[2] / n;
+    if (n > 1e-10 && n < kMaxDivisor) {
+      const Divisor by(n);
+      for (int i = 0; i < 3; ++i) a[i] = by.under(a[i]);
+    } else {
+      for (int i = 0; i < 3; ++i) a[i] = a[i] / n;
+    }
   }
+}
+
+using gfloat = __attribute__((address_space(1))) float;
+
+// a[q] of a list in registers.
+template <int N, typename V>
+__device__ __forceinline__ V pick(const V (&a)[N], int q) {
+  V r = a[0];
+#pragma unroll
+  for (int i = 1; i < N; ++i) {
+    V v = a[i];
+    asm("" : "+v"(v));  // keeps the choice one of values: one of addresses would put the list into memory
+    r = q == i ? v : r;
+  }
+  return r;
 }
 
 // combine_pairs per grid pixel (multi_stereo.cpp:103-213), double precision
 // in the reference's order of operations.
+//
+// Bound by vector instructions (about 1100 a wave for 4 pairs, most of them in
+// double precision): 4 pairs of 27 Mpx take 0.93 ms.  Every list of pairs is
+// indexed by the pair and unrolled to N, so that it lives in registers; lists
+// filled and indexed at run time went to scratch memory, and the kernel took
+// 2.1 ms.  Sums depend on the order of the pairs: it is ascending until a pair
+// is dropped, and from then on kept as 4-bit indexes in one word.
+template <int N>
 __global__ __launch_bounds__(256) void k_combine(const CombinePair* __restrict__ pairs, CombineGrid g,
                                                  float* __restrict__ depth, std::int64_t ds,
                                                  float* __restrict__ conf_out, std::int64_t cs,
                                                  std::uint16_t* __restrict__ mask_out, std::int64_t ms) {
   const int x = blockIdx.x * blockDim.x + threadIdx.x, yy = blockIdx.y;
   if (x >= g.w) return;
-  double cw[kMaxCombinePairs], ck[kMaxCombinePairs];
-  float cc[kMaxCombinePairs];
-  int cp[kMaxCombinePairs], used[kMaxCombinePairs];
-  int n = 0;
-  for (int i = 0; i < g.npairs; ++i) {
+  double cw[N], ck[N];
+  float cc[N];
+  unsigned seen = 0;  // pairs with a hypothesis here
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    cw[i] = ck[i] = 0.0;
+    cc[i] = 0.0F;
+    if (i >= g.npairs) continue;
     const CombinePair& P = pairs[i];
     const double rx = P.g[0] * x + P.g[1] * yy + P.g[2] * 1.0;
     const double ry = P.g[3] * x + P.g[4] * yy + P.g[5] * 1.0;
     const double c = P.g[6] * x + P.g[7] * yy + P.g[8] * 1.0;
-    if (!(c > 1e-9)) continue;
-    const double u = rx / c, v = ry / c;
-    const float d = sample_disparity(P.disp, P.ds, P.dw, P.dh, u, v);
-    if (!finite(d) || d <= P.offset) continue;
-    ck[n] = P.fb / c;
-    cw[n] = (d - P.offset) / ck[n];
-    cp[n] = i;
-    float cf = 0.0F;
-    if (P.conf != nullptr) {
-      const int xn = min(max(static_cast<int>(lround(u)), 0), P.cw - 1);
-      const int yn = min(max(static_cast<int>(lround(v)), 0), P.ch - 1);
-      cf = P.conf[yn * P.cs + xn];
+    double u, v;
+    if (P.shared != 0) {
+      const Divisor by(c);
+      u = by.under(rx);
+      v = by.under(ry);
+      ck[i] = by.under(P.fb);
+    } else {
+      u = rx / c;
+      v = ry / c;
+      ck[i] = P.fb / c;
     }
-    cc[n] = cf;
-    ++n;
+    const bool inside = (c > 1e-9) & (u > -0.5) & (v > -0.5) & (u < P.umax) & (v < P.vmax);
+    // Outside, pixel (0, 0) is read and not used: no branch around the loads,
+    // so those of all pairs are in flight together.
+    u = inside ? u : 0.0;
+    v = inside ? v : 0.0;
+    // sample_disparity (multi_stereo.cpp:44-72): bilinear when the four
+    // neighbours are finite and within one pixel of each other, else the
+    // nearest pixel (halves away from zero), which is one of the four.
+    const double uf = floor(u), vf = floor(v), ue = u - uf, ve = v - vf;
+    const int ui = static_cast<int>(uf), vi = static_cast<int>(vf);  // from -1 to the last column or row
+    const int xn = ui + (ue >= 0.5 ? 1 : 0), yn = vi + (ve >= 0.5 ? 1 : 0);  // the nearest pixel, inside the map
+    const int x0 = max(ui, 0), y0 = max(vi, 0);
+    const int dx = x0 + 1 < P.dw ? 1 : 0;
+    const std::int64_t dy = y0 + 1 < P.dh ? P.ds : 0;
+    const gfloat* at = (const gfloat*)P.disp + (y0 * P.ds + x0);
+    const float d00 = at[0], d10 = at[dx], d01 = at[dy], d11 = at[dy + dx];
+    if (P.conf != nullptr)
+      cc[i] = ((const gfloat*)P.conf)[min(yn, P.ch - 1) * P.cs + min(xn, P.cw - 1)];
+    const float fx = ui < 0 ? 0.0F : static_cast<float>(ue), fy = vi < 0 ? 0.0F : static_cast<float>(ve);
+    const float top = d00 + fx * (d10 - d00), bottom = d01 + fx * (d11 - d01);
+    const float lo = smin(smin(smin(d00, d10), d01), d11), hi = smax(smax(smax(d00, d10), d01), d11);
+    const bool smooth = finite(d00) & finite(d10) & finite(d01) & finite(d11) & (hi - lo <= 1.0F);
+    const float left = yn > y0 ? d01 : d00, right = yn > y0 ? d11 : d10;
+    const float d = smooth ? top + fy * (bottom - top) : (xn > x0 ? right : left);
+    seen |= inside & finite(d) & !(d <= P.offset) ? 1U << i : 0U;
+    cw[i] = (d - P.offset) / ck[i];
   }
+  const int n = __builtin_popcount(seen);
   float dep = 0.0F, cnf = 0.0F;
   std::uint16_t mask = 0;
   if (n >= g.min_pairs) {
     // The hypothesis with the most agreeing pairs (ties: higher summed confidence).
-    int best = -1, best_support = 0;
+    unsigned used = 0;
+    int best_support = 0;
     float best_conf = -1.0F;
-    for (int i = 0; i < n; ++i) {
-      int support = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      if (i >= g.npairs) continue;
+      unsigned agree = 0;
       float sc = 0.0F;
-      for (int j = 0; j < n; ++j) {
-        if (fabs(ck[j] * (cw[j] - cw[i])) <= g.inlier) {
-          ++support;
-          sc += cc[j];
-        }
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const bool ok = ((seen >> j & 1U) != 0) & (fabs(ck[j] * (cw[j] - cw[i])) <= g.inlier);
+        agree |= ok ? 1U << j : 0U;
+        sc = ok ? sc + cc[j] : sc;
       }
-      if (support > best_support || (support == best_support && sc > best_conf)) {
-        best = i;
-        best_support = support;
-        best_conf = sc;
-      }
+      const int support = __builtin_popcount(agree);
+      const bool better = ((seen >> i & 1U) != 0) &
+                          ((support > best_support) | ((support == best_support) & (sc > best_conf)));
+      used = better ? agree : used;
+      best_support = better ? support : best_support;
+      best_conf = better ? sc : best_conf;
     }
-    int m = 0;
-    for (int j = 0; j < n; ++j)
-      if (fabs(ck[j] * (cw[j] - cw[best])) <= g.inlier) used[m++] = j;
     // Weighted least squares on w, dropping the worst pair while a residual is too large.
+    int m = best_support;
     double w_opt = 0.0;
-    while (m > 0) {
+    float sc = 0.0F;
+    if (m > 0) {
       double sw = 0.0, swx = 0.0;
-      for (int t = 0; t < m; ++t) {
-        const int q = used[t];
-        sw += ck[q] * ck[q];
-        swx += ck[q] * ck[q] * cw[q];
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const bool in = (used >> i & 1U) != 0;
+        const double k2 = ck[i] * ck[i];
+        sw = in ? sw + k2 : sw;
+        swx = in ? swx + k2 * cw[i] : swx;
+        sc = in ? sc + cc[i] : sc;
       }
       w_opt = swx / sw;
-      int worst = -1;
-      double worst_res = g.max_res;
-      for (int t = 0; t < m; ++t) {
-        const int q = used[t];
-        const double res = fabs(ck[q] * (cw[q] - w_opt));
-        if (res > worst_res) {
-          worst_res = res;
-          worst = t;
+      bool drop = false;
+#pragma unroll
+      for (int i = 0; i < N; ++i) drop |= ((used >> i & 1U) != 0) & (fabs(ck[i] * (cw[i] - w_opt)) > g.max_res);
+      if (drop) {
+        // used as a list of indexes; the dropped place takes the last one.
+        std::uint64_t order = 0;
+        for (int i = 0, t = 0; i < N; ++i)
+          if ((used >> i & 1U) != 0) order |= std::uint64_t(i) << (4 * t++);
+        for (;;) {
+          int worst = -1;
+          double worst_res = g.max_res;
+          for (int t = 0; t < m; ++t) {
+            const int q = static_cast<int>(order >> (4 * t) & 15U);
+            const double res = fabs(pick<N>(ck, q) * (pick<N>(cw, q) - w_opt));
+            if (res > worst_res) {
+              worst_res = res;
+              worst = t;
+            }
+          }
+          if (worst < 0 || --m == 0) break;
+          const std::uint64_t last = order >> (4 * m) & 15U;
+          order = (order & ~(std::uint64_t{15} << (4 * worst))) | last << (4 * worst);
+          sw = swx = 0.0;
+          sc = 0.0F;
+          used = 0;
+          for (int t = 0; t < m; ++t) {
+            const int q = static_cast<int>(order >> (4 * t) & 15U);
+            const double k = pick<N>(ck, q);
+            sw += k * k;
+            swx += k * k * pick<N>(cw, q);
+            sc += pick<N>(cc, q);
+            used |= 1U << q;
+          }
+          w_opt = swx / sw;
         }
       }
-      if (worst < 0) break;
-      used[worst] = used[--m];
     }
     const bool majority = m > n - m || (m >= 2 && m >= n - m);
     if (m >= g.min_pairs && majority && w_opt > 0.0) {
@@ -732,22 +808,20 @@ __global__ __launch_bounds__(256) void k_combine(const CombinePair* __restrict__
         tb[i] = g.center[i] - xw[i];
       }
       unit3(tb);
+      // One used pair at a wide enough angle settles it: the rest is skipped.
       bool wide = false;
-      float sc = 0.0F;
-      for (int k = 0; k < m; ++k) {
-        const int q = used[k];
-        mask = static_cast<std::uint16_t>(mask | (1U << cp[q]));
-        const CombinePair& P = pairs[cp[q]];
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        if (i >= g.npairs || wide || (used >> i & 1U) == 0) continue;
+        const CombinePair& P = pairs[i];
         double tp[3] = {P.pc[0] - xw[0], P.pc[1] - xw[1], P.pc[2] - xw[2]};
         unit3(tp);
-        wide = wide || tb[0] * tp[0] + tb[1] * tp[1] + tb[2] * tp[2] <= g.cos_min;
-        sc += cc[q];
+        wide = tb[0] * tp[0] + tb[1] * tp[1] + tb[2] * tp[2] <= g.cos_min;
       }
       if (wide) {
         dep = static_cast<float>(z);
         cnf = sc / static_cast<float>(m);
-      } else {
-        mask = 0;
+        mask = static_cast<std::uint16_t>(used);
       }
     }
   }
@@ -993,7 +1067,17 @@ void launch_rectify_f32(const float* src, std::int64_t ss, const RectifyGeom& g,
 void launch_combine(const CombinePair* pairs, const CombineGrid& g, float* depth, std::int64_t ds, float* conf,
                     std::int64_t cs, std::uint16_t* mask, std::int64_t ms, hipStream_t s) {
   if (g.w <= 0 || g.h <= 0) return;
-  k_combine<<<dim3((g.w + 255) / 256, g.h), 256, 0, s>>>(pairs, g, depth, ds, conf, cs, mask, ms);
+  // The least N that holds the pairs: registers and unrolled work grow with it.
+  static_assert(kMaxCombinePairs <= 16, "the order of the pairs is 4-bit indexes in a 64-bit word");
+  const dim3 grid((g.w + 255) / 256, g.h);
+  if (g.npairs <= 2)
+    k_combine<2><<<grid, 256, 0, s>>>(pairs, g, depth, ds, conf, cs, mask, ms);
+  else if (g.npairs <= 4)
+    k_combine<4><<<grid, 256, 0, s>>>(pairs, g, depth, ds, conf, cs, mask, ms);
+  else if (g.npairs <= 8)
+    k_combine<8><<<grid, 256, 0, s>>>(pairs, g, depth, ds, conf, cs, mask, ms);
+  else
+    k_combine<kMaxCombinePairs><<<grid, 256, 0, s>>>(pairs, g, depth, ds, conf, cs, mask, ms);
 }
 
 

@@ -2834,6 +2834,10 @@ int32_t r3dg_combine_pairs(r3dg_ctx* h, const r3dg_grid* grid, const r3dg_pair_g
       P.ds = d.s;
       P.dw = d.w;
       P.dh = d.h;
+      P.umax = d.w - 0.5;
+      P.vmax = d.h - 0.5;
+      const double fb = std::abs(P.fb), by = std::abs(P.g[6]) * w + std::abs(P.g[7]) * hh + std::abs(P.g[8]);
+      P.shared = fb > 1.0 / kMaxDivisor && fb < kMaxDivisor && by < kMaxDivisor ? 1 : 0;
       if (!view_empty(q.confidence)) {
         maps.push_back(input_img<float>(c, q.confidence, "combine confidence"));
         const DImg<float>& cf = maps.back();
