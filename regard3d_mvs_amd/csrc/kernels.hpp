@@ -37,6 +37,7 @@ void launch_pyramid_f32(const float* in, std::int64_t is, int w, int h, float* t
 // Geometry of one rectify_image call (rectification.cpp:288-350): the target
 // pinhole intrinsics, the target-to-source rotation m (row-major) and the
 // source camera at the sampled pyramid level.
+constexpr double kMaxDivisor = 1e100;  // of quotients that share a reciprocal
 struct RectifyGeom {
   double m[9];
   double tfx, tfy, tcx, tcy;
@@ -45,6 +46,7 @@ struct RectifyGeom {
   int tw, th;
   int sw, sh;
   int model;
+  int shared;  // the divisors stay where quotients may share a reciprocal
 };
 // out (tw x th) and valid (may be null) from the source level image src.
 void launch_rectify_u8(const std::uint8_t* src, std::int64_t ss, const RectifyGeom& g, std::uint8_t* out,
@@ -55,7 +57,6 @@ void launch_rectify_f32(const float* src, std::int64_t ss, const RectifyGeom& g,
                         std::uint8_t* valid, std::int64_t vs, hipStream_t s);
 // combine_pairs (mvs/multi_stereo.cpp:74-216): one pair of a view (device
 // pointers) and the grid with the options.
-constexpr double kMaxDivisor = 1e100;  // of quotients that share a reciprocal
 struct CombinePair {
   double g[9];       // grid pixel -> rectified pixel, row-major
   double fb, offset;

@@ -2203,6 +2203,11 @@ void rectify(Context& c, const r3dg_image& src, const r3dg_camera& cam, const r3
   const double* Q = tgt.rotation;
   for (int i = 0; i < 3; ++i)
     for (int j = 0; j < 3; ++j) g.m[3 * i + j] = R[3 * i] * Q[3 * j] + R[3 * i + 1] * Q[3 * j + 1] + R[3 * i + 2] * Q[3 * j + 2];
+  // No quotient of a ray leaves the range of a shared reciprocal.
+  const double far = 1e40;
+  bool bounded = g.tfx > 1e-9 && g.tfx < far && g.tfy > 1e-9 && g.tfy < far && std::abs(g.tcx) < far && std::abs(g.tcy) < far;
+  for (const double v : g.m) bounded = bounded && std::abs(v) < far;
+  g.shared = bounded ? 1 : 0;
   // Device outputs of the target's size are written in place; host ones go
   // through a device image and the staged download.
   auto direct = [&](const r3dg_image& im) {
