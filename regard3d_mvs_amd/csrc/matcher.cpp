@@ -105,19 +105,32 @@ DImg<T> view_of(const DImg<T>& o) {
   return d;
 }
 
-// A caller image on the device: device views are used in place, host images
-// are uploaded.  Empty views stay empty.
-// Host memory the library's runtime page-locked (r3dg_host_alloc): copied by
-// DMA directly, without a staging copy.
-bool host_pinned(const void* p) {
+// Ordinary host memory goes through page-locked blocks of the context's pool
+// at any size: from pageable rows the runtime copies row by row, about 15 us
+// each way (a 384 x 288 pair with host images and maps took 10 ms of which
+// 0.9 were the matching, and takes 1.0).  Memory that r3dg_host_alloc page-locked is
+// copied by DMA directly, where that saves more than a query costs.
+bool pageable(const void* p) {
   hipPointerAttribute_t a{};
   if (hipPointerGetAttributes(&a, p) != hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return true;
   }
-  return a.type == hipMemoryTypeHost;
+  return a.type == hipMemoryTypeUnregistered;
 }
 
+// Rows between two buffers: one plain copy where both are contiguous.
+void copy_async(void* dst, std::size_t dst_stride, const void* src, std::size_t src_stride, std::size_t row_bytes,
+                std::size_t rows, hipMemcpyKind kind, hipStream_t s, const char* what) {
+  if (dst_stride == row_bytes && src_stride == row_bytes) {
+    hip_check(hipMemcpyAsync(dst, src, row_bytes * rows, kind, s), what);
+  } else {
+    hip_check(hipMemcpy2DAsync(dst, dst_stride, src, src_stride, row_bytes, rows, kind, s), what);
+  }
+}
+
+// A caller image on the device: device views are used in place, host images
+// are uploaded.  Empty views stay empty.
 template <typename T>
 DImg<T> input_img(Context& c, const r3dg_image& v, const char* name) {
   if (view_empty(v)) return DImg<T>{};
@@ -134,18 +147,16 @@ DImg<T> input_img(Context& c, const r3dg_image& v, const char* name) {
   }
   DImg<T> d = alloc_img<T>(c, v.width, v.height);
   const std::size_t row = std::size_t(v.width) * sizeof(T), bytes = row * std::size_t(v.height);
-  const bool direct = bytes >= (std::size_t{1} << 16) && host_pinned(v.data);
-  void* pin = !direct && bytes >= (std::size_t{1} << 20) ? c.pinned.get(bytes) : nullptr;
-  if (pin != nullptr) {
-    // Stage through pinned memory (released at the next stream sync).
-    c.staged_blocks.push_back(pin);
-    copy_rows(pin, row, v.data, std::size_t(v.stride) * sizeof(T), row, std::size_t(v.height));
-    hip_check(hipMemcpyAsync(d.p, pin, bytes, hipMemcpyHostToDevice, c.stream), "upload");
-    return d;
+  if (pageable(v.data)) {
+    if (void* pin = c.pinned.get(bytes)) {
+      c.staged_blocks.push_back(pin);  // released at the next stream sync
+      copy_rows(pin, row, v.data, std::size_t(v.stride) * sizeof(T), row, std::size_t(v.height));
+      hip_check(hipMemcpyAsync(d.p, pin, bytes, hipMemcpyHostToDevice, c.stream), "upload");
+      return d;
+    }
   }
-  hip_check(hipMemcpy2DAsync(d.p, std::size_t(d.s) * sizeof(T), v.data, std::size_t(v.stride) * sizeof(T), row,
-                             std::size_t(v.height), hipMemcpyHostToDevice, c.stream),
-            "upload");
+  copy_async(d.p, row, v.data, std::size_t(v.stride) * sizeof(T), row, std::size_t(v.height), hipMemcpyHostToDevice,
+             c.stream, "upload");
   return d;
 }
 
@@ -172,21 +183,18 @@ void output_img(Context& c, const r3dg_image& v, const T* src, int w, int h, std
                                           std::to_string(h));
   if (v.stride < v.width) fail(R3DG_ERROR_INVALID_ARGUMENT, std::string(name) + ": stride smaller than width");
   const std::size_t row = std::size_t(w) * sizeof(T), bytes = row * std::size_t(h);
-  if (v.memory != R3DG_DEVICE && bytes >= (std::size_t{1} << 20) && !host_pinned(v.data)) {
+  if (v.memory != R3DG_DEVICE && pageable(v.data)) {
     if (void* pin = c.pinned.get(bytes)) {
       // Into pinned memory; copied to the caller's buffer at the next sync.
       c.staged_blocks.push_back(pin);
-      hip_check(hipMemcpy2DAsync(pin, row, src, std::size_t(ss) * sizeof(T), row, std::size_t(h),
-                                 hipMemcpyDeviceToHost, c.stream),
-                "download");
+      copy_async(pin, row, src, std::size_t(ss) * sizeof(T), row, std::size_t(h), hipMemcpyDeviceToHost, c.stream,
+                 "download");
       c.staged_out.push_back({pin, v.data, row, std::size_t(h), std::size_t(v.stride) * sizeof(T)});
       return;
     }
   }
-  const hipMemcpyKind kind = v.memory == R3DG_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-  hip_check(hipMemcpy2DAsync(v.data, std::size_t(v.stride) * sizeof(T), src, std::size_t(ss) * sizeof(T), row,
-                             std::size_t(h), kind, c.stream),
-            "download");
+  copy_async(v.data, std::size_t(v.stride) * sizeof(T), src, std::size_t(ss) * sizeof(T), row, std::size_t(h),
+             v.memory == R3DG_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, c.stream, "download");
 }
 
 // A float map to the caller's buffer on stream cs (a copy stream beside the
@@ -202,20 +210,16 @@ void download_map(Context& c, hipStream_t cs, const r3dg_image& v, const DImg<fl
                                           std::to_string(m.h));
   if (v.stride < v.width) fail(R3DG_ERROR_INVALID_ARGUMENT, std::string(name) + ": stride smaller than width");
   const std::size_t row = std::size_t(m.w) * sizeof(float), rows = std::size_t(m.h), bytes = row * rows;
-  if (v.memory != R3DG_DEVICE && bytes >= (std::size_t{1} << 20) && !host_pinned(v.data)) {
+  if (v.memory != R3DG_DEVICE && pageable(v.data)) {
     if (void* pin = c.pinned.get(bytes)) {
       blocks.push_back(pin);
-      hip_check(hipMemcpy2DAsync(pin, row, m.p, std::size_t(m.s) * sizeof(float), row, rows, hipMemcpyDeviceToHost,
-                                 cs),
-                "download");
+      copy_async(pin, row, m.p, std::size_t(m.s) * sizeof(float), row, rows, hipMemcpyDeviceToHost, cs, "download");
       outs.push_back({pin, v.data, row, rows, std::size_t(v.stride) * sizeof(float)});
       return;
     }
   }
-  const hipMemcpyKind kind = v.memory == R3DG_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-  hip_check(hipMemcpy2DAsync(v.data, std::size_t(v.stride) * sizeof(float), m.p, std::size_t(m.s) * sizeof(float),
-                             row, rows, kind, cs),
-            "download");
+  copy_async(v.data, std::size_t(v.stride) * sizeof(float), m.p, std::size_t(m.s) * sizeof(float), row, rows,
+             v.memory == R3DG_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, cs, "download");
 }
 
 // Side stream that carries the downloads of a batch (the path scans use the
@@ -1831,7 +1835,7 @@ class Server {
         if (v->format != R3DG_FORMAT_NATIVE && v->format != R3DG_FORMAT_U8X257) continue;
         const std::size_t es = v->format == R3DG_FORMAT_U8X257 ? 1 : 2;
         const std::size_t row = std::size_t(v->width) * es, rows = std::size_t(v->height);
-        if (row * rows < (std::size_t{1} << 20) || host_pinned(v->data)) continue;
+        if (row * rows < (std::size_t{1} << 20) || !pageable(v->data)) continue;  // a small one is staged as it is admitted
         void* pin = c_.pinned.get(row * rows);
         if (pin == nullptr) continue;
         r->pre[k] = pin;
