@@ -164,9 +164,10 @@ struct PathArgs {
 void launch_sgm_path(int path, const PathArgs& a, int mode, hipStream_t s);
 // The eight paths of tiles whose pixels all have their job's D labels, each
 // into its own plane of bytes M = L - C (at most P2, which must be at most
-// 255).  A wave takes 64 / lps scanlines (rows for paths 0 and 1, columns for
-// the others); gprefix[t] counts the groups of all paths before tile t.
-// full_lanes: lanes per scanline for D labels, 0 if there is no such kernel.
+// 255).  A scanline takes `lanes` lanes of `labels` labels each, a wave
+// 64 / lanes scanlines (rows for paths 0 and 1, columns for the others);
+// gprefix[t] counts the groups of all paths before tile t.  full_split: for D
+// labels and a launch of that many scanlines; lanes 0 if there is no such kernel.
 struct FullArgs {
   const JobDesc* jobs;
   const TileDesc* tiles;
@@ -177,8 +178,11 @@ struct FullArgs {
   std::uint8_t* M;               // path p's plane at M + p * mstride
   std::uint64_t mstride;
 };
-int full_lanes(int D);
-void launch_full(const FullArgs& a, int lps, hipStream_t s);
+struct FullSplit {
+  int labels, lanes;
+};
+FullSplit full_split(int D, std::uint64_t scanlines);
+void launch_full(const FullArgs& a, FullSplit f, hipStream_t s);
 // The vertical and diagonal paths (2 .. 7) of tiles of at most 1024 columns,
 // row by row: np = 3 takes the three paths downwards (upwards) of a tile at
 // once and stores their sum in out[0] (out[1]) as uint16, np = 1 stores path

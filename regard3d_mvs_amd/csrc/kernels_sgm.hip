@@ -902,7 +902,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
 // The eight path scans of tiles whose pixels all have the same D labels (no
 // label ranges: single-level matches, the coarsest level of a hierarchy).
 // Nothing has to be aligned, so a scanline is LPS lanes (the power of two from
-// D / 16 on, lane q holding labels 16 q .. 16 q + 15 as packed pairs) and the
+// D / PL on, lane q holding labels PL q .. PL q + PL - 1 as packed pairs) and the
 // predecessor's path costs never leave their registers: the two neighbours
 // across lanes and the minimum over the labels are DPP moves.  A wave scans
 // 64 / LPS neighbouring scanlines in lockstep: columns of a tile row for the
@@ -914,25 +914,27 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
 //
 // Bound by the chain of a step at small sizes and by HBM at large ones (a byte
 // read and a byte written per label and path).  Aggregation of a 640x480 pair
-// with 64 labels: 0.92 ms with eight k_path launches, 0.19 ms here; 1024x768
-// with 128 labels: 3.4 ms, 0.92 ms.
-// Value of the lane below (above) in a wave; the first (last) lane keeps its own.
+// with 64 labels: 0.92 ms with eight k_path launches, 0.19 ms with 16 labels a
+// lane, 0.146 ms here; 1024x768 with 128 labels: 3.4 ms, 0.92 ms, 0.84 ms (1.9 GB
+// written and 1 GB read).
+// Value of the lane below (above) in a wave; 0 in the first (last) lane.  Like
+// the moves of the minima these fold into the operation that takes them.
 template <int LPS>
 __device__ __forceinline__ std::uint32_t lane_below(std::uint32_t v) {
   const int i = static_cast<int>(v);
-  return static_cast<std::uint32_t>(LPS <= 16 ? __builtin_amdgcn_update_dpp(i, i, 0x111, 0xF, 0xF, false)
-                                              : __builtin_amdgcn_update_dpp(i, i, 0x138, 0xF, 0xF, false));
+  return static_cast<std::uint32_t>(LPS <= 16 ? __builtin_amdgcn_update_dpp(0, i, 0x111, 0xF, 0xF, true)
+                                              : __builtin_amdgcn_update_dpp(0, i, 0x138, 0xF, 0xF, true));
 }
 template <int LPS>
 __device__ __forceinline__ std::uint32_t lane_above(std::uint32_t v) {
   const int i = static_cast<int>(v);
-  return static_cast<std::uint32_t>(LPS <= 16 ? __builtin_amdgcn_update_dpp(i, i, 0x101, 0xF, 0xF, false)
-                                              : __builtin_amdgcn_update_dpp(i, i, 0x130, 0xF, 0xF, false));
+  return static_cast<std::uint32_t>(LPS <= 16 ? __builtin_amdgcn_update_dpp(0, i, 0x101, 0xF, 0xF, true)
+                                              : __builtin_amdgcn_update_dpp(0, i, 0x130, 0xF, 0xF, true));
 }
 template <int CTRL>
 __device__ __forceinline__ std::uint32_t dpp_min(std::uint32_t v) {
   const int i = static_cast<int>(v);
-  return min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xF, 0xF, false)));
+  return min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, i, CTRL, 0xF, 0xF, true)));
 }
 // Minimum over aligned groups of LPS lanes.
 template <int LPS>
@@ -941,16 +943,24 @@ __device__ __forceinline__ std::uint32_t group_min(std::uint32_t v) {
   if constexpr (LPS >= 4) v = dpp_min<0x4E>(v);   // quad_perm 2 3 0 1
   if constexpr (LPS >= 8) v = dpp_min<0x141>(v);  // row_half_mirror
   if constexpr (LPS >= 16) v = dpp_min<0x140>(v); // row_mirror
-  if constexpr (LPS >= 32) v = min(v, static_cast<std::uint32_t>(__shfl_xor(static_cast<int>(v), 16)));
+  if constexpr (LPS >= 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = min(r[0], r[1]);
+  }
+  if constexpr (LPS >= 64) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    v = min(r[0], r[1]);
+  }
   return v;
 }
 
-template <int LPS>
+template <int LPS, int PL>
 __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
-  constexpr int S = 64 / LPS;
-  __shared__ std::uint16_t lut[256];
+  constexpr int S = 64 / LPS, W = PL / 2, B = PL / 4;
+  using Bytes = std::uint32_t __attribute__((ext_vector_type(B)));
+  __shared__ std::uint32_t lut[256];
   // The P2 table depends on the options only: the same for every job.
-  for (int k = threadIdx.x; k < 256; k += 64 * kWaves) lut[k] = A.jobs[0].lut[k];
+  for (int k = threadIdx.x; k < 256; k += 64 * kWaves) lut[k] = A.jobs[0].lut[k] * 0x10001U;
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, sc = lane / LPS, q = lane % LPS;
@@ -982,90 +992,108 @@ __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
   const int dx = path < 4 ? 0 : (path == 4 || path == 7 ? 1 : -1);
   const int nscan = horiz ? th : tw, steps = horiz ? tw : th;
   const int s = min(g * S + sc, nscan - 1);
-  const bool on = g * S + sc < nscan && 16 * q < D;
+  const bool on = g * S + sc < nscan && PL * q < D;
   const std::uint8_t* Ct = A.C + T.cell_base;
   std::uint8_t* Mt = A.M + std::uint64_t(path) * A.mstride + T.cell_base;
   const std::uint16_t* img = J.img;
-  const int img_stride = static_cast<int>(J.img_stride), iy0 = T.y0;
+  const int img_stride = static_cast<int>(J.img_stride);
   // Base columns of a mirrored job read the unmirrored image backwards.
   const int ix0 = J.mirrored != 0 ? J.width - 1 - T.x0 : T.x0, idx = J.mirrored != 0 ? -1 : 1;
-  const std::uint32_t P1x2 = static_cast<std::uint32_t>(J.p1) * 0x10001U;
-  const std::uint32_t qoff = 16U * static_cast<std::uint32_t>(min(q, D / 16 - 1));
+  const u16x2 P1x2 = as_pair(static_cast<std::uint32_t>(J.p1) * 0x10001U);
   // Sentinels for the neighbours of the first and the last label, and for the labels of idle lanes.
-  const std::uint32_t left_inf = q == 0 ? 0xFFFFFFFFU : 0U, right_inf = 16 * (q + 1) >= D ? 0xFFFFFFFFU : 0U;
+  const std::uint32_t left_inf = q == 0 ? 0xFFFFFFFFU : 0U, right_inf = PL * (q + 1) >= D ? 0xFFFFFFFFU : 0U;
+  const std::uint32_t off_inf = on ? 0U : 0xFFFFFFFFU;
 
-  // Cell and intensity of a step's pixel; the column of the next one to load
-  // is kept up to date.
-  int xr = s;
+  // Offsets of the next pixel to load: they move by a constant per step, and
+  // by another at the step a diagonal leaves the tile (left steps from now).
+  const int x0 = horiz ? (rev ? tw - 1 : 0) : s, y0 = horiz ? s : (rev ? th - 1 : 0);
+  const int sx = horiz ? (rev ? -1 : 1) : dx, sy = horiz ? 0 : (rev ? -1 : 1);
+  std::uint32_t cell = static_cast<std::uint32_t>(y0 * tw + x0) * static_cast<std::uint32_t>(D) +
+                       static_cast<std::uint32_t>(PL * min(q, D / PL - 1));
+  std::uint32_t pix = static_cast<std::uint32_t>((T.y0 + y0) * img_stride + ix0 + idx * x0) * 2U;
+  const std::uint32_t cmove = static_cast<std::uint32_t>((sy * tw + sx) * D);
+  const std::uint32_t pmove = static_cast<std::uint32_t>(sy * img_stride + idx * sx) * 2U;
+  const std::uint32_t cwrap = cmove - static_cast<std::uint32_t>(dx * tw * D);
+  const std::uint32_t pwrap = pmove - static_cast<std::uint32_t>(idx * dx * tw) * 2U;
+  int left = dx == 0 ? 1 << 30 : (dx > 0 ? nscan - s : s + 1);
+  bool start = true;
   struct In {
-    u32x4 c;
-    std::uint32_t cell;
-    std::uint16_t val;
+    Bytes c;
+    std::uint32_t cell, val;
+    bool first;  // starts a scanline
   };
-  auto load = [&](int i, In& d) {
-    const int r = rev ? steps - 1 - min(i, steps - 1) : min(i, steps - 1);
-    const int x = horiz ? r : xr, y = horiz ? s : r;
-    d.cell = static_cast<std::uint32_t>(y * tw + x) * static_cast<std::uint32_t>(D) + qoff;
-    d.c = ldb<u32x4>(Ct, d.cell);
-    d.val = ldb<std::uint16_t>(img, static_cast<std::uint32_t>((iy0 + y) * img_stride + ix0 + idx * x) * 2U);
-    if (!horiz) {
-      xr += dx;
-      xr = xr >= nscan ? 0 : (xr < 0 ? nscan - 1 : xr);
-    }
+  auto load = [&](In& d) __attribute__((always_inline)) {
+    d.cell = cell;
+    d.c = ldb<Bytes>(Ct, cell);
+    d.val = ldb<std::uint16_t>(img, pix);
+    d.first = start;
+    start = --left == 0;
+    left = start ? nscan : left;
+    cell += start ? cwrap : cmove;
+    pix += start ? pwrap : pmove;
   };
-  std::uint32_t L[8], pmin = 0, p2 = 0;
+  // Path costs, their minimum and the next step's P2, as pairs.
+  std::uint32_t L[W], pmin = 0, p2 = 0;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) L[j] = 0xFFFFFFFFU;
-  int nfirst = 0;
-  auto step = [&](int i, const In& in, const In& next) __attribute__((always_inline)) {
-    const bool first = i == nfirst;
-    // The next pixel of a diagonal that leaves the tile starts a scanline.
-    nfirst += first ? (dx == 0 ? (1 << 30) : (i == 0 ? (dx > 0 ? nscan - s : s + 1) : nscan)) : 0;
-    const std::uint32_t mp = first ? 0U : pmin, pen = first ? 0U : pmin + p2;
-    const std::uint32_t PENx2 = pen * 0x10001U, MPx2 = mp * 0x10001U;
+  for (int j = 0; j < W; ++j) L[j] = 0xFFFFFFFFU;
+  auto step = [&](const In& in, const In& next) __attribute__((always_inline)) {
+    const u16x2 MP = as_pair(in.first ? 0U : pmin), PEN = as_pair(in.first ? 0U : pmin + p2);
     // P2 of the next step, read while this one computes.
-    const std::uint32_t ia = in.val, ib = next.val;
-    const std::uint32_t p2n = lut[(max(ia, ib) - min(ia, ib)) >> 8];
-    const std::uint32_t below = lane_below<LPS>(L[7]) | left_inf, above = lane_above<LPS>(L[0]) | right_inf;
-    std::uint32_t Q[9], M[8], m;
+    p2 = lut[__builtin_amdgcn_sad_u16(in.val, next.val, 0U) >> 8];
+    const std::uint32_t below = lane_below<LPS>(L[W - 1]) | left_inf, above = lane_above<LPS>(L[0]) | right_inf;
+    std::uint32_t Q[W + 1], M[W];
     Q[0] = __builtin_amdgcn_alignbyte(L[0], below, 2U);
 #pragma unroll
-    for (int j = 1; j < 8; ++j) Q[j] = __builtin_amdgcn_alignbyte(L[j], L[j - 1], 2U);
-    Q[8] = __builtin_amdgcn_alignbyte(above, L[7], 2U);
+    for (int j = 1; j < W; ++j) Q[j] = __builtin_amdgcn_alignbyte(L[j], L[j - 1], 2U);
+    Q[W] = __builtin_amdgcn_alignbyte(above, L[W - 1], 2U);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < W; ++j) {
       const std::uint32_t Cx2 = __builtin_amdgcn_perm(0U, in.c[j >> 1], (j & 1) ? 0x0c030c02U : 0x0c010c00U);
-      const u16x2 nb =
-          __builtin_elementwise_add_sat(__builtin_elementwise_min(as_pair(Q[j]), as_pair(Q[j + 1])), as_pair(P1x2));
-      const u16x2 best = __builtin_elementwise_min(__builtin_elementwise_min(as_pair(L[j]), nb), as_pair(PENx2));
-      M[j] = as_u32(best - as_pair(MPx2));
+      const u16x2 nb = __builtin_elementwise_add_sat(__builtin_elementwise_min(as_pair(Q[j]), as_pair(Q[j + 1])), P1x2);
+      const u16x2 best = __builtin_elementwise_min(__builtin_elementwise_min(as_pair(L[j]), nb), PEN);
+      M[j] = as_u32(best - MP);
       L[j] = as_u32(as_pair(M[j]) + as_pair(Cx2));
     }
-    m = L[0];
+    u16x2 m[W];
 #pragma unroll
-    for (int j = 1; j < 8; ++j) m = as_u32(__builtin_elementwise_min(as_pair(m), as_pair(L[j])));
-    m = min(m & 0xFFFFU, m >> 16);
-    pmin = group_min<LPS>(on ? m : 0xFFFFU);
+    for (int j = 0; j < W; ++j) m[j] = as_pair(L[j]);
+#pragma unroll
+    for (int n = W / 2; n > 0; n /= 2)
+#pragma unroll
+      for (int j = 0; j < n; ++j) m[j] = __builtin_elementwise_min(m[j], m[j + n]);
+    const std::uint32_t both = as_u32(m[0]) | off_inf;
+    // Equal halves from here on: the order of the words is the order of the costs.
+    pmin = group_min<LPS>(as_u32(__builtin_elementwise_min(as_pair(both), as_pair(both >> 16 | both << 16))));
     if (on) {
-      u32x4 o;
+      Bytes o;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = __builtin_amdgcn_perm(M[2 * j + 1], M[2 * j], 0x06040200U);
-      stb<u32x4>(Mt, in.cell, o);
+      for (int j = 0; j < B; ++j) o[j] = __builtin_amdgcn_perm(M[2 * j + 1], M[2 * j], 0x06040200U);
+      stb<Bytes>(Mt, in.cell, o);
     }
-    p2 = p2n;
   };
-  // Costs and intensities three steps ahead; the loop is unrolled over the
-  // four sets so that every index is a constant.
-  constexpr int N = 4;
+  // Costs and intensities N - 1 steps ahead; the loops are unrolled over the N
+  // sets so that every index is a constant.  The first one loads in every step.
+  constexpr int N = 8;
   In in[N];
 #pragma unroll
-  for (int j = 0; j < N - 1; ++j) load(j, in[j]);
-  for (int i = 0; i < steps; i += N) {
+  for (int j = 0; j < N - 1; ++j) {
+    in[j] = In{};
+    if (j < steps) load(in[j]);
+  }
+  int i = 0;
+  for (; i + 2 * N - 1 <= steps; i += N) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      load(in[(j + N - 1) % N]);
+      step(in[j], in[(j + 1) % N]);
+    }
+  }
+  for (; i < steps; i += N) {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       if (i + j < steps) {
-        load(i + j + N - 1, in[(j + N - 1) % N]);
-        step(i + j, in[j], in[(j + 1) % N]);
+        if (i + j + N - 1 < steps) load(in[(j + N - 1) % N]);
+        step(in[j], in[(j + 1) % N]);
       }
     }
   }
@@ -1847,21 +1875,39 @@ void launch_sgm_path(int path, const PathArgs& a, int mode, hipStream_t s) {
   }
 }
 
-int full_lanes(int D) {
-  int lps = 2;
-  while (lps * kLabelAlign < D) lps *= 2;
-  return lps <= 32 ? lps : 0;
+// Four labels a lane where the launch then still has at most 1.5 waves per
+// SIMD: there a step's chain is all that counts (384 x 288 with 64 labels: 75 us
+// against 85 with eight, 127 with sixteen).  Eight otherwise: with more waves the
+// shorter steps of four no longer pay for the instructions they repeat
+// (640 x 480 with 64 labels: 172 us against 146, sixteen 176).
+FullSplit full_split(int D, std::uint64_t scanlines) {
+  auto lanes = [&](int labels) {
+    int n = 2;
+    while (n * labels < D) n *= 2;
+    return n;
+  };
+  int dev = 0, cus = 0;
+  (void)hipGetDevice(&dev);
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  const std::uint64_t waves = (scanlines * std::uint64_t(lanes(4)) + 63) / 64;
+  if (lanes(4) <= 32 && waves <= std::uint64_t(6 * std::max(cus, 1))) return {4, lanes(4)};
+  return lanes(8) <= 64 ? FullSplit{8, lanes(8)} : FullSplit{0, 0};
 }
 
-void launch_full(const FullArgs& a, int lps, hipStream_t s) {
+void launch_full(const FullArgs& a, FullSplit f, hipStream_t s) {
   if (a.groups == 0) return;
   const dim3 grid(static_cast<unsigned>((a.groups + kWaves - 1) / kWaves));
-  switch (lps) {
-    case 2: k_full<2><<<grid, 64 * kWaves, 0, s>>>(a); break;
-    case 4: k_full<4><<<grid, 64 * kWaves, 0, s>>>(a); break;
-    case 8: k_full<8><<<grid, 64 * kWaves, 0, s>>>(a); break;
-    case 16: k_full<16><<<grid, 64 * kWaves, 0, s>>>(a); break;
-    default: k_full<32><<<grid, 64 * kWaves, 0, s>>>(a); break;
+  switch (f.labels * 64 + f.lanes) {
+    case 4 * 64 + 4: k_full<4, 4><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 4 * 64 + 8: k_full<8, 4><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 4 * 64 + 16: k_full<16, 4><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 4 * 64 + 32: k_full<32, 4><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 8 * 64 + 2: k_full<2, 8><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 8 * 64 + 4: k_full<4, 8><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 8 * 64 + 8: k_full<8, 8><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 8 * 64 + 16: k_full<16, 8><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    case 8 * 64 + 32: k_full<32, 8><<<grid, 64 * kWaves, 0, s>>>(a); break;
+    default: k_full<64, 8><<<grid, 64 * kWaves, 0, s>>>(a); break;
   }
 }
 

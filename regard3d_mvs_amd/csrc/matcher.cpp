@@ -826,10 +826,16 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     sum_groups += g[nt];
   }
   std::vector<std::uint64_t> fp;
-  int lps = 0;
+  FullSplit split{0, 0};
   if (full) {
-    for (const TileDesc& T : td) lps = std::max(lps, full_lanes(A.full[std::size_t(T.job)]));
-    const int per = 64 / lps;
+    int labels = 0;
+    std::uint64_t scanlines = 0;
+    for (const TileDesc& T : td) {
+      labels = std::max(labels, A.full[std::size_t(T.job)]);
+      scanlines += std::uint64_t(2 * T.h + 6 * T.w);
+    }
+    split = full_split(labels, scanlines);
+    const int per = 64 / split.lanes;
     fp.assign(std::size_t(nt) + 1, 0);
     for (int t = 0; t < nt; ++t) {
       const TileDesc& T = td[std::size_t(t)];
@@ -926,7 +932,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     fa.C = ch.C.get();
     fa.M = ch.M.get();
     fa.mstride = ch.stride;
-    launch_full(fa, lps, c.stream);
+    launch_full(fa, split, c.stream);
     check_launch();
     c.agg_launches += 1;
     // Per cell and path its cost read and its byte stored; per tile pixel and
@@ -1056,7 +1062,7 @@ std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
   for (int t = 0; t < nt; ++t) {
     const auto job = std::size_t(A.td[std::size_t(t)].job);
     const Aggregate kind = !roomy ? Aggregate::kScan
-                           : planes && A.full[job] > 0 && full_lanes(A.full[job]) > 0 ? Aggregate::kFull
+                           : planes && A.full[job] > 0 && full_split(A.full[job], 0).lanes > 0 ? Aggregate::kFull
                                                                                       : Aggregate::kSweep;
     const std::uint64_t n = A.tcells[std::size_t(t)];
     if (out.empty() || out.back().kind != kind || cells + n > cap) {

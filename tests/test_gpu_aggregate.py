@@ -69,3 +69,11 @@ def test_small_budget_scans(hip_runtime, gpu):  # noqa: F811
         assert got.aggregate_launches > ref.aggregate_launches
         for k in ("disparity", "confidence", "labels", "lr_mask"):
             same_bits(getattr(got, k), getattr(ref, k))
+
+
+# Enough scanlines that a lane takes eight labels also where D is small
+# (16 labels: 4 lanes of four, 24576 scanlines at 256 CUs).
+@pytest.mark.parametrize("nd", [16, 32, 48, 128])
+def test_full_range_many_scanlines(gpu, nd):  # noqa: F811
+    left, right, _ = render_pair(Texture(43), 2600, 21, lambda x, y: 5.0 + 0.002 * x + 0.1 * y)
+    _match_both(gpu, left, right, None, None, 0, nd, StereoOptions(levels=0, **RAW))
