@@ -204,13 +204,14 @@ struct SweepArgs {
 };
 // Launch shape for tiles of at most max_w columns and max_chunks chunks a row:
 // words of an LDS row, words of a scratch row (0: none needed), the blocks
-// that run at once.  ok is false where the kernel does not apply.
+// that run at once, the chunks a thread holds.  mean_chunks: of the rows of the
+// tile with most.  ok is false where the kernel does not apply.
 struct SweepPlan {
   bool ok;
-  int wpad, cap, swords, lds_bytes, blocks;
+  int wpad, cap, swords, lds_bytes, blocks, held;
 };
 constexpr int kSweepRowPad = 8;  // words after an LDS row that a window may read
-SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks);
+SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks, std::uint64_t mean_chunks);
 void launch_sweep(const SweepArgs& a, int np, bool bytes, const SweepPlan& p, std::uint64_t blocks, hipStream_t s);
 // Extra elements S, C and a plane hold past their last cell.
 constexpr std::size_t kSPad = 64;

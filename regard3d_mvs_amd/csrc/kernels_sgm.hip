@@ -1115,7 +1115,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
 // conflicts).  Pixels past the LDS rows (cap words, the end of rows with many
 // wide pixels) use rows of the same layout in a global scratch, one per
 // parity.  Each row is two phases between barriers: windows and minima of the
-// last row are read, the new costs stay in registers (kHeld chunks per thread;
+// last row are read, the new costs stay in registers (H chunks per thread;
 // later ones are past cap and go to scratch) until every thread has read, then
 // they replace the last row.  Costs, map and records are loaded one row ahead.
 //
@@ -1123,8 +1123,6 @@ __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
 // paths) and the barriers.  The six paths of the 24 MP pair's finest level:
 // 19 ms by k_path; here 12 ms beside the two horizontal scans, on fewer CUs.
 constexpr int kSweepThreads = 1024;
-template <int NP>
-constexpr int kHeld = NP == 3 ? 2 : 4;
 
 // Barrier that orders LDS accesses only: loads in flight and stores of sums
 // stay in flight across it.
@@ -1134,10 +1132,10 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int NP, bool kByte>
+template <int NP, bool kByte, int H>
 __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
   static_assert(NP == 1 || !kByte, "a byte holds L - C of one path");
-  constexpr int H = kHeld<NP>, N = kSweepThreads;
+  constexpr int N = kSweepThreads;
   extern __shared__ __attribute__((aligned(16))) std::uint32_t lds[];
   // info[3][wpad] (pixel records of three rows), pmin[2][NP][wpad], lut, item, rows[NP][cap + pad].
   const int wpad = A.wpad, cap = A.cap, rstride = cap + kSweepRowPad;
@@ -1911,7 +1909,12 @@ void launch_full(const FullArgs& a, FullSplit f, hipStream_t s) {
   }
 }
 
-SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks) {
+// Two chunks held per thread, where three paths leave no registers for more or
+// no tile's mean row has more chunks than threads (rows past twice that are
+// rare there, and the sweep of one path is 3 % faster than with four: 2.94 ms
+// against 3.02 for the 1080p pair's aggregation); four for wider rows (the 24 MP
+// pair's: 17.5 ms against 17.7 with two).
+SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks, std::uint64_t mean_chunks) {
   SweepPlan p{};
   if (max_w > kSweepThreads) return p;
   int dev = 0, cus = 0, lds = 0;
@@ -1919,10 +1922,10 @@ SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks) {
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   (void)hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
   const int fixed = 4 * (6 * max_w + 2 * np * max_w + 128 + 4);
-  const int held = np == 3 ? kHeld<3> : kHeld<1>;
+  p.held = np == 3 || mean_chunks <= kSweepThreads ? 2 : 4;
   const int need = static_cast<int>(std::min<std::uint64_t>(8 * std::uint64_t(max_chunks) + std::uint64_t(max_w) + 2, 1 << 20));
   p.wpad = max_w;
-  p.cap = std::min({(lds - fixed) / (4 * np) - kSweepRowPad, 8 * kSweepThreads * held, need});
+  p.cap = std::min({(lds - fixed) / (4 * np) - kSweepRowPad, 8 * kSweepThreads * p.held, need});
   if (p.cap < 1024) return p;
   p.lds_bytes = fixed + 4 * np * (p.cap + kSweepRowPad);
   p.swords = p.cap >= need ? 0 : need + 16;
@@ -1932,25 +1935,25 @@ SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks) {
 }
 
 namespace {
-template <int NP, bool kByte>
+template <int NP, bool kByte, int H>
 void sweep_launch(const SweepArgs& a, const SweepPlan& p, std::uint64_t blocks, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(std::min<std::uint64_t>(a.units, blocks)));
   // Dynamic LDS past 64 KB has to be asked for (a failure is the launch's).
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep<NP, kByte>),
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep<NP, kByte, H>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, p.lds_bytes) != hipSuccess)
     return;
-  k_sweep<NP, kByte><<<grid, kSweepThreads, p.lds_bytes, s>>>(a);
+  k_sweep<NP, kByte, H><<<grid, kSweepThreads, p.lds_bytes, s>>>(a);
 }
 }  // namespace
 
 void launch_sweep(const SweepArgs& a, int np, bool bytes, const SweepPlan& p, std::uint64_t blocks, hipStream_t s) {
   if (a.units == 0) return;
   if (np == 3) {
-    sweep_launch<3, false>(a, p, blocks, s);
+    sweep_launch<3, false, 2>(a, p, blocks, s);
   } else if (bytes) {
-    sweep_launch<1, true>(a, p, blocks, s);
+    p.held == 2 ? sweep_launch<1, true, 2>(a, p, blocks, s) : sweep_launch<1, true, 4>(a, p, blocks, s);
   } else {
-    sweep_launch<1, false>(a, p, blocks, s);
+    p.held == 2 ? sweep_launch<1, false, 2>(a, p, blocks, s) : sweep_launch<1, false, 4>(a, p, blocks, s);
   }
 }
 

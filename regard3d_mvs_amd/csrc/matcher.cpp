@@ -788,8 +788,11 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   std::array<Sweep, 2> sw{};
   int heavy = 0;
   if (kind == Aggregate::kSweep) {
-    sw[0].plan = sweep_plan(1, A.max_w, A.max_row_chunks);
-    sw[1].plan = sweep_plan(3, A.max_w, A.max_row_chunks);
+    std::uint64_t mean_chunks = 0;
+    for (int t = 0; t < nt; ++t)
+      mean_chunks = std::max(mean_chunks, A.tcells[std::size_t(t0 + t)] / std::uint64_t(td[std::size_t(t)].h) / kLabelAlign);
+    sw[0].plan = sweep_plan(1, A.max_w, A.max_row_chunks, mean_chunks);
+    sw[1].plan = sweep_plan(3, A.max_w, A.max_row_chunks, mean_chunks);
     const auto mean_words = [&](std::int32_t t) {
       const TileDesc& T = td[std::size_t(t)];
       return A.tcells[std::size_t(t0 + t)] / std::uint64_t(T.h) / 2 + std::uint64_t(T.w);

@@ -77,3 +77,13 @@ def test_small_budget_scans(hip_runtime, gpu):  # noqa: F811
 def test_full_range_many_scanlines(gpu, nd):  # noqa: F811
     left, right, _ = render_pair(Texture(43), 2600, 21, lambda x, y: 5.0 + 0.002 * x + 0.1 * y)
     _match_both(gpu, left, right, None, None, 0, nd, StereoOptions(levels=0, **RAW))
+
+
+def test_sweep_few_wide_rows(gpu):  # noqa: F811
+    """Rows of far more chunks than a thread holds two of, in tiles whose mean
+    row has fewer than one per thread: noise in a few rows widens their ranges."""
+    left, right, _ = render_pair(Texture(47), 480, 400, lambda x, y: 60.0 + 0.02 * x + 0.01 * y)
+    rng = np.random.default_rng(47)
+    right = right.copy()
+    right[200:206] = rng.integers(0, 65536, right[200:206].shape)
+    _match_both(gpu, left, right, None, None, 0, 256, StereoOptions(levels=1, range_margin=4, **RAW))
