@@ -715,8 +715,8 @@ __device__ __forceinline__ V pick(const V (&a)[N], int q) {
 // combine_pairs per grid pixel (multi_stereo.cpp:103-213), double precision
 // in the reference's order of operations.
 //
-// Bound by vector instructions (about 1100 a wave for 4 pairs, most of them in
-// double precision): 4 pairs of 27 Mpx take 0.93 ms.  Every list of pairs is
+// Bound by vector instructions (about 950 a wave for 4 pairs, a third of them in
+// double precision): 4 pairs of 27 Mpx take 0.92 ms.  Every list of pairs is
 // indexed by the pair and unrolled to N, so that it lives in registers; lists
 // filled and indexed at run time went to scratch memory, and the kernel took
 // 2.1 ms.  Sums depend on the order of the pairs: it is ascending until a pair

@@ -926,8 +926,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
 // Bound by the chain of a step at small sizes and by HBM at large ones (a byte
 // read and a byte written per label and path).  Aggregation of a 640x480 pair
 // with 64 labels: 0.92 ms with eight k_path launches, 0.19 ms with 16 labels a
-// lane, 0.146 ms here; 1024x768 with 128 labels: 3.4 ms, 0.92 ms, 0.84 ms (1.9 GB
-// written and 1 GB read).
+// lane, 0.147 ms here; 1024x768 with 128 labels: 3.4 ms, 0.92 ms, 0.76 ms (1.9 GB
+// written and 2 GB read).
 // Value of the lane below (above) in a wave; 0 in the first (last) lane.  Like
 // the moves of the minima these fold into the operation that takes them.
 template <int LPS>
@@ -1130,9 +1130,10 @@ __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
 // later ones are past cap and go to scratch) until every thread has read, then
 // they replace the last row.  Costs, map and records are loaded one row ahead.
 //
-// Bound by VALU issue (about 180 instructions per chunk and path with three
-// paths) and the barriers.  The six paths of the 24 MP pair's finest level:
-// 19 ms by k_path; here 12 ms beside the two horizontal scans, on fewer CUs.
+// Bound by CU time: a block fills its CU's LDS and registers, and its 16 waves
+// issue vector instructions (about 180 per chunk and path with three paths, 260
+// with one) in 60 to 75% of the time, between the two barriers of a row.  The
+// six paths of the 24 MP pair's finest level: 19 ms by k_path; 11.5 ms here.
 constexpr int kSweepThreads = 1024;
 
 // Barrier that orders LDS accesses only: loads in flight and stores of sums
@@ -1469,10 +1470,11 @@ __device__ __forceinline__ std::uint32_t chunk_key(const std::uint32_t (&V)[8], 
 // next to the winner; last a thread per pixel fits and checks.  Chunks past
 // the kSelHeld a thread keeps are summed again for the second step.
 //
-// HBM-bound: the chunk's slices or planes once, 12 bytes per pixel (5.3 TB/s
-// with eight slices).  With a quad of lanes per pixel, 8 labels a lane, half
+// HBM-bound: the chunk's slices or planes once, 12 bytes per pixel (5.5 TB/s at
+// 24 MP).  With a quad of lanes per pixel, 8 labels a lane, half
 // the lanes idled on pixels of 16 labels: selection of 1024x768 with 128
-// labels 1.17 ms, 0.70 ms here; of the 24 MP pair 5.75 ms, 5.38 ms.
+// labels 1.17 ms, 0.69 ms here; of the 24 MP pair, whose paths then were eight
+// uint16 slices, 5.75 and 5.38 ms, 4.07 with bytes and sums of three paths.
 constexpr int kSelThreads = 256, kSelPx = 1024, kSelHeld = 4;
 template <bool kBytes>
 __global__ __launch_bounds__(kSelThreads) void k_select(const JobDesc* __restrict__ jobs,
