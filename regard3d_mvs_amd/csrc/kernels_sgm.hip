@@ -385,7 +385,7 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
       w[q] = v;
     }
     *reinterpret_cast<uint4*>(out + 16 * std::size_t(k)) = make_uint4(w[0], w[1], w[2], w[3]);
-    mout[k] = static_cast<std::uint32_t>(xa) | static_cast<std::uint32_t>(jb / kLabelAlign) << 16;
+    mout[k] = map_entry(xa, jb / kLabelAlign);
   };
   if (staged) {
     const bool mapped = chunks <= static_cast<std::uint32_t>(kMap);
@@ -1006,7 +1006,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
   const bool on = g * S + sc < nscan && PL * q < D;
   const std::uint8_t* Ct = A.C + T.cell_base;
   std::uint8_t* Mt = A.M + std::uint64_t(path) * A.mstride + T.cell_base;
-  const std::uint16_t* img = J.img;
+  const std::uint16_t* img = J.img + std::int64_t(T.y0) * J.img_stride;
   const int img_stride = static_cast<int>(J.img_stride);
   // Base columns of a mirrored job read the unmirrored image backwards.
   const int ix0 = J.mirrored != 0 ? J.width - 1 - T.x0 : T.x0, idx = J.mirrored != 0 ? -1 : 1;
@@ -1021,7 +1021,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
   const int sx = horiz ? (rev ? -1 : 1) : dx, sy = horiz ? 0 : (rev ? -1 : 1);
   std::uint32_t cell = static_cast<std::uint32_t>(y0 * tw + x0) * static_cast<std::uint32_t>(D) +
                        static_cast<std::uint32_t>(PL * min(q, D / PL - 1));
-  std::uint32_t pix = static_cast<std::uint32_t>((T.y0 + y0) * img_stride + ix0 + idx * x0) * 2U;
+  std::uint32_t pix = static_cast<std::uint32_t>(y0 * img_stride + ix0 + idx * x0) * 2U;
   const std::uint32_t cmove = static_cast<std::uint32_t>((sy * tw + sx) * D);
   const std::uint32_t pmove = static_cast<std::uint32_t>(sy * img_stride + idx * sx) * 2U;
   const std::uint32_t cwrap = cmove - static_cast<std::uint32_t>(dx * tw * D);
@@ -1213,14 +1213,14 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
     // bit 30 a predecessor exists, bit 31 the window needs the general read
     // (past a sentinel on either side, or in scratch).
     auto window = [&](std::uint32_t m, const u32x2& own, const u32x2* linfo, int p) {
-      const int x = static_cast<int>(m & 0xFFFFU), xp = x - path_dx(p);
+      const int x = map_col(m), xp = x - path_dx(p);
       const bool use = xp >= 0 && xp < w;
       const int xq = use ? xp : 0;
       const u32x2 pi = linfo[xq];
       const std::uint32_t ia = own.y >> 16, ib = pi.y >> 16;
       const std::uint32_t p2 = lut[(max(ia, ib) - min(ia, ib)) >> 8];
       const int pw = static_cast<int>(pi.x >> 24) * 8, base = 8 * static_cast<int>(pi.x & 0xFFFFFFU) + xq + 1;
-      const int k0 = static_cast<int>(own.y & 0xFFFFU) + kLabelAlign * static_cast<int>(m >> 16) -
+      const int k0 = static_cast<int>(own.y & 0xFFFFU) + kLabelAlign * map_place(m) -
                      static_cast<int>(pi.y & 0xFFFFU);
       const bool far = static_cast<unsigned>(k0 + 1) > static_cast<unsigned>(2 * pw - 14) || base + pw >= cap;
       const std::uint32_t at = use && !far ? static_cast<std::uint32_t>(base + ((k0 - 1) >> 1)) : 0U;
@@ -1230,7 +1230,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
     // A chunk's column, and what its row needs: bit 16 the pixel's first
     // chunk, bit 17 its last, bit 18 the pixel's costs go to LDS.
     auto place = [&](std::uint32_t m, const u32x2& own) {
-      const int x = static_cast<int>(m & 0xFFFFU), cc = static_cast<int>(m >> 16), n16 = static_cast<int>(own.x >> 24);
+      const int x = map_col(m), cc = map_place(m), n16 = static_cast<int>(own.x >> 24);
       const bool in_lds = 8 * (static_cast<int>(own.x & 0xFFFFFFU) + n16) + x + 1 < cap;
       return static_cast<std::uint32_t>(x) | (cc == 0 ? 1U << 16 : 0U) | (cc == n16 - 1 ? 1U << 17 : 0U) |
              (in_lds ? 1U << 18 : 0U);
@@ -1244,7 +1244,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) pre[r][p] = 0;
         if (tid + N * r < n) {
-          const u32x2 own = cinfo[cm[r] & 0xFFFFU];
+          const u32x2 own = cinfo[map_col(cm[r])];
           flags[r] = place(cm[r], own);
 #pragma unroll
           for (int p = 0; p < NP; ++p) pre[r][p] = top ? 0U : window(cm[r], own, linfo, p);
@@ -1282,7 +1282,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
       // Cx2) into L, their sum to S, their minima to cmin.
       auto chunk = [&](int k, std::uint32_t m, const std::uint32_t (&pp)[NP], const std::uint32_t (&Cx2)[8],
                        std::uint32_t (&L)[NP][8]) __attribute__((always_inline)) {
-        const int x = static_cast<int>(m & 0xFFFFU);
+        const int x = map_col(m);
         std::uint32_t sum[8];
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
@@ -1299,7 +1299,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
               const int xq = x - path_dx(p);
               const u32x2 own = cinfo[x], pi = linfo[xq];
               const int pw = static_cast<int>(pi.x >> 24) * 8, base = 8 * static_cast<int>(pi.x & 0xFFFFFFU) + xq + 1;
-              const int k0 = static_cast<int>(own.y & 0xFFFFU) + kLabelAlign * static_cast<int>(m >> 16) -
+              const int k0 = static_cast<int>(own.y & 0xFFFFU) + kLabelAlign * map_place(m) -
                              static_cast<int>(pi.y & 0xFFFFU);
               const int w0 = (k0 - 1) >> 1;
               if (base + pw < cap) {
@@ -1380,7 +1380,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs A) {
         std::uint32_t Cx2[8], X[NP][8], pp[NP];
         const std::uint32_t m = ldb<std::uint32_t>(tmap, ((first >> 4) + static_cast<std::uint32_t>(k)) * 4U);
         unpack(ldb<u32x4>(Ct, first + 16U * static_cast<std::uint32_t>(k)), Cx2);
-        const u32x2 own = cinfo[m & 0xFFFFU];
+        const u32x2 own = cinfo[map_col(m)];
 #pragma unroll
         for (int p = 0; p < NP; ++p) pp[p] = i == 0 ? 0U : window(m, own, linfo, p);
         chunk(k, m, pp, Cx2, X);
@@ -1577,11 +1577,11 @@ __global__ __launch_bounds__(kSelThreads) void k_select(const JobDesc* __restric
     const int kn = static_cast<int>((pix_off(recl) + pix_num(recl)) / kLabelAlign);
     for (int k = tid; k < kn; k += kSelThreads) {
       const std::uint32_t m = rmap[k];
-      const int x = static_cast<int>(m & 0xFFFFU);
+      const int x = map_col(m);
       if (x < xb || x >= xe) continue;
       std::uint32_t V[8];
       load(k, V);
-      const int d0 = x - pix_lo(pix[px + x]) - kLabelAlign * static_cast<int>(m >> 16) + D - 1;
+      const int d0 = x - pix_lo(pix[px + x]) - kLabelAlign * map_place(m) + D - 1;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         atomicMin(&keys[d0 - 2 * j], (V[j] << 16) | static_cast<std::uint32_t>(x));
@@ -1602,21 +1602,21 @@ __global__ __launch_bounds__(kSelThreads) void k_select(const JobDesc* __restric
     const int k = ka + tid + kSelThreads * i;
     if (k < kb) {
       load(k, V[i]);
-      atomicMin(&best[(m[i] & 0xFFFFU) - x0], chunk_key(V[i], (m[i] >> 16) * kLabelAlign));
+      atomicMin(&best[map_col(m[i]) - x0], chunk_key(V[i], static_cast<std::uint32_t>(map_place(m[i]) * kLabelAlign)));
     }
   }
   for (int k = ka + tid + kSelThreads * kSelHeld; k < kb; k += kSelThreads) {
     std::uint32_t X[8];
     const std::uint32_t mm = rmap[k];
     load(k, X);
-    atomicMin(&best[(mm & 0xFFFFU) - x0], chunk_key(X, (mm >> 16) * kLabelAlign));
+    atomicMin(&best[map_col(mm) - x0], chunk_key(X, static_cast<std::uint32_t>(map_place(mm) * kLabelAlign)));
   }
   __syncthreads();
   // Best cost of a chunk outside the winner and its neighbours (labels w - 1
   // .. w + 1, halves a .. a + 2 of the chunk: words a / 2 and a / 2 + 1).
   auto outside = [&](std::uint32_t mm, const std::uint32_t (&X)[8]) __attribute__((always_inline)) {
-    const int x = static_cast<int>(mm & 0xFFFFU) - x0;
-    const int a = static_cast<int>(best[x] & 0xFFFFU) - 1 - static_cast<int>(mm >> 16) * kLabelAlign, j0 = a >> 1;
+    const int x = map_col(mm) - x0;
+    const int a = static_cast<int>(best[x] & 0xFFFFU) - 1 - map_place(mm) * kLabelAlign, j0 = a >> 1;
     std::uint32_t w0 = 0xFFFFFFFFU, w1 = 0xFFFFFFFFU, lowest = 0xFFFFFFFFU;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {

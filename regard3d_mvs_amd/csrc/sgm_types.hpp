@@ -40,6 +40,13 @@ __host__ __device__ constexpr std::uint32_t pix_off(std::uint64_t r) { return st
 __host__ __device__ constexpr int pix_num(std::uint64_t r) { return int((r >> 24) & 0xFFU) * kLabelAlign; }
 __host__ __device__ constexpr int pix_lo(std::uint64_t r) { return int((r >> 32) & 0xFFFFU); }
 __host__ __device__ constexpr int pix_val(std::uint64_t r) { return int(r >> 48); }
+// Chunk map entry: the chunk's column in the tile (24 bits: a row of 2^24 columns
+// would have as many chunks) and its place in the pixel.
+__host__ __device__ constexpr std::uint32_t map_entry(int col, int place) {
+  return std::uint32_t(col) | std::uint32_t(place) << 24;
+}
+__host__ __device__ constexpr int map_col(std::uint32_t m) { return int(m & 0xFFFFFFU); }
+__host__ __device__ constexpr int map_place(std::uint32_t m) { return int(m >> 24); }
 constexpr int kMaxLevels = 13;
 
 struct JobDesc {

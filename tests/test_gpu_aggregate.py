@@ -87,3 +87,14 @@ def test_sweep_few_wide_rows(gpu):  # noqa: F811
     right = right.copy()
     right[200:206] = rng.integers(0, 65536, right[200:206].shape)
     _match_both(gpu, left, right, None, None, 0, 256, StereoOptions(levels=1, range_margin=4, **RAW))
+
+
+# One tile of more columns than 16 bits count: full-range scans, path scans
+# with label ranges, and penalties past a byte.
+@pytest.mark.parametrize("levels,p2", [(0, 100), (1, 100), (0, 300)])
+def test_tile_of_70000_columns(gpu, levels, p2):  # noqa: F811
+    rng = np.random.default_rng(53)
+    left = rng.integers(0, 65536, (24, 70000)).astype(np.uint16)
+    right = np.roll(left, -9, 1)
+    _match_both(gpu, left, right, None, None, 0, 32,
+                StereoOptions(levels=levels, p1=10, p2=p2, tile_size=100000, tile_margin=4, **RAW))
