@@ -9,6 +9,7 @@
 #include <mutex>
 
 #include "sgm_types.hpp"
+#include "sweep_plan.hpp"
 
 namespace r3dg {
 
@@ -201,15 +202,7 @@ struct SweepArgs {
   std::uint32_t* queue;
   int wpad, cap, swords;         // SweepPlan
 };
-// Launch shape for tiles of at most max_w columns and max_chunks chunks a row:
-// words of an LDS row, words of a scratch row (0: none needed), the blocks
-// that run at once, the chunks a thread holds.  mean_chunks: of the rows of the
-// tile with most.  ok is false where the kernel does not apply.
-struct SweepPlan {
-  bool ok;
-  int wpad, cap, swords, lds_bytes, blocks, held;
-};
-constexpr int kSweepRowPad = 8;  // words after an LDS row that a window may read
+// size_sweep for the current device.
 SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks, std::uint64_t mean_chunks);
 void launch_sweep(const SweepArgs& a, int np, bool bytes, const SweepPlan& p, std::uint64_t blocks, hipStream_t s);
 // Extra elements S, C and a plane hold past their last cell.

@@ -1134,8 +1134,6 @@ __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
 // issue vector instructions (about 180 per chunk and path with three paths, 260
 // with one) in 60 to 75% of the time, between the two barriers of a row.  The
 // six paths of the 24 MP pair's finest level: 19 ms by k_path; 11.5 ms here.
-constexpr int kSweepThreads = 1024;
-
 // Barrier that orders LDS accesses only: loads in flight and stores of sums
 // stay in flight across it.
 __device__ __forceinline__ void lds_barrier() {
@@ -1922,29 +1920,12 @@ void launch_full(const FullArgs& a, FullSplit f, hipStream_t s) {
   }
 }
 
-// Two chunks held per thread, where three paths leave no registers for more or
-// no tile's mean row has more chunks than threads (rows past twice that are
-// rare there, and the sweep of one path is 3 % faster than with four: 2.94 ms
-// against 3.02 for the 1080p pair's aggregation); four for wider rows (the 24 MP
-// pair's: 17.5 ms against 17.7 with two).
 SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks, std::uint64_t mean_chunks) {
-  SweepPlan p{};
-  if (max_w > kSweepThreads) return p;
   int dev = 0, cus = 0, lds = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   (void)hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-  const int fixed = 4 * (6 * max_w + 2 * np * max_w + 128 + 4);
-  p.held = np == 3 || mean_chunks <= kSweepThreads ? 2 : 4;
-  const int need = static_cast<int>(std::min<std::uint64_t>(8 * std::uint64_t(max_chunks) + std::uint64_t(max_w) + 2, 1 << 20));
-  p.wpad = max_w;
-  p.cap = std::min({(lds - fixed) / (4 * np) - kSweepRowPad, 8 * kSweepThreads * p.held, need});
-  if (p.cap < 1024) return p;
-  p.lds_bytes = fixed + 4 * np * (p.cap + kSweepRowPad);
-  p.swords = p.cap >= need ? 0 : need + 16;
-  p.blocks = std::max(cus, 1);
-  p.ok = true;
-  return p;
+  return size_sweep(np, max_w, max_chunks, mean_chunks, cus, lds);
 }
 
 namespace {

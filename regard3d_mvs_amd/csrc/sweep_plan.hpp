@@ -1,0 +1,49 @@
+// Launch shape of the row sweeps (k_sweep, kernels_sgm.hip): host arithmetic
+// only, so that it can be checked without a device.
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+
+namespace r3dg {
+
+constexpr int kSweepThreads = 1024;  // a block's threads: the columns and the chunks of a row it takes at once
+constexpr int kSweepRowPad = 8;      // words after an LDS row that a window may read
+
+// Launch shape for tiles of at most max_w columns and max_chunks chunks a row:
+// words of an LDS row, words of a scratch row (0: none needed), the blocks
+// that run at once, the chunks a thread holds.  ok is false where the kernel
+// does not apply.
+struct SweepPlan {
+  bool ok;
+  int wpad, cap, swords, lds_bytes, blocks, held;
+};
+
+// The same on a device of `cus` compute units with `lds` bytes of LDS a block.
+// mean_chunks: of the rows of the tile with most.  A row of k chunks takes
+// words 0 .. 8 k + max_w + 1 (8 per chunk, a sentinel before each pixel and
+// after the last): a scratch row holds all of them, however many (rows of 1024
+// columns have at most 1024 x 250 chunks).
+//
+// Two chunks held per thread, where three paths leave no registers for more or
+// no tile's mean row has more chunks than threads (rows past twice that are
+// rare there, and the sweep of one path is 3 % faster than with four: 2.94 ms
+// against 3.02 for the 1080p pair's aggregation); four for wider rows (the 24 MP
+// pair's: 17.5 ms against 17.7 with two).
+inline SweepPlan size_sweep(int np, int max_w, std::uint32_t max_chunks, std::uint64_t mean_chunks, int cus, int lds) {
+  SweepPlan p{};
+  const std::uint64_t need = 8 * std::uint64_t(max_chunks) + std::uint64_t(std::max(max_w, 0)) + 2;
+  if (max_w > kSweepThreads || need > (std::uint64_t{1} << 30)) return p;
+  const int fixed = 4 * (6 * max_w + 2 * np * max_w + 128 + 4);
+  p.held = np == 3 || mean_chunks <= kSweepThreads ? 2 : 4;
+  p.wpad = max_w;
+  p.cap = std::min({(lds - fixed) / (4 * np) - kSweepRowPad, 8 * kSweepThreads * p.held, static_cast<int>(need)});
+  if (p.cap < 1024) return p;
+  p.lds_bytes = fixed + 4 * np * (p.cap + kSweepRowPad);
+  p.swords = std::uint64_t(p.cap) >= need ? 0 : static_cast<int>(need) + 16;
+  p.blocks = std::max(cus, 1);
+  p.ok = true;
+  return p;
+}
+
+}  // namespace r3dg

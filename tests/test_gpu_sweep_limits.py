@@ -1,0 +1,27 @@
+"""Row sweeps at the limits of their rows (LDS, held chunks, scratch) against
+the CPU oracle.  Integer costs: every output bit-exact.  The launches are
+counted, so that a form of the aggregation that steps in unseen fails."""
+import numpy as np
+import pytest
+
+from regard3d_mvs_amd import StereoOptions
+from test_gpu_parity import _match_both, gpu  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+RAW = dict(speckle_size=0, median=False)
+SCANS = 8  # launches of a level of path scans alone; a level of sweeps takes 3 or 4, full-range scans 1
+
+
+def test_rows_past_a_million_words(gpu):  # noqa: F811
+    """Tiles of up to 736 columns whose pixels mostly hold all 4000 labels (the
+    coarse level finds little in noise, and nothing fills it): rows of up to
+    181754 chunks, past 2^20 words of a scratch row."""
+    rng = np.random.default_rng(59)
+    left = rng.integers(0, 65536, (24, 4700)).astype(np.uint16)
+    right = np.roll(left, -9, 1)
+    right[8:16] = rng.integers(0, 65536, (8, 4700))
+    g, _ = _match_both(gpu, left, right, None, None, -2000, 4000,
+                       StereoOptions(p1=1, p2=2, p2_adapt=0, levels=1, range_radius=0, range_fill=0, uniqueness=0.3,
+                                     tile_size=700, **RAW))
+    assert g.aggregate_launches < 2 * SCANS
