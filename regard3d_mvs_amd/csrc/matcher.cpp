@@ -1046,9 +1046,15 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
 // Consecutive tiles aggregated together, sized to the device memory left in
 // the context's budget (one range when everything fits): at most a twentieth
 // of it in cells where planes or sweep slices are kept, at most a quarter (S,
-// C and room for scratch rows and per-tile data) where only path scans fit;
-// at most 4 G cells, enough to fill the device, so that the volume blocks are
-// reused from range to range rather than freed and mapped again.
+// C and room for scratch rows and per-tile data) for path scans; at most 4 G
+// cells, enough to fill the device, so that the volume blocks are reused from
+// range to range rather than freed and mapped again.
+//
+// Tiles without label ranges that k_full does not take (P2 past a byte, more
+// than 512 labels) go to the path scans: their rows are long and alike, and a
+// sweep's few blocks with scratch rows lose to eight launches that fill the
+// device (640x480 with 1024 labels: 25 ms against 57; with 64 labels and P2 =
+// 300 1.18 against 1.81, 1024x768 with 128 labels 4.5 against 6.1).
 struct TileRange {
   int t0, t1;
   Aggregate kind;
@@ -1057,16 +1063,19 @@ std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
   const std::uint64_t free_bytes = c.arena.budget() > c.arena.live() ? c.arena.budget() - c.arena.live() : 0;
   const bool roomy = A.max_tile_cells <= free_bytes / 20;
   const bool planes = roomy && A.p2max <= kMaxByteP2;
-  const std::uint64_t cap =
-      std::max(A.max_tile_cells, std::min(free_bytes / (roomy ? 20 : 4), std::uint64_t{4} << 30));
   std::vector<TileRange> out;
   const int nt = static_cast<int>(A.td.size());
   std::uint64_t cells = 0;
   for (int t = 0; t < nt; ++t) {
     const auto job = std::size_t(A.td[std::size_t(t)].job);
-    const Aggregate kind = !roomy ? Aggregate::kScan
-                           : planes && A.full[job] > 0 && full_split(A.full[job], 0).lanes > 0 ? Aggregate::kFull
-                                                                                      : Aggregate::kSweep;
+    Aggregate kind = Aggregate::kScan;
+    if (A.full[job] > 0) {
+      if (planes && full_split(A.full[job], 0).lanes > 0) kind = Aggregate::kFull;
+    } else if (roomy) {
+      kind = Aggregate::kSweep;
+    }
+    const std::uint64_t cap = std::max(
+        A.max_tile_cells, std::min(free_bytes / (kind == Aggregate::kScan ? 4 : 20), std::uint64_t{4} << 30));
     const std::uint64_t n = A.tcells[std::size_t(t)];
     if (out.empty() || out.back().kind != kind || cells + n > cap) {
       out.push_back({t, t, kind});

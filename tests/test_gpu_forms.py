@@ -1,0 +1,24 @@
+"""Which form of the aggregation a level takes (full-range scans: one launch;
+row sweeps and horizontal path scans: 3, with both kinds of sweep 4; path
+scans: 8), by the launches counted, and its maps against the CPU oracle.
+Integer costs: every output bit-exact."""
+import numpy as np
+import pytest
+
+from refscenes import Texture, render_pair
+from regard3d_mvs_amd import StereoOptions
+from test_gpu_parity import _match_both, gpu  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+RAW = dict(speckle_size=0, median=False)
+FULL, SWEEPS, SCANS = 1, 3, 8
+
+
+# One full-range level: the last label count and P2 of the full-range scans,
+# and the first ones past them.
+@pytest.mark.parametrize("nd,p2,launches", [(512, 255, FULL), (528, 255, SCANS), (64, 256, SCANS), (1040, 300, SCANS)])
+def test_full_range_form(gpu, nd, p2, launches):  # noqa: F811
+    left, right, _ = render_pair(Texture(61), 83, 41, lambda x, y: 4.0 + 0.1 * x - 0.05 * y)
+    g, _ = _match_both(gpu, left, right, None, None, -5, nd, StereoOptions(levels=0, p2=p2, p2_adapt=0, **RAW))
+    assert g.aggregate_launches == launches
