@@ -130,7 +130,7 @@ void launch_tile_cells(const TileDesc* tiles, int ntiles, const std::uint64_t* r
 constexpr int kLanesPerScan = 8;
 constexpr int kScanPerWave = 64 / kLanesPerScan;
 // Matching costs (u8) of every tile cell into C (same cell indexing as S);
-// cmap receives per chunk of 16 cells its map_entry.
+// cmap receives per chunk of 16 cells its map_entry.  Either may be null.
 void launch_cost(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
                  std::uint64_t total_rows, const std::uint32_t* rowbase, const std::uint64_t* pix, std::uint8_t* C,
                  std::uint32_t* cmap, hipStream_t s);

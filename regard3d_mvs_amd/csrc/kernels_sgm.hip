@@ -359,6 +359,7 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
   const int bfirst = rows[0], blast = rows[1], pfirst = rows[2], plast = rows[3];
   const std::uint32_t invalid = static_cast<std::uint32_t>(J.invalid_cost);
   const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + y];
+  const bool costs = C != nullptr, map = cmap != nullptr;
   std::uint8_t* out = C + row_cell;
   std::uint32_t* mout = cmap + row_cell / kLabelAlign;
   auto partner = [&](int xr) {
@@ -384,8 +385,8 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
       }
       w[q] = v;
     }
-    *reinterpret_cast<uint4*>(out + 16 * std::size_t(k)) = make_uint4(w[0], w[1], w[2], w[3]);
-    mout[k] = map_entry(xa, jb / kLabelAlign);
+    if (costs) *reinterpret_cast<uint4*>(out + 16 * std::size_t(k)) = make_uint4(w[0], w[1], w[2], w[3]);
+    if (map) mout[k] = map_entry(xa, jb / kLabelAlign);
   };
   if (staged) {
     const bool mapped = chunks <= static_cast<std::uint32_t>(kMap);

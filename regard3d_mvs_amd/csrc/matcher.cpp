@@ -527,7 +527,8 @@ struct Chunk {
   // the chunk's first xcells cells; their other paths have planes or slices
   // of their own, xstride apart, in MX or X.
   DBuf<std::uint8_t> C, M, MX;
-  DBuf<std::uint32_t> cmap;  // per chunk of 16 cells its column and place in the pixel
+  DBuf<std::uint32_t> cmap;
+  std::uint32_t* map = nullptr;  // per chunk of 16 cells its column and place in the pixel: cmap, or in C (aggregate_tiles)
   DBuf<std::uint16_t> S, X;
   std::uint64_t stride = 0, xcells = 0, xstride = 0;
   int planes = 0, slices = 0;
@@ -740,9 +741,15 @@ enum class Aggregate { kFull, kSweep, kScan };
 // this: their blocks would leave most of the device idle.
 constexpr int kSweepTiles = 96;
 
+// Device memory that a chunk map has to leave: the rounding of its block.
+constexpr std::uint64_t kMapSlack = std::uint64_t{2} << 20;
+
 // Costs and the 8 paths of tiles [t0, t1) (their rows are consecutive).  With
 // `sum_slices` the slices of side-by-side scans are added into the first.
-Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind, bool sum_slices) {
+// Volumes are sized for `most` cells, those of the level's largest range, so
+// that its ranges take the same blocks one after the other.
+Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind, bool sum_slices,
+                      std::uint64_t most = 0) {
   Chunk ch;
   ch.t0 = t0;
   ch.t1 = t1;
@@ -771,7 +778,8 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     td[std::size_t(t)].cell_base = base;
     base += A.tcells[std::size_t(t0 + t)];
   }
-  ch.stride = (ch.cells + kSPad + 127) / 128 * 128;
+  const std::uint64_t alloc_cells = std::max(ch.cells, most);
+  ch.stride = (alloc_cells + kSPad + 127) / 128 * 128;
   const auto free_bytes = [&] { return c.arena.budget() > c.arena.live() ? c.arena.budget() - c.arena.live() : 0; };
 
   // Sweeps of one path (i = 0) for the first `heavy` tiles in order, of three
@@ -862,8 +870,9 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     dorder = view<std::int32_t>(ch.meta, oo);
     queues = view<std::uint32_t>(ch.meta, oq);
   }
-  ch.C = DBuf<std::uint8_t>(c.arena, ch.cells + kSPad);
-  ch.cmap = DBuf<std::uint32_t>(c.arena, ch.cells / kLabelAlign + 1);
+  // Volumes, the largest first: a smaller one may take a cached block of up to
+  // twice its size, which has to be one that the larger ones leave.
+  //
   // Scratch rows of the path scans' persistent waves (pixels wider than the
   // LDS rows; a multiple of 4: launches use whole blocks of 4 waves, one slot
   // each).
@@ -909,22 +918,31 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     ways = static_cast<int>(std::clamp<std::uint64_t>((resident + mean_groups - 1) / mean_groups, 2, 3));
     const std::uint64_t slice_bytes = (ch.stride + path_scratch_elems(slots, max_num)) * sizeof(std::uint16_t);
     const std::uint64_t room = free_bytes() - std::min(free_bytes(), 2 * ch.stride);
-    while (ways > 1 && std::uint64_t(ways - 1) * slice_bytes > room / 2) --ways;
+    while (ways > 1 && std::uint64_t(ways - 1) * slice_bytes + ch.stride > room / 2) --ways;
     ch.slices = ways;
     ch.S = DBuf<std::uint16_t>(c.arena, std::size_t(ways) * ch.stride);
   }
 
   const std::size_t scratch_elems = npaths > 0 ? path_scratch_elems(slots, max_num) : 0;
   DBuf<std::uint16_t> scratch(c.arena, std::max<std::size_t>(std::size_t(ways) * scratch_elems, 1));
+  ch.C = DBuf<std::uint8_t>(c.arena, alloc_cells + kSPad);
+  // The chunk map (a quarter of the costs' bytes) is read by the sweeps and by
+  // the selection.  Where path scans are left with no memory for it, it takes
+  // the place of the costs after them.  No selection follows with sum_slices.
+  const std::uint64_t map_words = alloc_cells / kLabelAlign + 1;
+  const bool late_map = kind == Aggregate::kScan && !sum_slices && 4 * map_words + kMapSlack > free_bytes();
+  if (!late_map && !sum_slices) ch.cmap = DBuf<std::uint32_t>(c.arena, map_words);
+  ch.map = late_map ? reinterpret_cast<std::uint32_t*>(ch.C.get()) : ch.cmap.get();
 
   // Matching costs of every cell (timed with the other cost preparation).
-  {
+  const auto cost_pass = [&](std::uint8_t* costs, std::uint32_t* map) {
     const StageTimer timer(c, R3DG_STAGE_PREPARE);
-    launch_cost(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), nt, ch.rows, A.rowbase.get(), A.pix.get(),
-                ch.C.get(), ch.cmap.get(), c.stream);
+    launch_cost(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), nt, ch.rows, A.rowbase.get(), A.pix.get(), costs,
+                map, c.stream);
     check_launch();
-  }
-  const StageTimer timer(c, R3DG_STAGE_AGGREGATE);
+  };
+  cost_pass(ch.C.get(), ch.cmap.get());
+  std::optional<StageTimer> timer(std::in_place, c, R3DG_STAGE_AGGREGATE);
   if (full) {
     FullArgs fa{};
     fa.jobs = A.djobs.get();
@@ -967,7 +985,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     sa.units = static_cast<std::uint32_t>(s.units);
     sa.rowbase = A.rowbase.get();
     sa.pix = A.pix.get();
-    sa.cmap = ch.cmap.get();
+    sa.cmap = ch.map;
     sa.C = ch.C.get();
     // Three paths at once: downwards into slice 0, upwards into slice 1.  One
     // path: a plane each, or the slices 0 and 1 and (diagonals) those of X.
@@ -1029,6 +1047,8 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     check_launch();
     ch.slices = 1;
   }
+  timer.reset();
+  if (late_map) cost_pass(nullptr, ch.map);
   c.agg_launches += std::uint64_t(npaths);
   // Per cell the cost bytes read, S written and read back (the first scan of
   // each slice only writes it) and the sweeps' map; per tile pixel and pass
@@ -1046,7 +1066,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
 // Consecutive tiles aggregated together, sized to the device memory left in
 // the context's budget (one range when everything fits): at most a twentieth
 // of it in cells where planes or sweep slices are kept, at most a quarter (S,
-// C and room for scratch rows and per-tile data) for path scans; at most 4 G
+// C, and room for scratch rows and the chunk map) for path scans; at most 4 G
 // cells, enough to fill the device, so that the volume blocks are reused from
 // range to range rather than freed and mapped again.
 //
@@ -1058,6 +1078,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
 struct TileRange {
   int t0, t1;
   Aggregate kind;
+  std::uint64_t cells;
 };
 std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
   const std::uint64_t free_bytes = c.arena.budget() > c.arena.live() ? c.arena.budget() - c.arena.live() : 0;
@@ -1065,7 +1086,6 @@ std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
   const bool planes = roomy && A.p2max <= kMaxByteP2;
   std::vector<TileRange> out;
   const int nt = static_cast<int>(A.td.size());
-  std::uint64_t cells = 0;
   for (int t = 0; t < nt; ++t) {
     const auto job = std::size_t(A.td[std::size_t(t)].job);
     Aggregate kind = Aggregate::kScan;
@@ -1077,11 +1097,8 @@ std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
     const std::uint64_t cap = std::max(
         A.max_tile_cells, std::min(free_bytes / (kind == Aggregate::kScan ? 4 : 20), std::uint64_t{4} << 30));
     const std::uint64_t n = A.tcells[std::size_t(t)];
-    if (out.empty() || out.back().kind != kind || cells + n > cap) {
-      out.push_back({t, t, kind});
-      cells = 0;
-    }
-    cells += n;
+    if (out.empty() || out.back().kind != kind || out.back().cells + n > cap) out.push_back({t, t, kind, 0});
+    out.back().cells += n;
     out.back().t1 = t + 1;
   }
   return out;
@@ -1097,13 +1114,16 @@ std::vector<TilesOut> match_jobs(Context& c, std::vector<Job>& jobs, const r3dg_
   DBuf<float> tdisp(c.arena, std::max<std::uint64_t>(total_px, 1)), tconf(c.arena, std::max<std::uint64_t>(total_px, 1));
   DBuf<std::int16_t> tlab;
   if (any_labels) tlab = DBuf<std::int16_t>(c.arena, std::max<std::uint64_t>(total_px, 1));
-  for (const auto& [t0, t1, kind] : chunk_tiles(c, A)) {
+  const std::vector<TileRange> ranges = chunk_tiles(c, A);
+  for (const TileRange& range : ranges) {
     poll_cancel(c);
-    Chunk ch = aggregate_tiles(c, A, t0, t1, kind, false);
+    std::uint64_t most = 0;
+    for (const TileRange& r : ranges) most = std::max(most, r.kind == range.kind ? r.cells : 0);
+    Chunk ch = aggregate_tiles(c, A, range.t0, range.t1, range.kind, false, most);
     // Selection into per-tile maps.
     const StageTimer timer(c, R3DG_STAGE_SELECT);
-    launch_select(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), t1 - t0, ch.rows, A.rowbase.get(),
-                  A.pix.get(), ch.cmap.get(), ch.source(), sp, A.max_w, A.max_D, tdisp.get(), tconf.get(), tlab.get(), c.stream);
+    launch_select(A.djobs.get(), ch.dtiles.get(), ch.drow_prefix.get(), range.t1 - range.t0, ch.rows, A.rowbase.get(),
+                  A.pix.get(), ch.map, ch.source(), sp, A.max_w, A.max_D, tdisp.get(), tconf.get(), tlab.get(), c.stream);
     check_launch();
   }
   std::vector<TilesOut> out(static_cast<std::size_t>(nj));

@@ -22,3 +22,24 @@ def test_full_range_form(gpu, nd, p2, launches):  # noqa: F811
     left, right, _ = render_pair(Texture(61), 83, 41, lambda x, y: 4.0 + 0.1 * x - 0.05 * y)
     g, _ = _match_both(gpu, left, right, None, None, -5, nd, StereoOptions(levels=0, p2=p2, p2_adapt=0, **RAW))
     assert g.aggregate_launches == launches
+
+
+# Device budgets that hold S and the costs of a range (3 bytes per cell) beside
+# the pair's images and maps and little more: the chunk map takes the costs'
+# place after the path scans, and the blocks of a first, smaller range do not
+# end up under a later one's smaller volumes.
+@pytest.mark.parametrize("w,h,mib", [(1024, 768, 140), (2000, 1500, 315), (2000, 1500, 653)])
+def test_tight_budgets(hip_runtime, gpu, w, h, mib):  # noqa: F811
+    import torch
+    from regard3d_mvs_amd.native import Matcher
+    rng = np.random.default_rng(w)
+    left = rng.integers(0, 65536, (h, w)).astype(np.uint16)
+    images = [torch.from_numpy(a).cuda() for a in (left, np.roll(left, -21, 1))]
+    o = StereoOptions(levels=0, **RAW)
+    ref = gpu.match(*images, dmin=0, nd=128, options=o)
+    with Matcher(0, hbm_budget=mib << 20) as small:
+        for _ in range(3):
+            got = small.match(*images, dmin=0, nd=128, options=o)
+            assert got.aggregate_launches >= 2 * SCANS
+            for k in ("disparity", "confidence"):
+                assert torch.equal(getattr(got, k).view(torch.int32), getattr(ref, k).view(torch.int32))
