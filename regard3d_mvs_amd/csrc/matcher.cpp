@@ -526,24 +526,26 @@ struct Chunk {
   // slices of S, `stride` elements apart.  Tiles aggregated path by path hold
   // the chunk's first xcells cells; their other paths have planes or slices
   // of their own, xstride apart, in MX or X.
-  DBuf<std::uint8_t> C, M, MX;
-  DBuf<std::uint32_t> cmap;
-  std::uint32_t* map = nullptr;  // per chunk of 16 cells its column and place in the pixel: cmap, or in C (aggregate_tiles)
-  DBuf<std::uint16_t> S, X;
+  // All of them, the costs C and the chunk map (per chunk of 16 cells its column
+  // and place in the pixel) lie in one block.
+  DBuf<std::uint8_t> mem;
+  std::uint8_t *C = nullptr, *M = nullptr, *MX = nullptr;
+  std::uint16_t *S = nullptr, *X = nullptr;
+  std::uint32_t* map = nullptr;
   std::uint64_t stride = 0, xcells = 0, xstride = 0;
   int planes = 0, slices = 0;
   SumSrc source() const {
     SumSrc v{};
-    for (v.n = 0; v.n < slices; ++v.n) v.p[v.n] = S.get() + std::uint64_t(v.n) * stride;
+    for (v.n = 0; v.n < slices; ++v.n) v.p[v.n] = S + std::uint64_t(v.n) * stride;
     v.xcells = xcells;
     if (planes > 0) {
-      v.m = M.get();
+      v.m = M;
       v.mstride = stride;
-      v.mx = planes == kPaths ? M.get() + 2 * stride : MX.get();
+      v.mx = planes == kPaths ? M + 2 * stride : MX;
       v.mxstride = planes == kPaths ? stride : xstride;
-      v.c = C.get();
+      v.c = C;
     } else if (xcells > 0) {
-      for (int k = slices; k < kPaths; ++k) v.p[k] = X.get() + std::uint64_t(k - slices) * xstride;
+      for (int k = slices; k < kPaths; ++k) v.p[k] = X + std::uint64_t(k - slices) * xstride;
     }
     return v;
   }
@@ -741,8 +743,8 @@ enum class Aggregate { kFull, kSweep, kScan };
 // this: their blocks would leave most of the device idle.
 constexpr int kSweepTiles = 96;
 
-// Device memory that a chunk map has to leave: the rounding of its block.
-constexpr std::uint64_t kMapSlack = std::uint64_t{2} << 20;
+// Rounding of a chunk's block of volumes.
+constexpr std::uint64_t kBlockSlack = std::uint64_t{2} << 20;
 
 // Costs and the 8 paths of tiles [t0, t1) (their rows are consecutive).  With
 // `sum_slices` the slices of side-by-side scans are added into the first.
@@ -778,8 +780,6 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     td[std::size_t(t)].cell_base = base;
     base += A.tcells[std::size_t(t0 + t)];
   }
-  const std::uint64_t alloc_cells = std::max(ch.cells, most);
-  ch.stride = (alloc_cells + kSPad + 127) / 128 * 128;
   const auto free_bytes = [&] { return c.arena.budget() > c.arena.live() ? c.arena.budget() - c.arena.live() : 0; };
 
   // Sweeps of one path (i = 0) for the first `heavy` tiles in order, of three
@@ -791,7 +791,6 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   struct Sweep {
     SweepPlan plan;
     std::uint64_t units, blocks, block_words;
-    DBuf<std::uint32_t> scratch;
   };
   std::array<Sweep, 2> sw{};
   int heavy = 0;
@@ -870,14 +869,31 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     dorder = view<std::int32_t>(ch.meta, oo);
     queues = view<std::uint32_t>(ch.meta, oq);
   }
-  // Volumes, the largest first: a smaller one may take a cached block of up to
-  // twice its size, which has to be one that the larger ones leave.
-  //
+  // Volumes and scratch rows, laid out in one block: of several, a smaller one
+  // might take a cached block of up to twice its size, and then a larger one
+  // find no room.  A small last range of path scans takes more slices instead
+  // of larger ones.
+  std::uint64_t block = 0;
+  const auto take = [&](std::uint64_t bytes) {
+    const std::uint64_t at = block;
+    block += (bytes + 255) / 256 * 256;
+    return at;
+  };
+  const std::uint64_t alloc_cells = std::max(ch.cells, most);
+  const auto strided = [](std::uint64_t cells) { return (cells + kSPad + 127) / 128 * 128; };
+  ch.stride = strided(kind == Aggregate::kScan ? ch.cells : alloc_cells);
   // Scratch rows of the path scans' persistent waves (pixels wider than the
   // LDS rows; a multiple of 4: launches use whole blocks of 4 waves, one slot
-  // each).
+  // each).  Where S and the costs leave no room for the rows of all waves, as
+  // many scan at once as half of what is left holds rows for.
   const std::uint64_t resident = path_slots();
-  const std::uint64_t slots = (std::min(resident, std::max<std::uint64_t>(max_groups, 1)) + 3) / 4 * 4;
+  std::uint64_t slots = (std::min(resident, std::max<std::uint64_t>(max_groups, 1)) + 3) / 4 * 4;
+  if (kind == Aggregate::kScan) {
+    const std::uint64_t volumes = 3 * strided(alloc_cells) + kBlockSlack;
+    const std::uint64_t left = free_bytes() - std::min(free_bytes(), volumes);
+    const std::uint64_t fit = left / 2 / (4 * sizeof(std::uint16_t) * path_scratch_elems(1, max_num)) * 4;
+    slots = std::min(slots, std::max<std::uint64_t>(fit, 4));
+  }
   // Streams of the path scans.  Alone they run side by side on 2 or 3 streams
   // (3 where their groups average less than the device holds), each stream
   // summing its paths into a slice of its own, when the slices and their
@@ -888,31 +904,35 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   // with 3).  Beside the sweeps the two horizontal scans take a stream each,
   // one between them beside two sweep launches.
   int ways = 0;
+  std::uint64_t at_m = 0, at_mx = 0, at_s = 0, at_x = 0;
+  std::array<std::uint64_t, 2> at_sweep{};
   if (full) {
     ch.planes = kPaths;
-    ch.M = DBuf<std::uint8_t>(c.arena, kPaths * ch.stride);
+    at_m = take(kPaths * ch.stride);
     ch.xcells = ch.cells;
   } else if (sweep) {
     ways = heavy == 0 || heavy == nt ? 2 : 1;
     if (heavy > 0) {
       ch.xcells = heavy < nt ? td[std::size_t(order[std::size_t(heavy)])].cell_base : ch.cells;
-      ch.xstride = (ch.xcells + kSPad + 127) / 128 * 128;
+      ch.xstride = strided(ch.xcells);
     }
     if (bytes) {
       ch.planes = 2;
-      ch.M = DBuf<std::uint8_t>(c.arena, 2 * ch.stride);
-      if (heavy > 0) ch.MX = DBuf<std::uint8_t>(c.arena, std::size_t(kPaths - 2) * ch.xstride);
+      at_m = take(2 * ch.stride);
+      if (heavy > 0) at_mx = take(std::uint64_t(kPaths - 2) * ch.xstride);
       if (heavy < nt) {
         ch.slices = 2;
-        ch.S = DBuf<std::uint16_t>(c.arena, 2 * ch.stride);
+        at_s = take(2 * ch.stride * sizeof(std::uint16_t));
       }
     } else {
       ch.slices = 4;
-      ch.S = DBuf<std::uint16_t>(c.arena, 4 * ch.stride);
-      if (heavy > 0) ch.X = DBuf<std::uint16_t>(c.arena, std::size_t(kPaths - 4) * ch.xstride);
+      at_s = take(4 * ch.stride * sizeof(std::uint16_t));
+      if (heavy > 0) at_x = take(std::uint64_t(kPaths - 4) * ch.xstride * sizeof(std::uint16_t));
     }
-    for (Sweep& s : sw)
-      if (s.units > 0 && s.block_words > 0) s.scratch = DBuf<std::uint32_t>(c.arena, s.blocks * s.block_words);
+    for (int i = 0; i < 2; ++i) {
+      const Sweep& s = sw[std::size_t(i)];
+      if (s.units > 0) at_sweep[std::size_t(i)] = take(s.blocks * s.block_words * sizeof(std::uint32_t));
+    }
   } else {
     const std::uint64_t mean_groups = std::max<std::uint64_t>((sum_groups + 7) / 8, 1);
     ways = static_cast<int>(std::clamp<std::uint64_t>((resident + mean_groups - 1) / mean_groups, 2, 3));
@@ -920,19 +940,26 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     const std::uint64_t room = free_bytes() - std::min(free_bytes(), 2 * ch.stride);
     while (ways > 1 && std::uint64_t(ways - 1) * slice_bytes + ch.stride > room / 2) --ways;
     ch.slices = ways;
-    ch.S = DBuf<std::uint16_t>(c.arena, std::size_t(ways) * ch.stride);
+    at_s = take(std::max(std::uint64_t(ways) * ch.stride, strided(alloc_cells)) * sizeof(std::uint16_t));
   }
 
-  const std::size_t scratch_elems = npaths > 0 ? path_scratch_elems(slots, max_num) : 0;
-  DBuf<std::uint16_t> scratch(c.arena, std::max<std::size_t>(std::size_t(ways) * scratch_elems, 1));
-  ch.C = DBuf<std::uint8_t>(c.arena, alloc_cells + kSPad);
+  const std::uint64_t scratch_elems = npaths > 0 ? path_scratch_elems(slots, max_num) : 0;
+  const std::uint64_t at_scratch = take(std::uint64_t(ways) * scratch_elems * sizeof(std::uint16_t));
+  const std::uint64_t at_c = take(alloc_cells + kSPad);
   // The chunk map (a quarter of the costs' bytes) is read by the sweeps and by
   // the selection.  Where path scans are left with no memory for it, it takes
   // the place of the costs after them.  No selection follows with sum_slices.
-  const std::uint64_t map_words = alloc_cells / kLabelAlign + 1;
-  const bool late_map = kind == Aggregate::kScan && !sum_slices && 4 * map_words + kMapSlack > free_bytes();
-  if (!late_map && !sum_slices) ch.cmap = DBuf<std::uint32_t>(c.arena, map_words);
-  ch.map = late_map ? reinterpret_cast<std::uint32_t*>(ch.C.get()) : ch.cmap.get();
+  const std::uint64_t map_bytes = (alloc_cells / kLabelAlign + 1) * sizeof(std::uint32_t);
+  const bool late_map = kind == Aggregate::kScan && !sum_slices && block + map_bytes + kBlockSlack > free_bytes();
+  const std::uint64_t at_map = late_map ? at_c : take(sum_slices ? 0 : map_bytes);
+  ch.mem = DBuf<std::uint8_t>(c.arena, block);
+  ch.C = ch.mem.get() + at_c;
+  ch.M = ch.mem.get() + at_m;
+  ch.MX = ch.mem.get() + at_mx;
+  ch.S = reinterpret_cast<std::uint16_t*>(ch.mem.get() + at_s);
+  ch.X = reinterpret_cast<std::uint16_t*>(ch.mem.get() + at_x);
+  ch.map = sum_slices ? nullptr : reinterpret_cast<std::uint32_t*>(ch.mem.get() + at_map);
+  std::uint16_t* const scratch = reinterpret_cast<std::uint16_t*>(ch.mem.get() + at_scratch);
 
   // Matching costs of every cell (timed with the other cost preparation).
   const auto cost_pass = [&](std::uint8_t* costs, std::uint32_t* map) {
@@ -941,7 +968,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
                 map, c.stream);
     check_launch();
   };
-  cost_pass(ch.C.get(), ch.cmap.get());
+  cost_pass(ch.C, late_map ? nullptr : ch.map);
   std::optional<StageTimer> timer(std::in_place, c, R3DG_STAGE_AGGREGATE);
   if (full) {
     FullArgs fa{};
@@ -950,8 +977,8 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     fa.gprefix = dfp.get();
     fa.ntiles = nt;
     fa.groups = fp.back();
-    fa.C = ch.C.get();
-    fa.M = ch.M.get();
+    fa.C = ch.C;
+    fa.M = ch.M;
     fa.mstride = ch.stride;
     launch_full(fa, split, c.stream);
     check_launch();
@@ -986,18 +1013,18 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     sa.rowbase = A.rowbase.get();
     sa.pix = A.pix.get();
     sa.cmap = ch.map;
-    sa.C = ch.C.get();
+    sa.C = ch.C;
     // Three paths at once: downwards into slice 0, upwards into slice 1.  One
     // path: a plane each, or the slices 0 and 1 and (diagonals) those of X.
     for (int u = 0; u < 6; ++u) {
       if (i == 0 && bytes) {
-        sa.out[u] = ch.MX.get() + std::uint64_t(u) * ch.xstride;
+        sa.out[u] = ch.MX + std::uint64_t(u) * ch.xstride;
       } else {
-        sa.out[u] = u < 2 ? ch.S.get() + std::uint64_t(u) * ch.stride
-                          : ch.X.get() + std::uint64_t(u - 2) * ch.xstride;
+        sa.out[u] = u < 2 ? ch.S + std::uint64_t(u) * ch.stride
+                          : ch.X + std::uint64_t(u - 2) * ch.xstride;
       }
     }
-    sa.scratch = s.scratch.get();
+    sa.scratch = reinterpret_cast<std::uint32_t*>(ch.mem.get() + at_sweep[std::size_t(i)]);
     sa.queue = queues.get() + kPaths + i;
     sa.wpad = s.plan.wpad;
     sa.cap = s.plan.cap;
@@ -1012,7 +1039,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   pa.ntiles = nt;
   pa.rowbase = A.rowbase.get();
   pa.pix = A.pix.get();
-  pa.C = ch.C.get();
+  pa.C = ch.C;
   pa.slots = slots;
   pa.max_num = max_num;
   for (int p = 0; p < npaths; ++p) {
@@ -1020,18 +1047,18 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
     const std::size_t o8 = std::size_t(p) * (std::size_t(nt) + 1);
     pa.gprefix = dgp.get() + o8;
     pa.groups = gp[o8 + std::size_t(nt)];
-    pa.scratch = scratch.get() + std::size_t(w) * scratch_elems;
+    pa.scratch = scratch + std::size_t(w) * scratch_elems;
     pa.queue = queues.get() + p;
     int mode = kFirstSum;
     if (bytes) {
       mode = kByteM;
-      pa.out = ch.M.get() + std::uint64_t(p) * ch.stride;
+      pa.out = ch.M + std::uint64_t(p) * ch.stride;
     } else if (sweep) {
-      pa.out = ch.S.get() + std::uint64_t(2 + p) * ch.stride;
+      pa.out = ch.S + std::uint64_t(2 + p) * ch.stride;
     } else {
       // Path p adds into its stream's slice.
       mode = p >= ways ? kAddSum : kFirstSum;
-      pa.out = ch.S.get() + std::uint64_t(w) * ch.stride;
+      pa.out = ch.S + std::uint64_t(w) * ch.stride;
     }
     launch_sgm_path(p, pa, mode, st[std::size_t(sweep ? w + 1 : w)]);
     check_launch();
@@ -1043,7 +1070,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   }
   for (int w = 0; w <= side && side > 0; ++w) c.event_pool.push_back(ev[std::size_t(w)]);
   if (sum_slices && ch.slices > 1) {
-    launch_sum_u16(ch.S.get(), ch.source(), ch.cells, c.stream);
+    launch_sum_u16(ch.S, ch.source(), ch.cells, c.stream);
     check_launch();
     ch.slices = 1;
   }
@@ -3058,7 +3085,7 @@ int32_t r3dg_cost_volume(r3dg_ctx* h, r3dg_image left, r3dg_image right, int32_t
     if (A.total_cells != out_cells) fail(R3DG_ERROR_INTERNAL, "cost_volume: cell count mismatch");
     const Chunk ch = aggregate_tiles(c, A, 0, static_cast<int>(A.td.size()), Aggregate::kScan, true);
     const hipMemcpyKind kind = out_memory == R3DG_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-    if (out_cells > 0) hip_check(hipMemcpyAsync(out, ch.S.get(), out_cells * 2, kind, c.stream), "download");
+    if (out_cells > 0) hip_check(hipMemcpyAsync(out, ch.S, out_cells * 2, kind, c.stream), "download");
     sync(c);
   });
 }

@@ -6,8 +6,8 @@ import numpy as np
 import pytest
 
 from refscenes import Texture, render_pair
-from regard3d_mvs_amd import StereoOptions
-from test_gpu_parity import _match_both, gpu  # noqa: F401
+from regard3d_mvs_amd import StereoOptions, synth
+from test_gpu_parity import _match_both, gpu, same_bits  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -26,9 +26,9 @@ def test_full_range_form(gpu, nd, p2, launches):  # noqa: F811
 
 # Device budgets that hold S and the costs of a range (3 bytes per cell) beside
 # the pair's images and maps and little more: the chunk map takes the costs'
-# place after the path scans, and the blocks of a first, smaller range do not
-# end up under a later one's smaller volumes.
-@pytest.mark.parametrize("w,h,mib", [(1024, 768, 140), (2000, 1500, 315), (2000, 1500, 653)])
+# place after the path scans, few waves scan at once, and cached blocks of other
+# ranges do not end up under smaller volumes.
+@pytest.mark.parametrize("w,h,mib", [(1024, 768, 137), (2000, 1500, 303), (2000, 1500, 653)])
 def test_tight_budgets(hip_runtime, gpu, w, h, mib):  # noqa: F811
     import torch
     from regard3d_mvs_amd.native import Matcher
@@ -43,3 +43,17 @@ def test_tight_budgets(hip_runtime, gpu, w, h, mib):  # noqa: F811
             assert got.aggregate_launches >= 2 * SCANS
             for k in ("disparity", "confidence"):
                 assert torch.equal(getattr(got, k).view(torch.int32), getattr(ref, k).view(torch.int32))
+
+
+def test_tight_budget_hierarchy(hip_runtime, gpu):  # noqa: F811
+    """The same with label ranges: ranges of few tiles, of sizes that differ
+    from level to level."""
+    from regard3d_mvs_amd.native import Matcher
+    p = synth.make_pair(800, 600, 128, 5)
+    ref = gpu.match(p.left, p.right, dmin=0, nd=128)
+    for mib in (60, 75, 106):
+        with Matcher(0, hbm_budget=mib << 20) as small:
+            for _ in range(2):
+                got = small.match(p.left, p.right, dmin=0, nd=128)
+                same_bits(got.disparity, ref.disparity)
+                same_bits(got.confidence, ref.confidence)
