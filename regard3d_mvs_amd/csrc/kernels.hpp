@@ -202,7 +202,8 @@ struct SweepArgs {
   std::uint32_t* queue;
   int wpad, cap, swords;         // SweepPlan
 };
-// size_sweep for the current device.
+// Compute units of the current device, and size_sweep for it.
+int compute_units();
 SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks, std::uint64_t mean_chunks);
 void launch_sweep(const SweepArgs& a, int np, bool bytes, const SweepPlan& p, std::uint64_t blocks, hipStream_t s);
 // Extra elements S, C and a plane hold past their last cell.

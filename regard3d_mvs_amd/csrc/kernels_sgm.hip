@@ -1921,12 +1921,18 @@ void launch_full(const FullArgs& a, FullSplit f, hipStream_t s) {
   }
 }
 
-SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks, std::uint64_t mean_chunks) {
-  int dev = 0, cus = 0, lds = 0;
+int compute_units() {
+  int dev = 0, cus = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  return cus;
+}
+
+SweepPlan sweep_plan(int np, int max_w, std::uint32_t max_chunks, std::uint64_t mean_chunks) {
+  int dev = 0, lds = 0;
+  (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-  return size_sweep(np, max_w, max_chunks, mean_chunks, cus, lds);
+  return size_sweep(np, max_w, max_chunks, mean_chunks, compute_units(), lds);
 }
 
 namespace {

@@ -1109,20 +1109,28 @@ struct TileRange {
 };
 std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
   const std::uint64_t free_bytes = c.arena.budget() > c.arena.live() ? c.arena.budget() - c.arena.live() : 0;
-  const bool roomy = A.max_tile_cells <= free_bytes / 20;
-  const bool planes = roomy && A.p2max <= kMaxByteP2;
+  const std::uint64_t most = std::uint64_t{4} << 30, room = std::min(free_bytes / 20, most);
+  const bool roomy = A.max_tile_cells <= room;
+  const bool bytes = A.p2max <= kMaxByteP2, planes = roomy && bytes;
   std::vector<TileRange> out;
   const int nt = static_cast<int>(A.td.size());
+  std::uint64_t ranged = 0, ranged_cells = 0;  // tiles with label ranges
+  for (int t = 0; t < nt; ++t) {
+    if (A.full[std::size_t(A.td[std::size_t(t)].job)] > 0) continue;
+    ++ranged;
+    ranged_cells += A.tcells[std::size_t(t)];
+  }
+  const bool sweeps =
+      roomy && A.max_w <= kSweepThreads && sweeps_fit(ranged, ranged_cells, room, bytes, compute_units());
   for (int t = 0; t < nt; ++t) {
     const auto job = std::size_t(A.td[std::size_t(t)].job);
     Aggregate kind = Aggregate::kScan;
     if (A.full[job] > 0) {
       if (planes && full_split(A.full[job], 0).lanes > 0) kind = Aggregate::kFull;
-    } else if (roomy) {
+    } else if (sweeps) {
       kind = Aggregate::kSweep;
     }
-    const std::uint64_t cap = std::max(
-        A.max_tile_cells, std::min(free_bytes / (kind == Aggregate::kScan ? 4 : 20), std::uint64_t{4} << 30));
+    const std::uint64_t cap = kind == Aggregate::kScan ? std::max(A.max_tile_cells, std::min(free_bytes / 4, most)) : room;
     const std::uint64_t n = A.tcells[std::size_t(t)];
     if (out.empty() || out.back().kind != kind || out.back().cells + n > cap) out.push_back({t, t, kind, 0});
     out.back().cells += n;

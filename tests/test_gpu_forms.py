@@ -57,3 +57,31 @@ def test_tight_budget_hierarchy(hip_runtime, gpu):  # noqa: F811
                 got = small.match(p.left, p.right, dmin=0, nd=128)
                 same_bits(got.disparity, ref.disparity)
                 same_bits(got.confidence, ref.confidence)
+
+
+# Two levels: sweeps take the fine one from three tiles on (one and its mirror
+# leave most of the device idle), with uint16 slices from six, and none wider
+# than their 1024 columns.
+@pytest.mark.parametrize("w,h,tile,p2,fine", [(150, 90, 512, 200, SCANS), (150, 90, 80, 200, SWEEPS),
+                                              (150, 90, 80, 300, SWEEPS), (150, 70, 80, 300, SCANS),
+                                              (1040, 30, 2048, 200, SCANS)])
+def test_ranged_form(gpu, w, h, tile, p2, fine):  # noqa: F811
+    p = synth.make_pair(w, h, 32, 11)
+    g, _ = _match_both(gpu, p.left, p.right, None, None, 0, 32,
+                       StereoOptions(levels=1, p2=p2, p2_adapt=0, tile_size=tile, tile_margin=4, tile_blend=4))
+    assert g.aggregate_launches == (FULL if p2 <= 255 else SCANS) + fine
+
+
+def test_cut_levels_by_path_scans(hip_runtime, gpu):  # noqa: F811
+    """A budget that cuts the fine level into ranges of few tiles: path scans,
+    in ranges of five times the cells that sweeps would take."""
+    from regard3d_mvs_amd.native import Matcher
+    p = synth.make_pair(1280, 960, 96, 5)
+    o = StereoOptions(levels=1)
+    ref = gpu.match(p.left, p.right, dmin=0, nd=96, options=o)
+    assert ref.aggregate_launches == FULL + SWEEPS
+    with Matcher(0, hbm_budget=600 << 20) as small:
+        got = small.match(p.left, p.right, dmin=0, nd=96, options=o)
+    assert got.aggregate_launches in (FULL + SCANS, 2 * FULL + SCANS)  # the coarse level may be cut in two
+    same_bits(got.disparity, ref.disparity)
+    same_bits(got.confidence, ref.confidence)
