@@ -182,6 +182,12 @@ struct FullSplit {
   int labels, lanes;
 };
 FullSplit full_split(int D, std::uint64_t scanlines);
+// k_full addresses a tile's intensities by 32-bit byte offsets from its first
+// row: whether those of h rows of an image of this stride (elements) fit.
+constexpr bool full_offsets_fit(int h, std::int64_t img_stride) {
+  return img_stride < (std::int64_t{1} << 31) / (h > 0 ? h : 1);
+}
+static_assert(full_offsets_fit(64, (1 << 25) - 1) && !full_offsets_fit(64, 1 << 25), "2^31 elements are 2^32 bytes");
 void launch_full(const FullArgs& a, FullSplit f, hipStream_t s);
 // The vertical and diagonal paths (2 .. 7) of tiles of at most 1024 columns,
 // row by row: np = 3 takes the three paths downwards (upwards) of a tile at

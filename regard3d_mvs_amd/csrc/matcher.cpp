@@ -512,6 +512,7 @@ struct Aggregation {
   std::uint32_t max_row_chunks = 1;
   int p2max = 0;
   std::vector<int> full;  // per job: its labels if every pixel has all of them, else 0
+  std::vector<std::int64_t> img_stride;  // per job
 };
 
 // Aggregated volume S of tiles [t0, t1) of a layout; the chunk's tile
@@ -556,7 +557,10 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
   const int nj = static_cast<int>(jobs.size());
   const auto lut = p2_table(o);
   A.p2max = *std::max_element(lut.begin(), lut.end());
-  for (const Job& J : jobs) A.full.push_back(J.ranges == nullptr ? J.D : 0);
+  for (const Job& J : jobs) {
+    A.full.push_back(J.ranges == nullptr ? J.D : 0);
+    A.img_stride.push_back(J.base->s);
+  }
   std::vector<JobDesc> jd(static_cast<std::size_t>(nj));
   for (int j = 0; j < nj; ++j) {
     const Job& J = jobs[std::size_t(j)];
@@ -1098,7 +1102,7 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
 // range to range rather than freed and mapped again.
 //
 // Tiles without label ranges that k_full does not take (P2 past a byte, more
-// than 512 labels) go to the path scans: their rows are long and alike, and a
+// than 512 labels, views whose rows lie too far apart) go to the path scans: their rows are long and alike, and a
 // sweep's few blocks with scratch rows lose to eight launches that fill the
 // device (640x480 with 1024 labels: 25 ms against 57; with 64 labels and P2 =
 // 300 1.18 against 1.81, 1024x768 with 128 labels 4.5 against 6.1).
@@ -1126,7 +1130,8 @@ std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
     const auto job = std::size_t(A.td[std::size_t(t)].job);
     Aggregate kind = Aggregate::kScan;
     if (A.full[job] > 0) {
-      if (planes && full_split(A.full[job], 0).lanes > 0) kind = Aggregate::kFull;
+      if (planes && full_split(A.full[job], 0).lanes > 0 && full_offsets_fit(A.td[std::size_t(t)].h, A.img_stride[job]))
+        kind = Aggregate::kFull;
     } else if (sweeps) {
       kind = Aggregate::kSweep;
     }

@@ -85,3 +85,24 @@ def test_cut_levels_by_path_scans(hip_runtime, gpu):  # noqa: F811
     assert got.aggregate_launches in (FULL + SCANS, 2 * FULL + SCANS)  # the coarse level may be cut in two
     same_bits(got.disparity, ref.disparity)
     same_bits(got.confidence, ref.confidence)
+
+
+def test_rows_far_apart(hip_runtime, gpu):  # noqa: F811
+    """Device views whose rows lie 80 MB apart: 70 of them span more than 32
+    bits of offsets, which full-range scans do not hold."""
+    import torch
+    rng = np.random.default_rng(67)
+    left = rng.integers(0, 65536, (70, 90)).astype(np.uint16)
+    right = np.roll(left, -7, 1)
+    o = StereoOptions(levels=0, **RAW)
+    ref = gpu.match(left, right, dmin=0, nd=32, options=o)
+    base = torch.empty((70, 40_000_000), dtype=torch.uint16, device="cuda")
+    views = []
+    for k, a in enumerate((left, right)):
+        v = base[:, 1000 * k:1000 * k + 90]
+        v.copy_(torch.from_numpy(a).cuda())
+        views.append(v)
+    got = gpu.match(*views, dmin=0, nd=32, options=o)
+    assert (ref.aggregate_launches, got.aggregate_launches) == (FULL, SCANS)
+    same_bits(got.disparity.cpu().numpy(), ref.disparity)
+    same_bits(got.confidence.cpu().numpy(), ref.confidence)
