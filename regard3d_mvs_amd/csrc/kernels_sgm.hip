@@ -1088,9 +1088,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
   constexpr int N = 8;
   In in[N];
 #pragma unroll
-  for (int j = 0; j < N - 1; ++j) {
-    in[j] = In{};
-    if (j < steps) load(in[j]);
+  for (int j = 0; j < N; ++j) {
+    in[j] = In{};  // all N: a scanline of N - 1 steps reads the one that none of its loads fills
+    if (j < N - 1 && j < steps) load(in[j]);
   }
   int i = 0;
   for (; i + 2 * N - 1 <= steps; i += N) {

@@ -106,3 +106,16 @@ def test_rows_far_apart(hip_runtime, gpu):  # noqa: F811
     assert (ref.aggregate_launches, got.aggregate_launches) == (FULL, SCANS)
     same_bits(got.disparity.cpu().numpy(), ref.disparity)
     same_bits(got.confidence.cpu().numpy(), ref.confidence)
+
+
+# Scanlines about the length of the sets of loads that a full-range scan keeps
+# in flight (eight), and twice that.
+@pytest.mark.parametrize("short", [6, 7, 8, 9, 14, 15, 16])
+@pytest.mark.parametrize("across", [False, True])
+def test_full_range_short_scanlines(gpu, short, across):  # noqa: F811
+    rng = np.random.default_rng(short)
+    shape = (37, short) if across else (short, 37)
+    left = rng.integers(0, 65536, shape).astype(np.uint16)
+    right = rng.integers(0, 65536, shape).astype(np.uint16)
+    g, _ = _match_both(gpu, left, right, None, None, -8, 32, StereoOptions(levels=0, **RAW))
+    assert g.aggregate_launches == FULL
