@@ -115,13 +115,13 @@ void launch_ranges_from_coarse(const float* coarse, int wc, int hc, int width, i
                                std::uint16_t* lo, std::uint16_t* num, std::int64_t rs, hipStream_t s);
 
 // ---- aggregation (kernels_sgm.hip)
-// Cells of every tile row (row_cells[row_base + y]), its largest label count
-// (row_max) and the pixel records.
+// Cells of every strip of every tile row (row_cells[row_base + y * strips + s]),
+// its largest label count (row_max) and the pixel records.
 void launch_tile_row_scan(const JobDesc* jobs, const TileDesc* tiles, const std::uint64_t* row_prefix, int ntiles,
                           std::uint64_t total_rows, std::uint64_t* pix, std::uint64_t* row_cells,
                           std::uint32_t* row_max, hipStream_t s);
-// First cell of every tile row in its tile's volume (rowbase[row_base + y]);
-// per tile its cells, its largest label count and the most chunks in a row.
+// First cell of every strip in its tile's volume (rowbase, as row_cells); per
+// tile its cells, its largest label count and the most chunks in a strip.
 void launch_tile_cells(const TileDesc* tiles, int ntiles, const std::uint64_t* row_cells, const std::uint32_t* row_max,
                        std::uint32_t* rowbase, std::uint64_t* tile_cells, std::uint32_t* tile_max,
                        std::uint32_t* tile_row, hipStream_t s);

@@ -157,7 +157,21 @@ __global__ __launch_bounds__(256) void k_tile_row_scan(const JobDesc* __restrict
   std::uint64_t* prow = pix + T.px_base + std::uint64_t(y) * T.w;
   std::uint64_t carry = 0;
   std::uint32_t vmax = 0;
+  std::uint64_t strip = T.row_base + std::uint64_t(y) * static_cast<std::uint32_t>(T.strips);
+  // Cells and largest label count (of the row so far) of the strip that ends.
+  auto end_strip = [&] {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) vmax = max(vmax, static_cast<std::uint32_t>(__shfl_xor(vmax, d)));
+    if (lane == 0) {
+      row_cells[strip] = carry;
+      row_max[strip] = vmax;
+    }
+    ++strip;
+    carry = 0;
+  };
+  static_assert((1 << kStripShift) % (64 * kItems) == 0, "strips end where a pass does");
   for (int base = 0; base < T.w; base += 64 * kItems) {
+    if (base > 0 && (base & ((1 << kStripShift) - 1)) == 0) end_strip();
     int lo[kItems], num[kItems], val[kItems];
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
@@ -185,16 +199,11 @@ __global__ __launch_bounds__(256) void k_tile_row_scan(const JobDesc* __restrict
       vmax = max(vmax, v);
     }
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) vmax = max(vmax, static_cast<std::uint32_t>(__shfl_xor(vmax, d)));
-  if (lane == 0) {
-    row_cells[T.row_base + y] = carry;
-    row_max[T.row_base + y] = vmax;
-  }
+  end_strip();
 }
 
-// Totals of one tile (cells, largest label count, most chunks in a row) and
-// the first cell of each of its rows: an exclusive scan of the row counts.
+// Totals of one tile (cells, largest label count, most chunks in a strip) and
+// the first cell of each of its strips: an exclusive scan of their counts.
 constexpr int kCellsThreads = 1024;  // k_tile_cells: one block of 16 waves per tile
 __global__ __launch_bounds__(kCellsThreads) void k_tile_cells(const TileDesc* __restrict__ tiles,
                                                     const std::uint64_t* __restrict__ row_cells,
@@ -212,17 +221,18 @@ __global__ __launch_bounds__(kCellsThreads) void k_tile_cells(const TileDesc* __
   }
   __syncthreads();
   std::uint64_t carry = 0;
-  for (int base = 0; base < T.h; base += kCellsThreads) {
+  const int strips = T.h * T.strips;
+  for (int base = 0; base < strips; base += kCellsThreads) {
     const int y = base + static_cast<int>(threadIdx.x);
     std::uint64_t v = 0;
-    if (y < T.h) {
+    if (y < strips) {
       v = row_cells[T.row_base + y];
       atomicMax(&smax, row_max[T.row_base + y]);
       atomicMax(&srow, static_cast<std::uint32_t>(min(v / kLabelAlign, std::uint64_t{0xFFFFFFFFU})));
     }
     std::uint64_t total;
     const std::uint64_t before = carry + block_scan_incl<kCellsThreads / 64>(v, wsum, total) - v;
-    if (y < T.h) rowbase[T.row_base + y] = static_cast<std::uint32_t>(before);
+    if (y < strips) rowbase[T.row_base + y] = static_cast<std::uint32_t>(before);
     carry += total;
   }
   if (threadIdx.x == 0) {
@@ -312,7 +322,8 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
   const int c0 = max(0, T.x0 - J.dmin - (J.D - 1)), c1 = min(pw1, T.x0 + T.w - 1 - J.dmin);
   const bool windowed = c1 >= c0 && c1 - c0 < kWin;
   const bool staged = T.w <= kPx;
-  const std::uint64_t last = rec[T.w - 1];
+  constexpr int kStrip = 1 << kStripShift;
+  const std::uint64_t last = rec[min(T.w, kStrip) - 1];  // of the first strip: the only one where staged
   // Staging: every global load of a thread is issued before the first LDS
   // store, so that the block waits for one memory latency, not one per
   // element (the launch has kCostThreads threads).
@@ -355,17 +366,19 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
     }
   }
   __syncthreads();
-  const std::uint32_t chunks = (pix_off(last) + static_cast<std::uint32_t>(pix_num(last))) >> 4;
+  auto chunks_to = [](std::uint64_t r) { return (pix_off(r) + static_cast<std::uint32_t>(pix_num(r))) >> 4; };
   const int bfirst = rows[0], blast = rows[1], pfirst = rows[2], plast = rows[3];
   const std::uint32_t invalid = static_cast<std::uint32_t>(J.invalid_cost);
-  const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + y];
+  const std::uint32_t* strip_base = rowbase + T.row_base + std::uint64_t(y) * T.strips;
   const bool costs = C != nullptr, map = cmap != nullptr;
-  std::uint8_t* out = C + row_cell;
-  std::uint32_t* mout = cmap + row_cell / kLabelAlign;
+  // Output of the strip in hand.
+  std::uint64_t strip_cell = T.cell_base + strip_base[0];
+  std::uint8_t* out = C + strip_cell;
+  std::uint32_t* mout = cmap + strip_cell / kLabelAlign;
   auto partner = [&](int xr) {
     return windowed ? swin[min(max(xr, c0), c1) - c0] : cr[pcol(min(max(xr, 0), pw1))];
   };
-  // Costs of chunk k of pixel xa (first cell off, first label lo, Census c).
+  // Costs of the strip's chunk k, of pixel xa (first cell off, first label lo, Census c).
   auto chunk = [&](std::uint32_t k, int xa, std::uint32_t off, int lo, std::uint64_t c) {
     const int X = T.x0 + xa;
     const int jb = static_cast<int>(16 * k - off);
@@ -386,9 +399,10 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
       w[q] = v;
     }
     if (costs) *reinterpret_cast<uint4*>(out + 16 * std::size_t(k)) = make_uint4(w[0], w[1], w[2], w[3]);
-    if (map) mout[k] = map_entry(xa, jb / kLabelAlign);
+    if (map) mout[k] = map_entry(xa & (kStrip - 1), jb / kLabelAlign);
   };
   if (staged) {
+    const std::uint32_t chunks = chunks_to(last);
     const bool mapped = chunks <= static_cast<std::uint32_t>(kMap);
     for (std::uint32_t k = threadIdx.x; k < chunks; k += blockDim.x) {
       int xa;
@@ -410,18 +424,27 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
       chunk(k, xa, soff[xa], slo[xa], scl[xa]);
     }
   } else {
-    for (std::uint32_t k = threadIdx.x; k < chunks; k += blockDim.x) {
-      int xa = 0, xb = min(static_cast<int>(k), T.w - 1);
-      while (xa < xb) {
-        const int mid = (xa + xb + 1) >> 1;
-        if (pix_off(rec[mid]) <= 16 * k) {
-          xa = mid;
-        } else {
-          xb = mid - 1;
-        }
+    for (int xs = 0; xs < T.w; xs += kStrip) {
+      const int xn = min(T.w - xs, kStrip);
+      if (xs > 0) {
+        strip_cell = T.cell_base + strip_base[xs >> kStripShift];
+        out = C + strip_cell;
+        mout = cmap + strip_cell / kLabelAlign;
       }
-      const std::uint64_t pr = rec[xa];
-      chunk(k, xa, pix_off(pr), pix_lo(pr), cl[bcol(T.x0 + xa)]);
+      const std::uint32_t chunks = chunks_to(xs > 0 ? rec[xs + xn - 1] : last);
+      for (std::uint32_t k = threadIdx.x; k < chunks; k += blockDim.x) {
+        int xa = xs, xb = xs + min(static_cast<int>(k), xn - 1);
+        while (xa < xb) {
+          const int mid = (xa + xb + 1) >> 1;
+          if (pix_off(rec[mid]) <= 16 * k) {
+            xa = mid;
+          } else {
+            xb = mid - 1;
+          }
+        }
+        const std::uint64_t pr = rec[xa];
+        chunk(k, xa, pix_off(pr), pix_lo(pr), cl[bcol(T.x0 + xa)]);
+      }
     }
   }
 }
@@ -611,7 +634,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_path(
     const int i = min(base + l8, len - 1);
     const int x = x0 + i * DX, y = y0 + i * DY;
     b.rec = ldb<std::uint64_t>(tpix, static_cast<std::uint32_t>(y * T.w + x) * 8U);
-    b.rs = ldb<std::uint32_t>(trow, static_cast<std::uint32_t>(y) * 4U);
+    b.rs = ldb<std::uint32_t>(trow, static_cast<std::uint32_t>(y * T.strips + (x >> kStripShift)) * 4U);
   };
   // Unpacks a batch into the ring (slot l8 of the group); last_ip carries the
   // intensity of the batch's last step to the next batch's first.
@@ -1499,7 +1522,10 @@ __global__ __launch_bounds__(kSelThreads) void k_select(const JobDesc* __restric
   const int lf = rows[0], ll = rows[1], rf = rows[2], rl = rows[3];
   const int xb = min(max(lf - T.x0, 0), T.w);
   const int xe = min(max(ll + 1 - T.x0, xb), T.w);
-  const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + y];
+  // A block's columns lie in one strip; the diagonal check's keys hold tiles of one.
+  static_assert((1 << kStripShift) % kSelPx == 0);
+  const int strip = x0 >> kStripShift, xs = x0 - (strip << kStripShift);  // the strip's column of x0
+  const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + std::uint64_t(y) * T.strips + strip];
   const std::uint64_t px = T.px_base + std::uint64_t(y) * T.w;
   const bool split = T.cell_base < S.xcells;  // a slice or plane per path
   const int slices = split ? kPaths : S.n;
@@ -1601,20 +1627,20 @@ __global__ __launch_bounds__(kSelThreads) void k_select(const JobDesc* __restric
     const int k = ka + tid + kSelThreads * i;
     if (k < kb) {
       load(k, V[i]);
-      atomicMin(&best[map_col(m[i]) - x0], chunk_key(V[i], static_cast<std::uint32_t>(map_place(m[i]) * kLabelAlign)));
+      atomicMin(&best[map_col(m[i]) - xs], chunk_key(V[i], static_cast<std::uint32_t>(map_place(m[i]) * kLabelAlign)));
     }
   }
   for (int k = ka + tid + kSelThreads * kSelHeld; k < kb; k += kSelThreads) {
     std::uint32_t X[8];
     const std::uint32_t mm = rmap[k];
     load(k, X);
-    atomicMin(&best[map_col(mm) - x0], chunk_key(X, static_cast<std::uint32_t>(map_place(mm) * kLabelAlign)));
+    atomicMin(&best[map_col(mm) - xs], chunk_key(X, static_cast<std::uint32_t>(map_place(mm) * kLabelAlign)));
   }
   __syncthreads();
   // Best cost of a chunk outside the winner and its neighbours (labels w - 1
   // .. w + 1, halves a .. a + 2 of the chunk: words a / 2 and a / 2 + 1).
   auto outside = [&](std::uint32_t mm, const std::uint32_t (&X)[8]) __attribute__((always_inline)) {
-    const int x = map_col(mm) - x0;
+    const int x = map_col(mm) - xs;
     const int a = static_cast<int>(best[x] & 0xFFFFU) - 1 - map_place(mm) * kLabelAlign, j0 = a >> 1;
     std::uint32_t w0 = 0xFFFFFFFFU, w1 = 0xFFFFFFFFU, lowest = 0xFFFFFFFFU;
 #pragma unroll

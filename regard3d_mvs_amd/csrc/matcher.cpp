@@ -505,11 +505,11 @@ struct Aggregation {
   std::vector<Grid> grids;
   std::vector<int> tile_base;
   std::vector<std::uint64_t> tcells;
-  DBuf<std::uint32_t> rowbase;  // first cell of every tile row
+  DBuf<std::uint32_t> rowbase;  // first cell of every strip of every tile row
   DBuf<std::uint64_t> pix;
   std::uint64_t total_rows = 0, total_px = 0, total_cells = 0, max_tile_cells = 0;
   int max_w = 1, max_h = 1, max_D = 16, max_num = 16;
-  std::uint32_t max_row_chunks = 1;
+  std::uint32_t max_row_chunks = 1;  // of a strip: of a row where the sweeps ask
   int p2max = 0;
   std::vector<int> full;  // per job: its labels if every pixel has all of them, else 0
   std::vector<std::int64_t> img_stride;  // per job
@@ -603,7 +603,7 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
   std::vector<std::uint32_t> trow;
   DBuf<std::uint32_t>& rowbase = A.rowbase;
   DBuf<std::uint64_t>& pix = A.pix;
-  // tile_counts: cells [nt], then (uint32) the largest label counts [nt] and the most chunks in a row [nt]
+  // tile_counts: cells [nt], then (uint32) the largest label counts [nt] and the most chunks in a strip [nt]
   DBuf<std::uint64_t> row_cells, tile_counts;
   DBuf<std::uint32_t> row_max;
   std::uint64_t& total_rows = A.total_rows;
@@ -615,6 +615,7 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
     row_prefix.clear();
     total_rows = 0;
     total_px = 0;
+    std::uint64_t total_strips = 0;
     for (int j = 0; j < nj; ++j) {
       const Job& J = jobs[std::size_t(j)];
       grids[std::size_t(j)] = layout(J.base->w, J.base->h, tsize[std::size_t(j)], ext);
@@ -628,10 +629,12 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
           t.h = r[1] - r[0];
           t.job = j;
           t.px_base = total_px;
-          t.row_base = total_rows;
+          t.row_base = total_strips;
+          t.strips = strips_of(t.w);
           row_prefix.push_back(total_rows);
           total_px += std::uint64_t(t.w) * std::uint64_t(t.h);
           total_rows += std::uint64_t(t.h);
+          total_strips += std::uint64_t(t.h) * std::uint64_t(t.strips);
           td.push_back(t);
         }
       }
@@ -647,9 +650,9 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
       drow_prefix = view<std::uint64_t>(A.meta, orp);
     }
     pix = DBuf<std::uint64_t>(c.arena, total_px);
-    row_cells = DBuf<std::uint64_t>(c.arena, total_rows);
-    row_max = DBuf<std::uint32_t>(c.arena, total_rows);
-    rowbase = DBuf<std::uint32_t>(c.arena, total_rows);
+    row_cells = DBuf<std::uint64_t>(c.arena, total_strips);
+    row_max = DBuf<std::uint32_t>(c.arena, total_strips);
+    rowbase = DBuf<std::uint32_t>(c.arena, total_strips);
     tile_counts = DBuf<std::uint64_t>(c.arena, 2 * std::size_t(nt));
     launch_tile_row_scan(A.djobs.get(), dtiles.get(), drow_prefix.get(), nt, total_rows, pix.get(), row_cells.get(),
                          row_max.get(), c.stream);
@@ -725,9 +728,6 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
                                           " cells exceeds the 2^31 cells a tile volume may hold on the GPU; "
                                           "use a smaller tile_size or memory_budget");
   A.max_row_chunks = *std::max_element(trow.begin(), trow.end());
-  if (A.max_row_chunks >= kMaxRowChunks)
-    fail(R3DG_ERROR_INVALID_ARGUMENT, "stereo: a tile row of 2^28 cells or more is not supported on the GPU; use a "
-                                      "smaller tile_size");
   upload(c, A.dtiles, td);
   layout_timer.reset();
   return A;
@@ -762,11 +762,10 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   const int nt = t1 - t0;
   std::vector<TileDesc> td(A.td.begin() + t0, A.td.begin() + t1);
   std::vector<std::uint64_t> row_prefix(static_cast<std::size_t>(nt));
-  const std::uint64_t row0 = td.front().row_base;
   int max_num = 16;
   for (int t = 0; t < nt; ++t) {
     TileDesc& T = td[std::size_t(t)];
-    row_prefix[std::size_t(t)] = T.row_base - row0;
+    row_prefix[std::size_t(t)] = ch.rows;
     ch.cells += A.tcells[std::size_t(t0 + t)];
     ch.rows += std::uint64_t(T.h);
     ch.px += std::uint64_t(T.w) * std::uint64_t(T.h);

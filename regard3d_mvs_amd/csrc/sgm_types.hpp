@@ -10,13 +10,14 @@
 //
 // HBM layout of the costs C (uint8), of the paths' planes (uint8) and of the
 // aggregated costs S (uint16): every tile owns a contiguous volume at
-// cell_base, its rows one after the other (rowbase[row_base + y] is row y's
-// first cell), a row's pixels in order; a pixel's labels follow each other, at
-// the offset held in its pixel record pix[px_base + y*w + x] (the TileLabels
-// ranges of stereo_matcher.cpp:172-224).  Label counts are multiples of 16, so
-// every pixel's labels are whole chunks of 16 cells.
+// cell_base, its rows one after the other, a row's pixels in order; a pixel's
+// labels follow each other (the TileLabels ranges of stereo_matcher.cpp:172-224).
+// rowbase[row_base + y * strips + s] is the first cell of strip s of row y, the
+// pixel record pix[px_base + y*w + x] holds the offset from there (tiles of at
+// most 2^16 columns, nearly all, have one strip a row).  Label counts are
+// multiples of 16, so every pixel's labels are whole chunks of 16 cells.
 //
-// Pixel record (uint64): bits 0-23 chunk offset inside the tile row, bits
+// Pixel record (uint64): bits 0-23 chunk offset inside the strip, bits
 // 24-31 label count / 16, bits 32-47 first label `lo`, bits 48-63 intensity.
 #pragma once
 
@@ -28,7 +29,11 @@ namespace r3dg {
 
 constexpr int kLabelAlign = 16;
 constexpr int kMaxLabels = 4000;           // per pixel and level: a record keeps label count / 16 in 8 bits
-constexpr std::uint32_t kMaxRowChunks = 1U << 24;  // a record keeps a row's chunk offsets in 24 bits
+// A tile row is counted in strips of 2^16 columns: a record keeps a chunk offset
+// inside its strip in 24 bits, a map entry a column in 16.
+constexpr int kStripShift = 16;
+static_assert((std::uint64_t{kMaxLabels / kLabelAlign} << kStripShift) < (1U << 24));
+__host__ __device__ constexpr int strips_of(int columns) { return (columns + (1 << kStripShift) - 1) >> kStripShift; }
 constexpr int kPaths = 8;
 constexpr int kMaxByteP2 = 255;  // largest P2 with which a path's M = L - C is a byte
 
@@ -40,13 +45,12 @@ __host__ __device__ constexpr std::uint32_t pix_off(std::uint64_t r) { return st
 __host__ __device__ constexpr int pix_num(std::uint64_t r) { return int((r >> 24) & 0xFFU) * kLabelAlign; }
 __host__ __device__ constexpr int pix_lo(std::uint64_t r) { return int((r >> 32) & 0xFFFFU); }
 __host__ __device__ constexpr int pix_val(std::uint64_t r) { return int(r >> 48); }
-// Chunk map entry: the chunk's column in the tile (24 bits: a row of 2^24 columns
-// would have as many chunks) and its place in the pixel.
+// Chunk map entry: the chunk's column in its strip and its place in the pixel.
 __host__ __device__ constexpr std::uint32_t map_entry(int col, int place) {
-  return std::uint32_t(col) | std::uint32_t(place) << 24;
+  return std::uint32_t(col) | std::uint32_t(place) << kStripShift;
 }
-__host__ __device__ constexpr int map_col(std::uint32_t m) { return int(m & 0xFFFFFFU); }
-__host__ __device__ constexpr int map_place(std::uint32_t m) { return int(m >> 24); }
+__host__ __device__ constexpr int map_col(std::uint32_t m) { return int(m & ((1U << kStripShift) - 1)); }
+__host__ __device__ constexpr int map_place(std::uint32_t m) { return int(m >> kStripShift); }
 constexpr int kMaxLevels = 13;
 
 struct JobDesc {
@@ -84,9 +88,9 @@ struct TileDesc {
   std::int32_t max_num;       // largest label count of the tile
   std::uint64_t cell_base;    // first cell of the tile in S
   std::uint64_t px_base;      // first tile pixel in per-pixel arrays
-  std::uint64_t row_base;     // first tile row in per-row arrays
+  std::uint64_t row_base;     // first strip of the first row in per-strip arrays
   std::uint32_t cells;        // cells of the tile
-  std::uint32_t reserved;
+  std::int32_t strips;        // per row
 };
 
 // Tile grid of one job for blending (stereo_matcher.cpp:688-766): tile (i, j)
