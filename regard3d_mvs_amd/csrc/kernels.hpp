@@ -167,7 +167,7 @@ void launch_sgm_path(int path, const PathArgs& a, int mode, hipStream_t s);
 // 255).  A scanline takes `lanes` lanes of `labels` labels each, a wave
 // 64 / lanes scanlines (rows for paths 0 and 1, columns for the others);
 // gprefix[t] counts the groups of all paths before tile t.  full_split: for D
-// labels and a launch of that many scanlines; lanes 0 if there is no such kernel.
+// labels (full_takes) and a launch of that many scanlines.
 struct FullArgs {
   const JobDesc* jobs;
   const TileDesc* tiles;
@@ -182,6 +182,7 @@ struct FullSplit {
   int labels, lanes;
 };
 FullSplit full_split(int D, std::uint64_t scanlines);
+constexpr bool full_takes(int D) { return D <= 8 * 64; }
 // k_full addresses a tile's intensities by 32-bit byte offsets from its first
 // row: whether those of h rows of an image of this stride (elements) fit.
 constexpr bool full_offsets_fit(int h, std::int64_t img_stride) {

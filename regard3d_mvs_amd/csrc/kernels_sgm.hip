@@ -1927,7 +1927,7 @@ FullSplit full_split(int D, std::uint64_t scanlines) {
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   const std::uint64_t waves = (scanlines * std::uint64_t(lanes(4)) + 63) / 64;
   if (lanes(4) <= 32 && waves <= std::uint64_t(6 * std::max(cus, 1))) return {4, lanes(4)};
-  return lanes(8) <= 64 ? FullSplit{8, lanes(8)} : FullSplit{0, 0};
+  return {8, lanes(8)};
 }
 
 void launch_full(const FullArgs& a, FullSplit f, hipStream_t s) {

@@ -1129,7 +1129,7 @@ std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
     const auto job = std::size_t(A.td[std::size_t(t)].job);
     Aggregate kind = Aggregate::kScan;
     if (A.full[job] > 0) {
-      if (planes && full_split(A.full[job], 0).lanes > 0 && full_offsets_fit(A.td[std::size_t(t)].h, A.img_stride[job]))
+      if (planes && full_takes(A.full[job]) && full_offsets_fit(A.td[std::size_t(t)].h, A.img_stride[job]))
         kind = Aggregate::kFull;
     } else if (sweeps) {
       kind = Aggregate::kSweep;
@@ -1588,9 +1588,9 @@ ViewCache& view_cache(Context& c) {
 }
 
 // Device bytes a pair is expected to need: per-pixel buffers (pyramids,
-// Census, mirrored copies, maps) and its largest level's volumes (S and
-// costs, 3 bytes per cell) with about 48 labels per pixel when ranges come
-// from a coarser level.  Volumes beyond the memory left are chunked anyway.
+// Census, mirrored copies, maps) and its largest level's volumes, with about
+// 48 labels per pixel when ranges come from a coarser level.  Volumes beyond
+// the memory left are chunked anyway.
 // The part that cannot be chunked: images, pyramids, Census and maps.
 // Sizes of a pair for its memory estimates.  The disparity output has the
 // left image's size also where the left image comes from a cached view (the
@@ -1611,13 +1611,25 @@ std::uint64_t pair_fixed_bytes(const r3dg_pair& q) {
   return 96 * (z.wl + z.wr) * z.h;
 }
 
+// Quarters of a byte per cell of the form that aggregates a level where memory
+// allows (aggregate_tiles): costs and chunk map 5, and eight byte planes 32 for
+// full-range scans and one-path sweeps, eight uint16 slices 64 for sweeps past a
+// byte's P2, one slice 8 for path scans (full range past a byte's P2 or 512 labels).
+std::uint64_t volume_quarters(bool ranged, int labels, const r3dg_options& o) {
+  const auto lut = p2_table(o);
+  const bool bytes = *std::max_element(lut.begin(), lut.end()) <= kMaxByteP2;
+  if (ranged) return bytes ? 37 : 69;
+  return bytes && full_takes(labels) ? 37 : 13;
+}
+
 std::uint64_t pair_footprint(const r3dg_pair& q, const r3dg_options& o) {
   const PairSize z = pair_size(q);
   const std::uint64_t wl = z.wl, h = z.h;
   const int levels = o.levels >= 0 ? o.levels
                                    : automatic_levels(static_cast<int>(wl), static_cast<int>(h), q.num_disparities);
   const std::uint64_t labels = levels > 0 ? 48 : std::uint64_t(align16(std::max(q.num_disparities, 1)));
-  return pair_fixed_bytes(q) + 3 * 12 * wl * h * labels / 5;
+  const std::uint64_t quarters = volume_quarters(levels > 0, static_cast<int>(labels), o);
+  return pair_fixed_bytes(q) + quarters * 3 * wl * h * labels / 5;
 }
 
 struct Request {
