@@ -37,8 +37,10 @@ inline SweepPlan size_sweep(int np, int max_w, std::uint32_t max_chunks, std::ui
   const int fixed = 4 * (6 * max_w + 2 * np * max_w + 128 + 4);
   p.held = np == 3 || mean_chunks <= kSweepThreads ? 2 : 4;
   p.wpad = max_w;
-  p.cap = std::min({(lds - fixed) / (4 * np) - kSweepRowPad, 8 * kSweepThreads * p.held, static_cast<int>(need)});
-  if (p.cap < 1024) return p;
+  const int room = (lds - fixed) / (4 * np) - kSweepRowPad;
+  if (room < 1024) return p;
+  // At least 16 words: a window that is not used reads the row's first ten.
+  p.cap = std::min({room, 8 * kSweepThreads * p.held, std::max(static_cast<int>(need), 16)});
   p.lds_bytes = fixed + 4 * np * (p.cap + kSweepRowPad);
   p.swords = std::uint64_t(p.cap) >= need ? 0 : static_cast<int>(need) + 16;
   p.blocks = std::max(cus, 1);

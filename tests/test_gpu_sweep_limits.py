@@ -4,13 +4,15 @@ counted, so that a form of the aggregation that steps in unseen fails."""
 import numpy as np
 import pytest
 
-from regard3d_mvs_amd import StereoOptions
+from regard3d_mvs_amd import StereoOptions, synth
 from test_gpu_parity import _match_both, gpu  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
 RAW = dict(speckle_size=0, median=False)
-SCANS = 8  # launches of a level of path scans alone; a level of sweeps takes 3 or 4, full-range scans 1
+# Launches of a level: path scans, full-range scans, sweeps of one or of three
+# paths with two horizontal path scans, and both kinds of sweep with them.
+SCANS, FULL, SWEEPS, MIXED = 8, 1, 3, 4
 
 
 def test_rows_past_a_million_words(gpu):  # noqa: F811
@@ -25,3 +27,12 @@ def test_rows_past_a_million_words(gpu):  # noqa: F811
                        StereoOptions(p1=1, p2=2, p2_adapt=0, levels=1, range_radius=0, range_fill=0, uniqueness=0.3,
                                      tile_size=700, **RAW))
     assert g.aggregate_launches < 2 * SCANS
+
+
+# Rows far below an LDS row: few tiles (one path a sweep) and many (three).
+@pytest.mark.parametrize("w,h", [(60, 40), (200, 180)])
+def test_narrow_tiles(gpu, w, h):  # noqa: F811
+    p = synth.make_pair(w, h, 16, 17)
+    g, _ = _match_both(gpu, p.left, p.right, None, None, 0, 16,
+                       StereoOptions(levels=1, tile_size=16, tile_margin=2, tile_blend=0))
+    assert g.aggregate_launches == FULL + SWEEPS

@@ -49,7 +49,10 @@ def test_rows_hold_every_chunk(plans):
         assert lds_bytes <= 160 << 10
         # Chunks past the held ones start past the LDS row.
         assert 8 * 1024 * held >= cap
-    # Rows of more than 2^17 chunks are among them.
+        # What a window that is not used reads: the first ten words and none past the row's pad.
+        assert cap + 8 >= 10
+    # The shortest rows are taken (they all fit), and rows of more than 2^17 chunks.
+    assert all(ok for _, w, chunks, ok, *_ in plans if w <= 113)
     assert any(ok and chunks > 1 << 17 for _, _, chunks, ok, *_ in plans)
 
 
