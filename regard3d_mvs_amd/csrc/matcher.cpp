@@ -508,7 +508,7 @@ struct Aggregation {
   DBuf<std::uint32_t> rowbase;  // first cell of every strip of every tile row
   DBuf<std::uint64_t> pix;
   std::uint64_t total_rows = 0, total_px = 0, total_cells = 0, max_tile_cells = 0;
-  int max_w = 1, max_h = 1, max_D = 16, max_num = 16;
+  int max_w = 1, max_D = 16, max_num = 16;
   std::uint32_t max_row_chunks = 1;  // of a strip: of a row where the sweeps ask
   int p2max = 0;
   std::vector<int> full;  // per job: its labels if every pixel has all of them, else 0
@@ -716,7 +716,6 @@ Aggregation layout_jobs(Context& c, std::vector<Job>& jobs, const r3dg_options& 
     total_cells += tcells[std::size_t(t)];
     max_num = std::max<int>(max_num, static_cast<int>(tmax[std::size_t(t)]));
     max_w = std::max(max_w, td[std::size_t(t)].w);
-    A.max_h = std::max(A.max_h, td[std::size_t(t)].h);
   }
   for (const Job& J : jobs) max_D = std::max(max_D, J.D);
   if (max_num > kMaxLabels)
@@ -825,9 +824,8 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   const bool bytes = sweep && A.p2max <= kMaxByteP2;  // a path's M = L - C fits a byte
   // Path scans: all eight, or the horizontal two beside the sweeps.
   const int npaths = full ? 0 : (sweep ? 2 : kPaths);
-  // Group prefixes of the path scans (kScanPerWave scanlines per wave), of the
-  // full-range scans, and the tiles in the order of their work, largest first,
-  // so that the sweeps end with short ones.
+  // Group prefixes of the path scans (kScanPerWave scanlines per wave) and of
+  // the full-range scans.
   std::vector<std::uint64_t> gp(std::size_t(npaths) * (std::size_t(nt) + 1), 0);
   std::uint64_t max_groups = 0, sum_groups = 0;
   for (int p = 0; p < npaths; ++p) {
