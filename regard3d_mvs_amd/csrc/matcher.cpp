@@ -885,13 +885,15 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   ch.stride = strided(kind == Aggregate::kScan ? ch.cells : alloc_cells);
   // Scratch rows of the path scans' persistent waves (pixels wider than the
   // LDS rows; a multiple of 4: launches use whole blocks of 4 waves, one slot
-  // each).  Where S and the costs leave no room for the rows of all waves, as
-  // many scan at once as half of what is left holds rows for.
+  // each).  Where the volumes leave no room for the rows of all waves (S and
+  // the costs of path scans; of the sweeps at most half of the memory, and an
+  // eighth for their own scratch), as many scan at once as half of what is left
+  // holds rows for.
   const std::uint64_t resident = path_slots();
   std::uint64_t slots = (std::min(resident, std::max<std::uint64_t>(max_groups, 1)) + 3) / 4 * 4;
-  if (kind == Aggregate::kScan) {
-    const std::uint64_t volumes = 3 * strided(alloc_cells) + kBlockSlack;
-    const std::uint64_t left = free_bytes() - std::min(free_bytes(), volumes);
+  if (!full) {
+    const std::uint64_t left = sweep ? free_bytes() / 4
+                                     : free_bytes() - std::min(free_bytes(), 3 * strided(alloc_cells) + kBlockSlack);
     const std::uint64_t fit = left / 2 / (4 * sizeof(std::uint16_t) * path_scratch_elems(1, max_num)) * 4;
     slots = std::min(slots, std::max<std::uint64_t>(fit, 4));
   }
