@@ -155,51 +155,49 @@ __global__ __launch_bounds__(256) void k_tile_row_scan(const JobDesc* __restrict
   // Base columns of a mirrored job read the unmirrored image backwards.
   const int img_x0 = J.mirrored != 0 ? J.width - 1 - T.x0 : T.x0, img_dx = J.mirrored != 0 ? -1 : 1;
   std::uint64_t* prow = pix + T.px_base + std::uint64_t(y) * T.w;
-  std::uint64_t carry = 0;
-  std::uint32_t vmax = 0;
-  std::uint64_t strip = T.row_base + std::uint64_t(y) * static_cast<std::uint32_t>(T.strips);
-  // Cells and largest label count (of the row so far) of the strip that ends.
-  auto end_strip = [&] {
+  constexpr int kStrip = 1 << kStripShift;
+  static_assert(kStrip % (64 * kItems) == 0, "strips end where a pass does");
+  std::uint64_t strip = T.row_base + static_cast<std::uint32_t>(y * T.strips);
+#pragma unroll 1
+  for (int xs = 0; xs < T.w; xs += kStrip, ++strip) {
+    const int xe = min(T.w, xs + kStrip);
+    std::uint64_t carry = 0;
+    std::uint32_t vmax = 0;
+    for (int base = xs; base < xe; base += 64 * kItems) {
+      int lo[kItems], num[kItems], val[kItems];
+#pragma unroll
+      for (int k = 0; k < kItems; ++k) {
+        const int x = base + 64 * k + lane;
+        lo[k] = 0;
+        num[k] = 0;
+        val[k] = 0;
+        if (x < T.w) {
+          val[k] = img[img_x0 + img_dx * x];
+          if (jlo != nullptr) {
+            lo[k] = jlo[rbase + x];
+            num[k] = jnum[rbase + x];
+          } else {
+            num[k] = J.D;
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kItems; ++k) {
+        const int x = base + 64 * k + lane;
+        const std::uint32_t v = static_cast<std::uint32_t>(num[k]);
+        const std::uint32_t incl = wave_scan_incl(v);
+        if (x < T.w) prow[x] = pix_record(carry + incl - v, lo[k], num[k], val[k]);
+        carry += static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
+        vmax = max(vmax, v);
+      }
+    }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) vmax = max(vmax, static_cast<std::uint32_t>(__shfl_xor(vmax, d)));
     if (lane == 0) {
       row_cells[strip] = carry;
       row_max[strip] = vmax;
     }
-    ++strip;
-    carry = 0;
-  };
-  static_assert((1 << kStripShift) % (64 * kItems) == 0, "strips end where a pass does");
-  for (int base = 0; base < T.w; base += 64 * kItems) {
-    if (base > 0 && (base & ((1 << kStripShift) - 1)) == 0) end_strip();
-    int lo[kItems], num[kItems], val[kItems];
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-      const int x = base + 64 * k + lane;
-      lo[k] = 0;
-      num[k] = 0;
-      val[k] = 0;
-      if (x < T.w) {
-        val[k] = img[img_x0 + img_dx * x];
-        if (jlo != nullptr) {
-          lo[k] = jlo[rbase + x];
-          num[k] = jnum[rbase + x];
-        } else {
-          num[k] = J.D;
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-      const int x = base + 64 * k + lane;
-      const std::uint32_t v = static_cast<std::uint32_t>(num[k]);
-      const std::uint32_t incl = wave_scan_incl(v);
-      if (x < T.w) prow[x] = pix_record(carry + incl - v, lo[k], num[k], val[k]);
-      carry += static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
-      vmax = max(vmax, v);
-    }
   }
-  end_strip();
 }
 
 // Totals of one tile (cells, largest label count, most chunks in a strip) and
@@ -369,7 +367,7 @@ __global__ __launch_bounds__(kCostThreads) void k_cost(const JobDesc* __restrict
   auto chunks_to = [](std::uint64_t r) { return (pix_off(r) + static_cast<std::uint32_t>(pix_num(r))) >> 4; };
   const int bfirst = rows[0], blast = rows[1], pfirst = rows[2], plast = rows[3];
   const std::uint32_t invalid = static_cast<std::uint32_t>(J.invalid_cost);
-  const std::uint32_t* strip_base = rowbase + T.row_base + std::uint64_t(y) * T.strips;
+  const std::uint32_t* strip_base = rowbase + T.row_base + static_cast<std::uint32_t>(y * T.strips);
   const bool costs = C != nullptr, map = cmap != nullptr;
   // Output of the strip in hand.
   std::uint64_t strip_cell = T.cell_base + strip_base[0];
@@ -1525,7 +1523,7 @@ __global__ __launch_bounds__(kSelThreads) void k_select(const JobDesc* __restric
   // A block's columns lie in one strip; the diagonal check's keys hold tiles of one.
   static_assert((1 << kStripShift) % kSelPx == 0);
   const int strip = x0 >> kStripShift, xs = x0 - (strip << kStripShift);  // the strip's column of x0
-  const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + std::uint64_t(y) * T.strips + strip];
+  const std::uint64_t row_cell = T.cell_base + rowbase[T.row_base + static_cast<std::uint32_t>(y * T.strips + strip)];
   const std::uint64_t px = T.px_base + std::uint64_t(y) * T.w;
   const bool split = T.cell_base < S.xcells;  // a slice or plane per path
   const int slices = split ? kPaths : S.n;

@@ -1124,7 +1124,7 @@ std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
     ranged_cells += A.tcells[std::size_t(t)];
   }
   const bool sweeps =
-      roomy && A.max_w <= kSweepThreads && sweeps_fit(ranged, ranged_cells, room, bytes, compute_units());
+      ranged > 0 && roomy && A.max_w <= kSweepThreads && sweeps_fit(ranged, ranged_cells, room, bytes, compute_units());
   for (int t = 0; t < nt; ++t) {
     const auto job = std::size_t(A.td[std::size_t(t)].job);
     Aggregate kind = Aggregate::kScan;
