@@ -590,7 +590,7 @@ __device__ __forceinline__ void load4(const T* p, float* v) {
   for (int i = 0; i < 4; ++i) v[i] = static_cast<float>(t[i]);
 }
 
-// Bound by vector instructions, 215 a pixel: a call on 24 Mpx of uint16 takes
+// Bound by vector instructions, 218 a pixel: a call on 24 Mpx of uint16 takes
 // 0.169 ms where 16 single loads and 4 divisions a pixel took 0.188.  A thread
 // takes kRectRows pixels of a column, whose x terms are computed once, and a
 // row's four taps come by one load wherever all four lie inside the source;
@@ -718,7 +718,7 @@ __device__ __forceinline__ V pick(const V (&a)[N], int q) {
 // combine_pairs per grid pixel (multi_stereo.cpp:103-213), double precision
 // in the reference's order of operations.
 //
-// Bound by vector instructions (about 950 a wave for 4 pairs, a third of them in
+// Bound by vector instructions (about 890 a wave for 4 pairs, a third of them in
 // double precision): 4 pairs of 27 Mpx take 0.90 ms.  Every list of pairs is
 // indexed by the pair and unrolled to N, so that it lives in registers; lists
 // filled and indexed at run time went to scratch memory, and the kernel took

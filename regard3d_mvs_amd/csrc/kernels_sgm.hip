@@ -11,7 +11,8 @@
 //            16-label chunks, up to three paths at once;
 //   k_path   one path direction over every tile by waves of 8 scanlines: the
 //            horizontal paths beside the sweeps, and all eight where the
-//            memory left or the tiles' width rule the others out.
+//            memory left, the tiles' width, labels or P2 rule the others out
+//            or sweeps would be too few to fill the device.
 // Each writes uint16 slices of S (uint16 wrap-around, so the order of the
 // paths does not matter) or byte planes; the selection sums them.
 //
@@ -1154,7 +1155,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_full(FullArgs A) {
 //
 // Bound by CU time: a block fills its CU's LDS and registers, and its 16 waves
 // issue vector instructions (about 180 per chunk and path with three paths, 260
-// with one) in 60 to 75% of the time, between the two barriers of a row.  The
+// with one) in 60 to 75% of the time, between the two barriers of a row (with
+// three paths at the limit of 128 registers, 76 bytes a lane in scratch).  The
 // six paths of the 24 MP pair's finest level: 19 ms by k_path; 11.5 ms here.
 // Barrier that orders LDS accesses only: loads in flight and stores of sums
 // stay in flight across it.

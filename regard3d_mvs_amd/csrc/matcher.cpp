@@ -495,8 +495,8 @@ std::size_t estimated_tile_bytes(std::uint64_t cells64, int w_, int h_, int righ
 }
 
 // Tile layout of a set of jobs: the tiles of all jobs share the layout pass,
-// and chunks of consecutive tiles share the cost pass, the 8 path launches
-// and the selection launch.
+// and chunks of consecutive tiles share the cost pass, the launches of the
+// aggregation and the selection launch.
 struct Aggregation {
   DBuf<unsigned char> meta;  // job descriptors (and the layout pass's tiles and row prefix)
   DView<JobDesc> djobs;
@@ -739,7 +739,8 @@ int path_scanlines(int p, int w, int h) { return p < 2 ? h : (p < 4 ? w : w + h 
 // kSweep: row sweeps for the vertical and diagonal paths, path scans for the
 // horizontal ones (k_sweep, k_path: at least 7 bytes per cell).  kScan: a path
 // scan per path, summed in S (3 bytes per cell), where the memory left holds
-// no more or the other kernels do not apply.
+// no more, sweeps would be too few to fill the device (sweeps_fit) or the other
+// kernels do not apply.
 enum class Aggregate { kFull, kSweep, kScan };
 
 // Sweeps of one path each instead of three where the tiles are fewer than
