@@ -1114,6 +1114,7 @@ struct TileRange {
 std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
   const std::uint64_t free_bytes = c.arena.budget() > c.arena.live() ? c.arena.budget() - c.arena.live() : 0;
   const std::uint64_t most = std::uint64_t{4} << 30, room = std::min(free_bytes / 20, most);
+  const std::uint64_t scan_room = std::max(A.max_tile_cells, std::min(free_bytes / 4, most));
   const bool roomy = A.max_tile_cells <= room;
   const bool bytes = A.p2max <= kMaxByteP2, planes = roomy && bytes;
   std::vector<TileRange> out;
@@ -1125,7 +1126,7 @@ std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
     ranged_cells += A.tcells[std::size_t(t)];
   }
   const bool sweeps =
-      ranged > 0 && roomy && A.max_w <= kSweepThreads && sweeps_fit(ranged, ranged_cells, room, bytes, compute_units());
+      ranged > 0 && roomy && A.max_w <= kSweepThreads && sweeps_fit(ranged, ranged_cells, room, scan_room, bytes, compute_units());
   for (int t = 0; t < nt; ++t) {
     const auto job = std::size_t(A.td[std::size_t(t)].job);
     Aggregate kind = Aggregate::kScan;
@@ -1135,7 +1136,7 @@ std::vector<TileRange> chunk_tiles(const Context& c, const Aggregation& A) {
     } else if (sweeps) {
       kind = Aggregate::kSweep;
     }
-    const std::uint64_t cap = kind == Aggregate::kScan ? std::max(A.max_tile_cells, std::min(free_bytes / 4, most)) : room;
+    const std::uint64_t cap = kind == Aggregate::kScan ? scan_room : room;
     const std::uint64_t n = A.tcells[std::size_t(t)];
     if (out.empty() || out.back().kind != kind || out.back().cells + n > cap) out.push_back({t, t, kind, 0});
     out.back().cells += n;

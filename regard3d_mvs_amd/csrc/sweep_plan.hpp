@@ -49,23 +49,29 @@ inline SweepPlan size_sweep(int np, int max_w, std::uint32_t max_chunks, std::ui
 }
 
 // Whether sweeps take the `tiles` tiles with label ranges of a level, of `cells`
-// cells in all, where a range of tiles may hold `cap` cells; path scans
-// otherwise.  A sweep is one block's chain of rows, six a tile, as long with
-// few tiles as with many: with 12 (one tile and its mirror) path scans are
-// over sooner (384x288 with a half-size level 0.97 and 0.93 ms, 480x270 1.02 and 0.96),
-// with 48 sweeps (960x540 1.37 and 1.52 ms; 800x600 1.29 and 1.26).  The line is at a
-// sixteenth of the compute units, at an eighth where a path's slices are
-// uint16 (P2 past a byte; 640x480, 24 sweeps: 1.86 and 1.60 ms).
+// cells in all, where a range of tiles may hold `cap` cells (`scan_cap` of path
+// scans); path scans otherwise.  A sweep is one block's chain of rows, six a
+// tile, as long with few tiles as with many: with 12 (one tile and its mirror)
+// path scans are over sooner (384x288 with a half-size level 0.97 and 0.93 ms,
+// 480x270 1.02 and 0.96), with 48 sweeps (960x540 1.37 and 1.52 ms; 800x600 1.29 and
+// 1.26).  The line is at a sixteenth of the compute units, at an eighth where a
+// path's slices are uint16 (P2 past a byte; 640x480, 24 sweeps: 1.86 and 1.60 ms).
 //
-// Where the level is cut into ranges, each waits for its slowest tile, and path
-// scans, of five times the cells a range, are cut into fewer: then only with
-// four blocks a compute unit (aggregation of 24 MP in 10 GiB, 32 tiles a range:
-// 52 ms by sweeps and 37 by path scans, of 1080p in 1.2 GiB, 8 tiles a range:
-// 12.5 and 7.4; the 24 MP pair in 30 GiB, 96 tiles a range: 33.7 and 34).
-inline bool sweeps_fit(std::uint64_t tiles, std::uint64_t cells, std::uint64_t cap, bool bytes, int cus) {
-  const std::uint64_t ranges = cells / std::max<std::uint64_t>(cap, 1) + 1, units = 6 * tiles / ranges;
+// Where the level is cut into ranges, each waits for its slowest tile.  Path
+// scans hold five times the cells in the same memory; where they are cut into
+// fewer ranges, sweeps have to have four blocks a compute unit in each of theirs
+// (aggregation of 24 MP in 10 GiB, 32 tiles a range: 52 ms by sweeps and 37 by path
+// scans, of 1080p in 1.2 GiB, 8 tiles a range: 12.5 and 7.4; the 24 MP pair in 30
+// GiB, 96 tiles a range: 33.7 and 34).  Where both are cut alike, at the most
+// cells a range may have, a quarter is enough (24 MP with 400 labels a pixel, 48
+// tiles a range: 149 and 174 ms; 3 MP with 900, 12 tiles a range: 51 and 53).
+inline bool sweeps_fit(std::uint64_t tiles, std::uint64_t cells, std::uint64_t cap, std::uint64_t scan_cap, bool bytes,
+                       int cus) {
+  const auto cut = [&](std::uint64_t most) { return cells / std::max<std::uint64_t>(most, 1) + 1; };
+  const std::uint64_t ranges = cut(cap), units = 6 * tiles / ranges;
   const auto n = std::uint64_t(std::max(cus, 0));
-  return ranges == 1 ? (bytes ? 16 : 8) * units >= n : units >= 4 * n;
+  if (ranges == 1) return (bytes ? 16 : 8) * units >= n;
+  return ranges > cut(scan_cap) ? units >= 4 * n : 4 * units >= n;
 }
 
 }  // namespace r3dg

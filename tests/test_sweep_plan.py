@@ -60,25 +60,27 @@ FORMS = r"""
 #include <cstdio>
 #include "sweep_plan.hpp"
 int main() {
-  unsigned long long tiles, cells, cap;
+  unsigned long long tiles, cells, cap, scan_cap;
   int bytes;
-  while (std::scanf("%llu %llu %llu %d", &tiles, &cells, &cap, &bytes) == 4)
-    std::printf("%d\n", r3dg::sweeps_fit(tiles, cells, cap, bytes != 0, 256) ? 1 : 0);
+  while (std::scanf("%llu %llu %llu %llu %d", &tiles, &cells, &cap, &scan_cap, &bytes) == 5)
+    std::printf("%d\n", r3dg::sweeps_fit(tiles, cells, cap, scan_cap, bytes != 0, 256) ? 1 : 0);
 }
 """
 
 
 def test_sweeps_fit(tmp_path):
-    """Sweeps where a range has blocks enough; cut levels only with many."""
+    """Sweeps where a range has blocks enough; levels that path scans would cut
+    into fewer ranges only with many."""
     cxx = shutil.which("g++")
     if cxx is None:
         pytest.skip("no host C++ compiler")
     (tmp_path / "fit.cpp").write_text(FORMS)
     subprocess.run([cxx, "-std=c++20", "-Wall", "-Werror", "-I", os.path.join(ROOT, "regard3d_mvs_amd", "csrc"),
                     str(tmp_path / "fit.cpp"), "-o", str(tmp_path / "fit")], check=True)
-    cases = [(2, 10, 100, 1, 0), (3, 10, 100, 1, 1), (5, 10, 100, 0, 0), (6, 10, 100, 0, 1), (0, 0, 100, 1, 0),
-             (96, 150, 100, 1, 0), (342, 150, 100, 1, 1), (341, 150, 100, 1, 0), (700, 1050, 100, 1, 0),
-             (48, 99, 100, 0, 1), (10, 10, 0, 1, 0)]
-    text = "".join("%d %d %d %d\n" % c[:4] for c in cases)
+    cases = [(2, 10, 100, 500, 1, 0), (3, 10, 100, 500, 1, 1), (5, 10, 100, 500, 0, 0), (6, 10, 100, 500, 0, 1),
+             (0, 0, 100, 500, 1, 0), (96, 150, 100, 500, 1, 0), (342, 150, 100, 500, 1, 1), (341, 150, 100, 500, 1, 0),
+             (700, 1050, 100, 500, 1, 0), (48, 99, 100, 500, 0, 1), (10, 10, 0, 0, 1, 0),
+             (96, 150, 100, 100, 1, 1), (22, 150, 100, 100, 1, 1), (21, 150, 100, 100, 1, 0)]
+    text = "".join("%d %d %d %d %d\n" % c[:5] for c in cases)
     out = subprocess.run([str(tmp_path / "fit")], input=text, check=True, capture_output=True, text=True).stdout
-    assert [int(v) for v in out.split()] == [c[4] for c in cases]
+    assert [int(v) for v in out.split()] == [c[5] for c in cases]
