@@ -886,14 +886,14 @@ Chunk aggregate_tiles(Context& c, Aggregation& A, int t0, int t1, Aggregate kind
   ch.stride = strided(kind == Aggregate::kScan ? ch.cells : alloc_cells);
   // Scratch rows of the path scans' persistent waves (pixels wider than the
   // LDS rows; a multiple of 4: launches use whole blocks of 4 waves, one slot
-  // each).  Where the volumes leave no room for the rows of all waves (S and
-  // the costs of path scans; of the sweeps at most half of the memory, and an
-  // eighth for their own scratch), as many scan at once as half of what is left
-  // holds rows for.
+  // each).  Where the volumes leave no room for the rows of all waves, as many
+  // scan at once as half of what S and the costs leave holds rows for, or, beside
+  // sweeps (whose volumes take up to 0.7 of the memory and their own scratch an
+  // eighth), a sixteenth of it each.
   const std::uint64_t resident = path_slots();
   std::uint64_t slots = (std::min(resident, std::max<std::uint64_t>(max_groups, 1)) + 3) / 4 * 4;
   if (!full) {
-    const std::uint64_t left = sweep ? free_bytes() / 4
+    const std::uint64_t left = sweep ? free_bytes() / 8
                                      : free_bytes() - std::min(free_bytes(), 3 * strided(alloc_cells) + kBlockSlack);
     const std::uint64_t fit = left / 2 / (4 * sizeof(std::uint16_t) * path_scratch_elems(1, max_num)) * 4;
     slots = std::min(slots, std::max<std::uint64_t>(fit, 4));
